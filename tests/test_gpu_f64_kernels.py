@@ -1,0 +1,59 @@
+"""The direct-to-LDS FP64 kernels at the edges of their tiles and of the rules that choose them: the
+even deal of the dielectric builds (64 x 64 and 128 x 128 tiles, flocks of frequencies, shared and
+whole units) and the split second-stage and exchange products (every width of the narrow tile)."""
+import numpy as np
+import pytest
+
+from oracle import xtp_oracle as X
+from votca_amd import pyxtp as px
+
+pytestmark = pytest.mark.gpu
+
+# sums of at most ~4000 products: |error| <= K 2^-53 relative to the sum of magnitudes
+TOL = 1e-12
+
+
+def tensor(rng, o, v, P, scale=0.05):
+    n = o + v
+    M = rng.normal(scale=scale, size=(n, n, P))
+    return 0.5 * (M + M.transpose(1, 0, 2))
+
+
+def energies(rng, o, v):
+    return np.concatenate([np.sort(rng.uniform(-1, -0.3, o)), np.sort(rng.uniform(0.1, 2.0, v))])
+
+
+@pytest.mark.parametrize("o,v,P,nw", [(1, 1, 1, 1), (2, 3, 16, 4), (3, 21, 63, 1), (3, 22, 64, 5), (5, 13, 65, 12),
+                                      (7, 31, 130, 3), (11, 47, 200, 8), (2, 5, 1535, 2), (2, 5, 1536, 4),
+                                      (3, 7, 1601, 1)])
+def test_eps_even_deal(o, v, P, nw):
+    rng = np.random.default_rng(o * 1000 + P + nw)
+    M = rng.normal(scale=0.1, size=(o, o + v, P))
+    e = energies(rng, o, v)
+    t = px.TCMatrix_gwbse().Initialize(P, 0, o - 1, 0, o + v - 1).set_tensor(M)
+    rpa = px.RPA(t)
+    rpa.configure(o - 1, 0, o + v - 1)
+    rpa.setRPAInputEnergies(e)
+    w = np.linspace(0.0, 3.0, nw)
+    out = rpa.calculate_epsilon(px.EPS_IMAG, w)
+    A = M[:, o:, :].reshape(o * v, P)
+    D = (e[None, o:] - e[:o, None]).reshape(-1)
+    for i in range(nw):
+        ref = np.eye(P) + A.T @ ((4.0 * D / (D * D + w[i] * w[i]))[:, None] * A)
+        assert np.linalg.norm(out[:, :, i] - ref) <= TOL * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("o,v,P,k", [(1, 1, 1, 1), (1, 9, 40, 3), (3, 17, 33, 16), (15, 5, 50, 2), (16, 20, 24, 17),
+                                     (17, 40, 31, 1), (33, 12, 20, 4), (49, 7, 12, 2), (65, 9, 11, 2), (81, 6, 9, 1),
+                                     (97, 5, 8, 1), (113, 4, 7, 2), (129, 3, 6, 1), (9, 129, 64, 5)])
+@pytest.mark.parametrize("c", [(1, 2, 1, 0), (0, 2, 0, 1)])
+def test_products_narrow_tiles(o, v, P, k, c):
+    rng = np.random.default_rng(o * 100 + v + P + k)
+    M, e = tensor(rng, o, v, P), energies(rng, o, v)
+    eps, H = rng.uniform(0.3, 1.0, P), np.diag(e)
+    n = o + v
+    t = px.TCMatrix_gwbse().Initialize(P, 0, n - 1, 0, n - 1).set_tensor(M)
+    op = px.BSE_OPERATOR(*c, eps, t, H).configure(px.BSEOperator_Options(o - 1, 0, 0, 0, n - 1))
+    x = rng.normal(size=(o * v, k))
+    ref = X.bse_dense(*c, eps, M, H, o - 1, 0, 0, n - 1) @ x
+    assert np.linalg.norm(op.matmul(x) - ref) <= TOL * np.linalg.norm(ref)

@@ -32,6 +32,7 @@
 #include "gemm_kernels.h"
 #include "gemm_pipe.h"
 #include "gemm_lds.h"
+#include "gemm_f64_lds.h"
 #include "host_eigen.h"
 #include "kernels_misc.h"
 #include "qp_solver.h"
@@ -199,24 +200,39 @@ inline int lower_tile_group(const GemmDims& d) {
 
 template <bool AK, bool BK_, class Epi>
 void gemm64(hipStream_t st, int M, int N, int K, int batch, int ksplit, Opnd<double> A, Opnd<double> B,
-            const double* s, long s_bs, bool lower, Epi epi) {
+            bool lower, Epi epi) {
   if (M <= 0 || N <= 0 || batch <= 0) return;
-  // 128x128 tiles halve the operand traffic per FLOP; used when the grid still fills the chip
+  K = std::max(K, 0);
   const long big_tiles = (long)((M + 127) / 128) * ((N + 127) / 128) * batch * std::max(ksplit, 1);
+  if constexpr (AK && BK_) {
+    // K-contiguous, 16-byte aligned operands: direct-to-LDS kernels. Up to 64 columns the tile is as
+    // wide as N; beyond, 128 x 64 tiles while they give half the chip's 512 resident workgroups one
+    // each, 64 x 64 tiles below that and for a lower triangle.
+    if (f64_lds_ok(A, B, K, nullptr, 0)) {
+      const long big = (long)((M + 127) / 128) * ((N + 63) / 64) * batch * std::max(ksplit, 1);
+      if (!lower && N <= 64) {
+        XG_HIP(launch_f64_narrow(st, M, N, K, batch, ksplit, A, B, epi));
+      } else if (!lower && M > 64 && big >= 256) {
+        GemmDims d = make_dims<128, 64>(M, N, K, batch, ksplit, 16, false);
+        d.group = tile_group(d);
+        XG_HIP(launch_f64_big(st, d, A, B, epi));
+      } else {
+        GemmDims d = make_dims<64, 64>(M, N, K, batch, ksplit, 16, lower);
+        if (lower) d.group = lower_tile_group(d);
+        XG_HIP(launch_f64_mid(st, d, A, B, epi));
+      }
+      return;
+    }
+  }
+  // 128x128 tiles halve the operand traffic per FLOP; used when the grid still fills the chip
   if (ksplit <= 1 && M >= 256 && N >= 256 && big_tiles >= 512) {
-    GemmDims d = make_dims<128, 128>(M, N, std::max(K, 0), batch, ksplit, 16, lower);
+    GemmDims d = make_dims<128, 128>(M, N, K, batch, ksplit, 16, lower);
     d.group = lower ? lower_tile_group(d) : tile_group(d);
-    // registers capped for two waves per SIMD (210 VGPRs, accumulators in VGPRs): 61 against 44
-    // TFLOP/s at one wave per SIMD on the Hd stage-1 product; XTPGPU_F64_KERNEL=occ1 selects the latter
-    const char* e = std::getenv("XTPGPU_F64_KERNEL");
-    if (e && std::strcmp(e, "occ1") == 0)
-      XG_HIP((launch_gemm_f64<128, 128, AK, BK_>(st, d, A, B, s, s_bs, epi)));
-    else
-      XG_HIP((launch_gemm_f64<128, 128, AK, BK_, Epi, 2>(st, d, A, B, s, s_bs, epi)));
+    XG_HIP((launch_gemm_f64<128, 128, AK, BK_>(st, d, A, B, epi)));
     return;
   }
-  GemmDims d = make_dims<64, 64>(M, N, std::max(K, 0), batch, ksplit, 16, lower);
-  XG_HIP((launch_gemm_f64<64, 64, AK, BK_>(st, d, A, B, s, s_bs, epi)));
+  GemmDims d = make_dims<64, 64>(M, N, K, batch, ksplit, 16, lower);
+  XG_HIP((launch_gemm_f64<64, 64, AK, BK_>(st, d, A, B, epi)));
 }
 
 // BF16 kernel choice (XTPGPU_BF16_KERNEL, for A/B timing; anything else is the default, 1):
@@ -639,7 +655,7 @@ extern "C" int xtpgpu_mmn_multiply_right(xtpgpu_mmn mmn, const double* A, int64_
     for (long n0 = 0; n0 < MN; n0 += (1L << 30)) {
       int nn = (int)std::min<long>(MN - n0, 1L << 30);
       gemm64<true, false>(ctx->stream, (int)P, nn, (int)P, 1, 1, Opnd<double>{dA.as<double>(), nullptr, lda, 0},
-                          Opnd<double>{mmn->d() + n0, nullptr, MN, 0}, nullptr, 0, false,
+                          Opnd<double>{mmn->d() + n0, nullptr, MN, 0}, false,
                           EpiStore{out.as<double>() + n0, MN, 1, 0, 1.0, 0.0});
     }
     XG_HIP(hipStreamSynchronize(ctx->stream));
@@ -667,12 +683,12 @@ extern "C" int xtpgpu_mmn_fill_ao2mo(xtpgpu_mmn mmn, const double* ao3c, int64_t
     const double* Cn = dC.as<double>() + (long)mmn->nmin * ldc;
     // A(m, mu) = Cm[mu + m*ldc] (K-contiguous); B(mu, nu) = T[Q][mu + nu*nb] (K-contiguous)
     gemm64<true, true>(ctx->stream, (int)mt, (int)nb, (int)nb, (int)P, 1, Opnd<double>{Cm, nullptr, ldc, 0},
-                       Opnd<double>{dT.as<double>(), nullptr, nb, nb * nb}, nullptr, 0, false,
+                       Opnd<double>{dT.as<double>(), nullptr, nb, nb * nb}, false,
                        EpiStore{dH.as<double>(), nb, 1, mt * nb, 1.0, 0.0});
     // step 2: M[Q][m][n] = sum_nu H[Q](m, nu) Cn(nu, n)  ->  data[Q*mt*nt + m*nt + n]
     gemm64<true, true>(ctx->stream, (int)mt, (int)nt, (int)nb, (int)P, 1,
                        Opnd<double>{dH.as<double>(), nullptr, nb, mt * nb}, Opnd<double>{Cn, nullptr, ldc, 0},
-                       nullptr, 0, false, EpiStore{mmn->d(), nt, 1, mt * nt, 1.0, 0.0});
+                       false, EpiStore{mmn->d(), nt, 1, mt * nt, 1.0, 0.0});
     XG_HIP(hipStreamSynchronize(ctx->stream));
     mmn->version++;
   });
@@ -802,14 +818,6 @@ size_t eps_scale_budget() {
   return (size_t)12 << 30;
 }
 
-// FP64 eps with the frequency weights in scaled copies (default: 43.7 against 37.3 TFLOP/s for the
-// weights applied on the B-operand load at the single-segment shapes; XTPGPU_EPS64_SCALED=0 selects
-// the latter).
-bool eps64_scaled() {
-  const char* e = std::getenv("XTPGPU_EPS64_SCALED");
-  return !(e && std::strcmp(e, "0") == 0);
-}
-
 // K splits of a lower-triangle eps GEMM so that its workgroups fill whole rounds of the resident
 // slots (`resident` = workgroups the kernel keeps on the chip at once): 136 tiles x 12 frequencies at
 // P = 2000 are 3.2 rounds of 512 slots, the last one a fifth full; three splits make 9.6 of 10.
@@ -917,46 +925,13 @@ void rpa_epsilon_impl(xtpgpu_ctx ctx, xtpgpu_mmn mmn, const double* energies, in
   // algorithmic FLOPs: n_omega * K * P * (P+1) (symmetric rank-K update); bytes: M read once + eps written
   ProfScope prof(ctx, "rpa_eps_gemm", (double)n_omega * K * P * (P + 1),
                  (double)P * K * (use16 ? (precision == XTPGPU_BF16X3 ? 4 : 2) : 8) + (double)n_omega * P * P * 8);
-  if (!use16 && !eps64_scaled()) {
-    Opnd<double> A{pk.A64.as<double>(), nullptr, Kp, 0};
-    gemm64<true, true>(st, (int)P, (int)P, (int)Kp, n_omega, 1, A, A, d64, Kp, true, epi);
-  } else if (!use16) {
-    // FP64 with the weights in scaled copies B_w = M diag(d_w), as the mixed forms do
-    const size_t plane = (size_t)P * Kp;
-    const size_t per_w = plane * 8;
-    const long gmax = std::max<long>(1, std::min<long>(n_omega, (long)(eps_scale_budget() / per_w)));
-    const long ngroups = (n_omega + gmax - 1) / gmax;
-    const long gsz = (n_omega + ngroups - 1) / ngroups;
-    DevBuf& sc = ctx->ws[1];  // kept on the context: a multi-GB allocation and free per build costs more than the build
-    sc.ensure(per_w * gsz);
-    double* Bs = sc.as<double>();
-    const double* A64 = pk.A64.as<double>();
-    const Opnd<double> A{A64, nullptr, Kp, 0};
-    for (long w0 = 0; w0 < n_omega; w0 += gsz) {
-      const long nw_g = std::min<long>(gsz, n_omega - w0);
-      const double* dg = d64 + w0 * Kp;
-      const long Kpl = Kp;
-      launch_map(st, plane, [=] __device__(size_t i) {
-        const double a = A64[i];
-        const long k = (long)(i % (size_t)Kpl);
-        for (long f = 0; f < nw_g; ++f) Bs[f * plane + i] = a * dg[f * Kpl + k];
-      });
-      EpiEpsSym eg{out_dev + w0 * P * P, P};
-      const Opnd<double> Bo{Bs, nullptr, Kp, (long)plane};
-      const long tl = (P + 127) / 128;
-      const int ks = P >= 256 ? eps_ksplit(tl * (tl + 1) / 2 * nw_g, 2L * cus, Kp, 16) : 1;
-      if (ks > 1) {  // 128 x 128 two-wave tiles over K splits, FP64 partials, one reduction
-        GemmDims d = make_dims<128, 128>((int)P, (int)P, (int)Kp, (int)nw_g, ks, 16, true);
-        d.group = lower_tile_group(d);
-        DevBuf& pb = ctx->ws[2];
-        pb.ensure((size_t)d.ksplit * nw_g * P * P * 8);
-        XG_HIP((launch_gemm_f64<128, 128, true, true, EpiPartial, 2>(
-            st, d, A, Bo, nullptr, 0, EpiPartial{pb.as<double>(), (int)P, (int)P, (int)nw_g})));
-        eps_reduce_splits(st, pb.as<double>(), d.ksplit, nw_g, P, out_dev + w0 * P * P);
-      } else {
-        gemm64<true, true>(st, (int)P, (int)P, (int)Kp, (int)nw_g, 1, A, Bo, nullptr, 0, true, eg);
-      }
-    }
+  if (!use16) {
+    // both operands are the packed transitions; the kernel applies the weights to the B fragments
+    const Opnd<double> A{pk.A64.as<double>(), nullptr, Kp, 0};
+    const EvenPlan pl = f64_even_plan(P, Kp, n_omega, cus);
+    DevBuf& pb = ctx->ws[2];
+    pb.ensure(pl.part_bytes());
+    XG_HIP(launch_f64_even(st, pl, (int)P, (int)Kp, n_omega, A, A, d64, Kp, pb.as<double>(), epi));
   } else {
     // the weights go into a scaled copy of the transitions, B_w = M diag(d_w) as BF16 hi (+ lo),
     // built once per frequency, so the GEMM's inner loop is plain MFMA work; frequencies are
@@ -1156,7 +1131,26 @@ void zero_bytes(hipStream_t st, void* p, size_t bytes) {
 // aux function (both planes), for the given precision and block width.
 struct MatmulPlan {
   size_t xp = 0, xh = 0, xl = 0, part = 0, wbuf = 0, per_p = 0;
+  size_t part_more = 0;  // partials of every K split the FP64 products would take; part is enough to run
 };
+
+// K splits of an FP64 product of `units` output tiles (128 rows each, full width) so that its
+// workgroups cover the chip's 512 resident ones: as many as fit one round, at least 128 k each; from
+// a round on, up to four where they fill the last round. A second-stage product of one segment has
+// ct x vt outputs per vector over K = (P, v'): 30 tiles over K = 30720 at (30, 210, 960) with 15
+// vectors took 1606 us unsplit, 17 splits of it 120 us.
+int f64_ksplit(long units, long K) {
+  constexpr long kResident = 512;
+  if (units <= 0) return 1;
+  if (units <= kResident / 2) return (int)std::max<long>(1, std::min<long>(kResident / units, K / 128));
+  return eps_ksplit(units, kResident, K, 16);
+}
+
+// Output tiles of the narrow FP64 kernel.
+long f64_narrow_tiles(long M, long N) {
+  const long w = 16L * f64_narrow_tn((int)N);
+  return (M + 127) / 128 * ((N + w - 1) / w);
+}
 
 MatmulPlan plan_matmul(const xtpgpu_bseop_s* op, int precision, long k) {
   MatmulPlan pl;
@@ -1176,8 +1170,55 @@ MatmulPlan plan_matmul(const xtpgpu_bseop_s* op, int precision, long k) {
     const GemmDims dd = make_dims<64, 64>((int)P, (int)k, (int)Np, 1, pick_ksplit(tiles, Np, 16), 16, false);
     pl.part = std::max(pl.part, (size_t)dd.ksplit * P * k * 8);
     pl.wbuf = (size_t)op->Pp * k * 8;
+    pl.part_more = (size_t)f64_ksplit(f64_narrow_tiles(op->N, k), op->Pp) * op->N * k * 8;
   }
+  if ((op->cd || op->cd2) && !m16)
+    pl.part_more = std::max(pl.part_more,
+                            (size_t)f64_ksplit(f64_narrow_tiles(ct, vt) * k, P * op->vtp) * ct * vt * k * 8);
+  pl.part_more = std::max(pl.part_more, pl.part);
   return pl;
+}
+
+// Y[b][r] += alpha * (sum over the K splits of part[q][b][r], in order); grid (rows of n / 256, batch)
+template <typename T>
+__global__ __launch_bounds__(256) void add_partials_kernel(const T* __restrict__ part, int nsp, long n,
+                                                           double* __restrict__ Y, long ldy, double alpha) {
+  const long r = (long)blockIdx.x * 256 + threadIdx.x;
+  if (r >= n) return;
+  const long b = blockIdx.y, stride = n * gridDim.y;
+  const T* p = part + b * n + r;
+  double acc = 0.0;
+  for (int q = 0; q < nsp; ++q) acc += (double)p[q * stride];
+  Y[b * ldy + r] += alpha * acc;
+}
+template <typename T>
+void add_partials(hipStream_t st, const T* part, int nsp, long n, long batch, double* Y, long ldy, double alpha) {
+  hipLaunchKernelGGL(add_partials_kernel<T>, dim3((unsigned)((n + 255) / 256), (unsigned)batch), dim3(256), 0, st, part,
+                     nsp, n, Y, ldy, alpha);
+  XG_HIP(hipGetLastError());
+}
+
+// Padded copies of the k input vectors (FP64, and BF16 hi / lo when Xh / Xl are given) and the start
+// of the result: Y = cqp (H_c - H_v) X for a diagonal Hqp (hc given), else 0. One thread per padded
+// element, grid (k * vt, row length / 256).
+__global__ __launch_bounds__(256) void prep_vectors_kernel(const double* __restrict__ X, long ldx, int vt, int ct, int ctp,
+                                                           double* __restrict__ Xp, unsigned short* __restrict__ Xh,
+                                                           unsigned short* __restrict__ Xl, double* __restrict__ Y,
+                                                           long ldy, const double* __restrict__ hc,
+                                                           const double* __restrict__ hv, double cqp) {
+  const int c = blockIdx.y * 256 + threadIdx.x;
+  if (c >= ctp) return;
+  const int col = blockIdx.x, kv = col / vt, v = col - kv * vt;
+  const double x = c < ct ? X[kv * ldx + (long)v * ct + c] : 0.0;
+  const long i = (long)col * ctp + c;
+  Xp[i] = x;
+  if (Xh) {
+    unsigned short h, l;
+    split_bf16(x, h, l);
+    Xh[i] = h;
+    if (Xl) Xl[i] = l;
+  }
+  if (c < ct) Y[kv * ldy + (long)v * ct + c] = hc ? cqp * (hc[c] - hv[v]) * x : 0.0;
 }
 
 // BSE_OPERATOR::matmul (bse_operator.cc:39-119) on device buffers. Scratch comes from the
@@ -1224,45 +1265,37 @@ void bse_matmul_impl(xtpgpu_bseop op, int precision, const double* X, long ldx, 
   double* Xp = static_cast<double*>(buf(op->xp, pl.xp));
   unsigned short* Xh = need16 ? static_cast<unsigned short*>(buf(op->xh, pl.xh)) : nullptr;
   unsigned short* Xl = need16 && split ? static_cast<unsigned short*>(buf(op->xl, pl.xl)) : nullptr;
-  void* part_p = buf(op->part, pl.part);
+  size_t part_bytes = pl.part_more;
+  if (arena && arena->left() < ScratchArena::up(pl.part_more) + ScratchArena::up(pl.wbuf) +
+                                   ScratchArena::up(pl.per_p * (size_t)P) + 4096)
+    part_bytes = pl.part;  // the region is kept for the aux chunks
+  void* part_p = buf(op->part, part_bytes);
   double* Wb = op->cx ? static_cast<double*>(zbuf(op->wbuf, pl.wbuf)) : nullptr;
-  launch_map(st, (size_t)Np * k, [=] __device__(size_t i) {
-    long col = (long)(i / (size_t)ctp), c = (long)(i % (size_t)ctp);  // col = kv*vt + v
-    long kv = col / vt, v = col % vt;
-    double x = c < ct ? X[kv * ldx + v * ct + c] : 0.0;
-    Xp[i] = x;
-    if (Xh) {
-      unsigned short h, l;
-      split_bf16(x, h, l);
-      Xh[i] = h;
-      if (Xl) Xl[i] = l;
-    }
-  });
-  // Y = 0
-  launch_map(st, (size_t)N * k, [=] __device__(size_t i) { Y[(i / N) * ldy + i % N] = 0.0; });
+  // K splits of an FP64 product with `out` result values that the partials' buffer holds
+  auto splits64 = [&](long units, long K, size_t out) {
+    return (int)std::min<size_t>((size_t)f64_ksplit(units, K), part_bytes / (out * 8));
+  };
+  const bool diag_qp = op->cqp && op->hqp_diag;
+  {
+    ProfScope prof(pctx, diag_qp ? "hqp" : nullptr, 2.0 * N * k, 8.0 * 3.0 * N * k);
+    hipLaunchKernelGGL(prep_vectors_kernel, dim3((unsigned)(k * vt), (unsigned)((ctp + 255) / 256)), dim3(256), 0, st, X,
+                       ldx, (int)vt, (int)ct, (int)ctp, Xp, Xh, Xl, Y, ldy, diag_qp ? op->hcd.as<double>() : nullptr,
+                       diag_qp ? op->hvd.as<double>() : nullptr, (double)op->cqp);
+    XG_HIP(hipGetLastError());
+  }
 
   // ---------------- Hqp (bse_operator.cc:121-132): cqp (H_c^T X - X H_v) per vector
-  if (op->cqp) {
-    ProfScope prof(pctx, "hqp", 2.0 * N * k * (op->hqp_diag ? 1.0 : (double)(ct + vt)), 8.0 * 3.0 * N * k);
+  if (op->cqp && !op->hqp_diag) {
+    ProfScope prof(pctx, "hqp", 2.0 * N * k * (double)(ct + vt), 8.0 * 3.0 * N * k);
     const double cqp = op->cqp;
-    if (op->hqp_diag) {
-      const double* hc = op->hcd.as<double>();
-      const double* hv = op->hvd.as<double>();
-      launch_map(st, (size_t)N * k, [=] __device__(size_t i) {
-        long kv = (long)(i / N), r = (long)(i % N);
-        long v = r / ct, c = r % ct;
-        Y[kv * ldy + r] += cqp * (hc[c] - hv[v]) * Xp[(kv * vt + v) * ctp + c];
-      });
-    } else {
-      // out_kv(c1, v1) += cqp * sum_c' Hc(c', c1) X_kv(c', v1)   (batched over kv)
-      gemm64<true, true>(st, (int)ct, (int)vt, (int)ct, (int)k, 1, Opnd<double>{op->hc.as<double>(), nullptr, ct, 0},
-                         Opnd<double>{Xp, nullptr, ctp, vt * ctp}, nullptr, 0, false,
-                         EpiStore{Y, 1, ct, ldy, cqp, 1.0});
-      // out_kv(c1, v1) -= cqp * sum_v' X_kv(c1, v') Hv(v', v1)
-      gemm64<false, true>(st, (int)ct, (int)vt, (int)vt, (int)k, 1, Opnd<double>{Xp, nullptr, ctp, vt * ctp},
-                          Opnd<double>{op->hv.as<double>(), nullptr, vt, 0}, nullptr, 0, false,
-                          EpiStore{Y, 1, ct, ldy, -cqp, 1.0});
-    }
+    // out_kv(c1, v1) += cqp * sum_c' Hc(c', c1) X_kv(c', v1)   (batched over kv)
+    gemm64<true, true>(st, (int)ct, (int)vt, (int)ct, (int)k, 1, Opnd<double>{op->hc.as<double>(), nullptr, ct, 0},
+                       Opnd<double>{Xp, nullptr, ctp, vt * ctp}, false,
+                       EpiStore{Y, 1, ct, ldy, cqp, 1.0});
+    // out_kv(c1, v1) -= cqp * sum_v' X_kv(c1, v') Hv(v', v1)
+    gemm64<false, true>(st, (int)ct, (int)vt, (int)vt, (int)k, 1, Opnd<double>{Xp, nullptr, ctp, vt * ctp},
+                        Opnd<double>{op->hv.as<double>(), nullptr, vt, 0}, false,
+                        EpiStore{Y, 1, ct, ldy, -cqp, 1.0});
   }
 
   // aux chunk for the two-stage Hd / Hd2 contraction (first-stage scratch <= budget, or what the
@@ -1284,6 +1317,21 @@ void bse_matmul_impl(xtpgpu_bseop op, int precision, const double* X, long ldx, 
       if (split) s1b = static_cast<unsigned char*>(zbuf(op->s1l, s1n * 2));
     }
   }
+
+  // second stage in FP64: Y[kv] += alpha sum_(P, v') A[kv](c1, (P, v')) B[kv](v1, (P, v'))
+  auto stage2_fp64 = [&](Opnd<double> A, Opnd<double> B, long np, double alpha) {
+    const long K2 = np * vtp;
+    const int ks = splits64(f64_narrow_tiles(ct, vt) * k, K2, (size_t)ct * vt * k);
+    if (ks > 1 && f64_lds_ok(A, B, (int)K2, nullptr, 0)) {
+      double* pt = static_cast<double*>(part_p);
+      const GemmDims dd = make_dims<128, 16>((int)ct, (int)vt, (int)K2, (int)k, ks, 16, false);
+      XG_HIP(launch_f64_narrow(st, (int)ct, (int)vt, (int)K2, (int)k, ks, A, B, EpiPartial{pt, (int)ct, (int)vt, (int)k}));
+      add_partials(st, pt, dd.ksplit, ct * vt, k, Y, ldy, alpha);
+    } else {
+      gemm64<true, true>(st, (int)ct, (int)vt, (int)K2, (int)k, 1, A, B, false,
+                         EpiStore{Y, 1, ct, ldy, alpha, 1.0});
+    }
+  };
 
   // ---------------- Hd (bse_operator.cc:70-89, PrepareMatrix1/2): -cd sum_P eps_P M^P_cc' X M^P_vv'^T
   if (op->cd) {
@@ -1319,13 +1367,11 @@ void bse_matmul_impl(xtpgpu_bseop op, int precision, const double* X, long ldx, 
         {
           ProfScope prof(pctx, "hd_stage1_fp64", f1, b1);
           gemm64<true, true>(st, (int)M1, (int)N1, (int)round8(ct), 1, 1, Opnd<double>{mcc, nullptr, ctp, 0},
-                             Opnd<double>{Xp, nullptr, ctp, 0}, nullptr, 0, false, e1);
+                             Opnd<double>{Xp, nullptr, ctp, 0}, false, e1);
         }
         ProfScope prof(pctx, "hd_stage2_fp64", f2, b2);
-        gemm64<true, true>(st, (int)ct, (int)vt, (int)(np * vtp), (int)k, 1,
-                           Opnd<double>{S, nullptr, k * np * vtp, np * vtp},
-                           Opnd<double>{op->Bvv.as<double>() + p0 * vtp, nullptr, P * vtp, 0}, nullptr, 0, false,
-                           EpiStore{Y, 1, ct, ldy, alpha, 1.0});
+        stage2_fp64(Opnd<double>{S, nullptr, k * np * vtp, np * vtp},
+                    Opnd<double>{op->Bvv.as<double>() + p0 * vtp, nullptr, P * vtp, 0}, np, alpha);
       } else {
         unsigned short* Sh = reinterpret_cast<unsigned short*>(s1a);
         unsigned short* Sl = split ? reinterpret_cast<unsigned short*>(s1b) : nullptr;
@@ -1355,14 +1401,7 @@ void bse_matmul_impl(xtpgpu_bseop op, int precision, const double* X, long ldx, 
           float* pt = static_cast<float*>(part_p);
           XG_HIP((launch_gemm_bf16<128, 128, true, true>(st, dd, s2a, s2b, nullptr, 0, split, EpiPart32{pt, ct, vt, k},
                                                          true)));
-          const long nout = k * ct * vt, nsp = dd.ksplit, ctl = ct, vtl = vt;
-          launch_map(st, (size_t)nout, [=] __device__(size_t i) {
-            double acc = 0.0;
-            for (long q = 0; q < nsp; ++q) acc += (double)pt[q * nout + (long)i];
-            const long b = (long)i / (ctl * vtl), r = (long)i - b * ctl * vtl;
-            const long n = r / ctl, m = r - n * ctl;
-            Y[b * ldy + n * ctl + m] += alpha * acc;
-          });
+          add_partials(st, pt, dd.ksplit, ct * vt, k, Y, ldy, alpha);
         } else {
           gemm16<true, true>(st, (int)ct, (int)vt, (int)(np * vtp), (int)k, 1, s2a, s2b, nullptr, 0, split, false,
                              EpiStore{Y, 1, ct, ldy, alpha, 1.0});
@@ -1385,11 +1424,9 @@ void bse_matmul_impl(xtpgpu_bseop op, int precision, const double* X, long ldx, 
         e1.S64 = S;
         gemm64<true, true>(st, (int)M1, (int)N1, (int)round8(ct), 1, 1,
                            Opnd<double>{op->Mvc.as<double>() + p0 * Np, nullptr, ctp, 0},
-                           Opnd<double>{Xp, nullptr, ctp, 0}, nullptr, 0, false, e1);
-        gemm64<true, true>(st, (int)ct, (int)vt, (int)(np * vtp), (int)k, 1,
-                           Opnd<double>{op->McvT.as<double>() + p0 * vtp, nullptr, P * vtp, 0},
-                           Opnd<double>{S, nullptr, np * vtp, vt * np * vtp}, nullptr, 0, false,
-                           EpiStore{Y, 1, ct, ldy, alpha, 1.0});
+                           Opnd<double>{Xp, nullptr, ctp, 0}, false, e1);
+        stage2_fp64(Opnd<double>{op->McvT.as<double>() + p0 * vtp, nullptr, P * vtp, 0},
+                    Opnd<double>{S, nullptr, np * vtp, vt * np * vtp}, np, alpha);
       } else {
         unsigned short* Sh = reinterpret_cast<unsigned short*>(s1a);
         unsigned short* Sl = split ? reinterpret_cast<unsigned short*>(s1b) : nullptr;
@@ -1416,7 +1453,7 @@ void bse_matmul_impl(xtpgpu_bseop op, int precision, const double* X, long ldx, 
     GemmDims dd = make_dims<64, 64>((int)P, (int)k, (int)Np, 1, ks, 16, false);
     double* part = static_cast<double*>(part_p);
     gemm64<true, true>(st, (int)P, (int)k, (int)Np, 1, ks, Opnd<double>{op->Mvc.as<double>(), nullptr, Np, 0},
-                       Opnd<double>{Xp, nullptr, Np, 0}, nullptr, 0, false, EpiPartial{part, (int)P, (int)k, 1});
+                       Opnd<double>{Xp, nullptr, Np, 0}, false, EpiPartial{part, (int)P, (int)k, 1});
     // W[kv][Pp] (pads stay zero)
     const int nsp = dd.ksplit;
     launch_map(st, (size_t)P * k, [=] __device__(size_t i) {
@@ -1425,9 +1462,16 @@ void bse_matmul_impl(xtpgpu_bseop op, int precision, const double* X, long ldx, 
       for (int q = 0; q < nsp; ++q) acc += part[(long)q * P * k + i];
       Wb[kv * Pp + p] = acc;
     });
-    gemm64<true, true>(st, (int)N, (int)k, (int)Pp, 1, 1, Opnd<double>{op->MvcT.as<double>(), nullptr, Pp, 0},
-                       Opnd<double>{Wb, nullptr, Pp, 0}, nullptr, 0, false,
-                       EpiStore{Y, 1, ldy, 0, (double)op->cx, 1.0});
+    const Opnd<double> vt_op{op->MvcT.as<double>(), nullptr, Pp, 0}, w_op{Wb, nullptr, Pp, 0};
+    const int ksb = splits64(f64_narrow_tiles(N, k), Pp, (size_t)N * k);
+    if (ksb > 1 && f64_lds_ok(vt_op, w_op, (int)Pp, nullptr, 0)) {
+      const GemmDims db = make_dims<128, 16>((int)N, (int)k, (int)Pp, 1, ksb, 16, false);
+      XG_HIP(launch_f64_narrow(st, (int)N, (int)k, (int)Pp, 1, ksb, vt_op, w_op, EpiPartial{part, (int)N, (int)k, 1}));
+      add_partials(st, part, db.ksplit, N, k, Y, ldy, (double)op->cx);
+    } else {
+      gemm64<true, true>(st, (int)N, (int)k, (int)Pp, 1, 1, vt_op, w_op, false,
+                         EpiStore{Y, 1, ldy, 0, (double)op->cx, 1.0});
+    }
   }
 }
 
@@ -1874,7 +1918,7 @@ extern "C" int xtpgpu_bse_create_streamed(xtpgpu_ctx ctx, xtpgpu_mmn_chunk_fn so
       // p * vtp + j) and W's column q read as row q (W = eps^-1(0) is symmetric)
       gemm64<false, true>(st, (int)vtp, (int)P, (int)P, (int)vt, 1,
                           Opnd<double>{braw.as<double>(), nullptr, vtp, P * vtp},
-                          Opnd<double>{wm.as<double>(), nullptr, P, 0}, nullptr, 0, false,
+                          Opnd<double>{wm.as<double>(), nullptr, P, 0}, false,
                           EpiStore{Bvv, 1, vtp, P * vtp, 1.0, 0.0});
       XG_HIP(hipStreamSynchronize(st));
     }
