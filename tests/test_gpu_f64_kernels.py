@@ -57,3 +57,44 @@ def test_products_narrow_tiles(o, v, P, k, c):
     x = rng.normal(size=(o * v, k))
     ref = X.bse_dense(*c, eps, M, H, o - 1, 0, 0, n - 1) @ x
     assert np.linalg.norm(op.matmul(x) - ref) <= TOL * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("o,v,P,r", [(1, 2, 3, 1), (3, 7, 9, 2), (5, 16, 20, 3), (9, 33, 140, 1), (17, 20, 15, 4)])
+@pytest.mark.parametrize("a,b,with_y", [((1, 2, 1, 0), (0, 2, 0, 1), True), ((1, 2, 1, 0), None, False),
+                                        ((1, 0, 1, 0), (0, 0, 0, 1), True), ((0, 1, 0, 1), (0, 1, 0, 1), True),
+                                        ((0, 0, 0, 1), None, False), ((1, 2, 1, 0), (0, 2, 0, 1), False)])
+def test_weighted_adjoint_forms(o, v, P, r, a, b, with_y):
+    """Every combination of exchange and Hd2 parts, with and without Y, against the formula written out."""
+    import ctypes as C
+    rng = np.random.default_rng(o + 10 * v + P + r)
+    M, e, n = tensor(rng, o, v, P, 0.3), energies(rng, o, v), o + v
+    eps = rng.uniform(-0.2, 1.0, P)
+    eps[0] = 0.0
+    t = px.TCMatrix_gwbse().Initialize(P, 0, n - 1, 0, n - 1).set_tensor(M)
+    opt = px.BSEOperator_Options(o - 1, 0, 0, 0, n - 1)
+    A = px.BSE_OPERATOR(*a, eps, t, np.diag(e)).configure(opt)
+    B = px.BSE_OPERATOR(*b, eps, t, np.diag(e)).configure(opt) if b else None
+    Xv = np.asfortranarray(rng.normal(size=(o * v, r)))
+    Yv = np.asfortranarray(rng.normal(size=(o * v, r))) if with_y else None
+    w = rng.normal(size=r)
+    w[0] = 0.0 if r > 2 else w[0]
+    de, buf = np.zeros(n), px.DeviceBuffer(t.ctx, P * o * v * 8)
+    px._check(px.lib().xtpgpu_bse_adjoint_weighted_device(
+        A.h, B.h if B else None, r, px._dptr(Xv), px._dptr(Yv) if with_y else None, o * v, px._dptr(w), px._dptr(de),
+        C.c_void_p(buf.ptr.value)))
+    got = buf.download((P, o, v), order="C")
+    m = M[:o, o:, :].transpose(2, 0, 1)
+    ref, dref = np.zeros((P, o, v)), np.zeros(n)
+    cxb, c2b = (b[1], b[3]) if b else (0, 0)
+    for i in range(r):
+        x = Xv[:, i].reshape(o, v)
+        y = Yv[:, i].reshape(o, v) if with_y else np.zeros((o, v))
+        sx, sy = (np.einsum("pvc,vc->p", m, q)[:, None, None] for q in (x, y))
+        g = 2 * a[1] * (x * sx + y * sy) + 2 * cxb * (x * sy + y * sx)
+        lmr = lambda p, q: np.einsum("vc,puc,ud->pvd", p, m, q)  # noqa: E731
+        g = g - 2 * eps[:, None, None] * (c2b * (lmr(y, x) + lmr(x, y)) + a[3] * (lmr(x, x) + lmr(y, y)))
+        ref += w[i] * g
+        dref[:o] -= w[i] * a[0] * (x * x + y * y).sum(1)
+        dref[o:] += w[i] * a[0] * (x * x + y * y).sum(0)
+    assert np.linalg.norm(got - ref) <= TOL * max(np.linalg.norm(ref), 1e-300)
+    assert np.linalg.norm(de - dref) <= TOL * max(np.linalg.norm(dref), 1e-300)

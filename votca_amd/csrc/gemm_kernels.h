@@ -121,7 +121,7 @@ __device__ __forceinline__ float bf16_bits_to_f(unsigned short h) {
 
 // Epilogue protocol. Every epilogue is callable as epi(b, ks, m, n, v). A "separable" one
 // (kSeparable = true) also splits its output address into a row term and a column term:
-//   typename Epi::Row r = epi.row(b, ks, m);  long c = epi.col(b, n);  epi.put(r, c, v);
+//   typename Epi::Row r = epi.row(b, ks, m);  auto c = epi.col(b, n);  epi.put(r, c, v);
 // so a tile computes the (division-heavy) index arithmetic once per row and once per column
 // instead of once per element.
 template <class E, class = void>
@@ -135,13 +135,14 @@ template <int TM, int TN, int NR, class Epi, class Acc, class RowOf, class ColOf
 __device__ __forceinline__ void epilogue_store(const GemmDims& d, const Epi& epi, int b, int ks, const Acc& acc,
                                                RowOf row_of, ColOf col_of) {
   if constexpr (epi_separable<Epi>::value) {
-    long co[TN];
+    using Col = decltype(epi.col(0, 0));
+    Col co[TN];
     bool cv[TN];
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
       const int gn = col_of(j);
       cv[j] = gn < d.N;
-      co[j] = cv[j] ? epi.col(b, gn) : 0;
+      co[j] = cv[j] ? epi.col(b, gn) : Col{};
     }
 #pragma unroll
     for (int i = 0; i < TM; ++i)
