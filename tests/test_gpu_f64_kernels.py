@@ -98,3 +98,32 @@ def test_weighted_adjoint_forms(o, v, P, r, a, b, with_y):
         dref[o:] += w[i] * a[0] * (x * x + y * y).sum(0)
     assert np.linalg.norm(got - ref) <= TOL * max(np.linalg.norm(ref), 1e-300)
     assert np.linalg.norm(de - dref) <= TOL * max(np.linalg.norm(dref), 1e-300)
+
+
+@pytest.mark.parametrize("o,v,P,levels,per", [(1, 1, 1, 1, 1), (2, 61, 31, 3, 2), (2, 62, 32, 2, 7), (3, 62, 33, 4, 8),
+                                              (5, 123, 64, 2, 9), (5, 130, 40, 1, 17), (7, 240, 65, 6, 3),
+                                              (9, 300, 20, 5, 5)])
+def test_sigma_ppm_row_widths(o, v, P, levels, per):
+    """Row lengths around the 64, 128 and 256-element steps, group sizes 1..8 and beyond, skipped weights."""
+    rng = np.random.default_rng(o + v + P)
+    M, e, n = tensor(rng, o, v, P), energies(rng, o, v), o + v
+    t = px.TCMatrix_gwbse().Initialize(P, 0, n - 1, 0, n - 1).set_tensor(M)
+    rpa = px.RPA(t)
+    rpa.configure(o - 1, 0, n - 1)
+    q0 = max(0, o - levels // 2)
+    s = px.Sigma_PPM(t, rpa).configure(o - 1, q0, q0 + levels - 1, 0, n - 1)
+    s.ppm_weight, s.ppm_freq = rng.uniform(0, 0.5, P), rng.uniform(0.5, 2.0, P)
+    s.ppm_weight[rng.random(P) < 0.2] = 0.0
+    s.set_rpa_energies(e)
+    lv = rng.permutation(np.repeat(np.arange(levels), per))
+    om = rng.uniform(-2, 2, lv.size)
+    sig, dsig = s.diag_batch(lv, om)
+    f = s.ppm_freq[:, None]
+    sh = np.where(np.arange(n)[None, :] < o, f, -f) - e[None, :]
+    for i in range(lv.size):
+        m2 = (0.5 * s.ppm_weight * s.ppm_freq)[:, None] * M[q0 + lv[i]].T ** 2
+        tt = om[i] + sh
+        den = tt * tt + 1e-6
+        # each sum relative to the sum of its terms' magnitudes
+        for got, terms in ((sig[i], m2 * tt / den), (dsig[i], m2 * (1e-6 - tt * tt) / (den * den))):
+            assert abs(got - terms.sum()) <= TOL * max(np.abs(terms).sum(), 1e-300)
