@@ -39,9 +39,9 @@ PEAK = {"fp64": 78.6e12, "bf16": 2.5e15, "hbm": 8.0e12}
 # WRITE_SIZE 1.0 GiB -> x1.0); FETCH_SIZE 4.462e6 / 3.159e6 KiB, WRITE_SIZE 3.450e6 / 3.490e6 KiB
 # per dispatch. The P-chunk keeps the stage-1 intermediate under 3 GiB: 286 levels for the split
 # form (two output planes), 573 for plain BF16.
-HD_STAGE1_TRAFFIC = {"bf16x3": {"read": 4.462e6 * 2.0 * 1024, "write": 3.450e6 * 1.0 * 1024,
+HD_STAGE1_TRAFFIC = {"bf16x3": {"read": 2.745e6 * 2.0 * 1024, "write": 4.090e6 * 1.0 * 1024,
                                 "launch": "30-column H X stage-1 launch, split BF16 (P-chunk 286)"},
-                     "bf16": {"read": 3.159e6 * 2.0 * 1024, "write": 3.490e6 * 1.0 * 1024,
+                     "bf16": {"read": 2.371e6 * 2.0 * 1024, "write": 4.060e6 * 1.0 * 1024,
                               "launch": "30-column H X stage-1 launch, plain BF16 (P-chunk 573)"}}
 
 
@@ -49,10 +49,10 @@ HD_STAGE1_TRAFFIC = {"bf16x3": {"read": 4.462e6 * 2.0 * 1024, "write": 3.450e6 *
 # the clock the chip holds under the load (GRBM_GUI_ACTIVE / 8 XCDs / duration), MFMA busy
 # (SQ_VALU_MFMA_BUSY_CYCLES / cycles / 1024 SIMDs) and the share of cycles the L1 waits on L2 data
 # (TCP_PENDING_STALL_CYCLES_sum / 256 CUs / cycles).
-HD_STAGE1_COUNTERS = {"bf16x3": {"clock_GHz": 1.95, "peak_at_clock_tflops": 2500.0 * 1.95 / 2.4,
-                                 "mfma_busy": 0.446, "tcp_pending_stall": 0.330},
-                      "bf16": {"clock_GHz": 1.81, "peak_at_clock_tflops": 2500.0 * 1.81 / 2.4,
-                               "mfma_busy": 0.373, "tcp_pending_stall": 0.365}}
+HD_STAGE1_COUNTERS = {"bf16x3": {"clock_GHz": 1.98, "peak_at_clock_tflops": 2500.0 * 1.98 / 2.4,
+                                 "mfma_busy": 0.476, "tcp_pending_stall": 0.487},
+                      "bf16": {"clock_GHz": 2.13, "peak_at_clock_tflops": 2500.0 * 2.13 / 2.4,
+                               "mfma_busy": 0.337, "tcp_pending_stall": 0.560}}
 
 
 def log(*a):
@@ -1059,15 +1059,11 @@ def main():
     ach = tm["flops"] / max(tm["ms"] / 1e3, 1e-30)
     issue = 3.0 if dom == "bf16x3" else 1.0
     choice = os.environ.get("XTPGPU_BF16_KERNEL", "")
-    kname = {"staged32": "gemm_bf16_kernel<128,128,..,EpiStage1,32>", "pipe": "gemm_bf16x3_pipe_kernel<..,EpiStage1>",
-             "big": "gemm_bf16_kernel<256,256,..,EpiStage1,32>", "tall": "gemm_bf16_kernel<256,128,..,EpiStage1,64,512>",
-             "wide": "gemm_bf16_kernel<128,128,..,EpiStage1,128>" if dom == "bf16" else None,
-             }.get(choice) or ("gemm_bf16_kernel<128,128,..,EpiStage1,64,256,DB=0,MINW=3>" if dom == "bf16"
-                               else "gemm_bf16_kernel<128,128,..,EpiStage1,64>")
+    kname = {"staged32": "gemm_bf16_kernel<128,128,..,EpiStage1,32>", "staged64": "gemm_bf16_kernel<128,128,..,EpiStage1,64>",
+             }.get(choice, "gemm_bf16_ring_kernel<256 x 256,..,EpiStage1>")
     kname = kname.replace("<", "<" + ("split," if dom == "bf16x3" else "plain,"), 1)
     traffic = (HD_STAGE1_TRAFFIC[dom]["read"] + HD_STAGE1_TRAFFIC[dom]["write"]
-               if dom in HD_STAGE1_TRAFFIC and "512" not in kname and "256,256" not in kname and "pipe" not in kname
-               else None)
+               if dom in HD_STAGE1_TRAFFIC and "ring" in kname else None)
     roofline = {"bound": "mfma", "kernel": f"hd_stage1 {dom} ({kname})",
                 "achieved": ach / 1e12,
                 "peak": PEAK["bf16"] / 1e12, "unit": "TFLOP/s", "frac": ach / PEAK["bf16"], "traffic": traffic,
@@ -1086,7 +1082,7 @@ def main():
     if "fp64" in res:
         t64 = res["fp64"]["hd_stage1"]["fp64"]
         a64 = t64["flops"] / max(t64["ms"] / 1e3, 1e-30)
-        roofline["fp64_form"] = {"kernel": "hd_stage1_fp64 (gemm_f64_kernel<128,128,..,EpiStage1>)",
+        roofline["fp64_form"] = {"kernel": "hd_stage1_fp64 (gemm_f64_lds_kernel<128 x 64,..,EpiStage1>)",
                                  "achieved": a64 / 1e12, "peak": PEAK["fp64"] / 1e12, "frac": a64 / PEAK["fp64"],
                                  "avg_launch_ms": t64["ms"] / max(1, t64["launches"])}
 

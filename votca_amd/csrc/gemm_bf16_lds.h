@@ -1,0 +1,266 @@
+// BF16 GEMM for gfx950 with operands moved straight to LDS (lds_dma.h).
+//
+//   C[b](m,n) = epilogue( sum_k A[b](m,k) B[b](n,k) )   (both operands K-contiguous bf16 rows)
+//   SPLIT:   operands a = a_hi + a_lo, products hi*hi + hi*lo + lo*hi (FP32 accumulation)
+//
+// WR x WC waves, wave tile 16 TM x 16 TN of v_mfma_f32_16x16x32_bf16 tiles, a ring of STAGES LDS
+// stages (64 k, or 32 k of both planes), one barrier per stage. Three forms are used:
+//   256 x 256, 16 waves of 64 x 64, 2 stages: large products. What bounds the 128 x 128
+//     register-staged tiles of gemm_bf16_kernel is LDS traffic (fragment reads plus staged writes
+//     come to the 128 bytes a CU moves per cycle at half of the MFMA rate); twice the tile edge halves
+//     the writes, which the loads do themselves, and four waves per SIMD cover the barrier. Stage 1
+//     of the Hd contraction at 128700 x 3000 x 900, split / plain: 2.64 / 0.98 ms with 128 x 128
+//     tiles, 2.00 / 0.83 here (347 / 840 TFLOP/s); eight waves of 128 x 64 2.11 / 0.85, of 64 x 128
+//     2.12 / 0.84, 256 x 128 tiles 2.42 / 1.01; the same without the stores 1.65 / 0.60.
+//   256 rows x (16 TN) columns, 8 waves of 32 rows, 3 stages: second-stage products with enough of
+//     them (900 x 100 per vector, K = 29744, 30 vectors: 1193 -> 1054 us split, 440 -> 410 plain).
+//   32 rows x (32, 64, 128) columns, 2 x 2 waves, 4 stages: the same with few outputs, where each
+//     workgroup walks a long K alone and the ring hides the latency (210 x 30 per vector,
+//     K = 30720 in 4 splits, 8 vectors: 197 -> 67 us split, 99 -> 35 plain).
+//
+// The MFMAs take B as their first operand, so a lane holds four consecutive n of one m (n =
+// 4 (lane / 16) + r, m = lane % 16). Every output accumulates its 32-k steps in order, per step
+// hi*hi, hi*lo, lo*hi, as in gemm_bf16_kernel: the results are those of the 128 x 128 tiles bit for bit.
+#pragma once
+#include "lds_dma.h"
+
+namespace xg {
+
+// Epilogues whose rows are BF16 planes (kPlanes): the kernel rounds to hi (and lo, planes() == 2) and
+// stores four consecutive columns of a row at once, which planes_ok() allows: 4 columns from a
+// multiple of four are adjacent in memory, 8-byte aligned. Row m carries factor(m).
+template <class E, class = void>
+struct epi_planes { static constexpr bool value = false; };
+template <class E>
+struct epi_planes<E, decltype((void)E::kPlanes)> { static constexpr bool value = E::kPlanes; };
+
+typedef unsigned short us4v __attribute__((ext_vector_type(4)));
+
+template <int TM, int TN, int WR, int WC, int STAGES, bool SPLIT, class Epi>
+__global__ __launch_bounds__(64 * WR * WC) void gemm_bf16_ring_kernel(
+    GemmDims d, Opnd<unsigned short> A, Opnd<unsigned short> B, Epi epi) {
+  constexpr int NW = WR * WC;
+  constexpr int KSTEP = SPLIT ? 32 : 64;  // k per stage
+  constexpr int NSUB = SPLIT ? 1 : 2;     // 32-k steps per stage
+  constexpr int NP = SPLIT ? 2 : 1;       // planes
+  constexpr int ROWB = 128;
+  constexpr int WM = 16 * TM, WN = 16 * TN;
+  constexpr int BM = WR * WM, BN = WC * WN;
+  constexpr int STAGE_BYTES = (BM + BN) * ROWB;
+  constexpr int G = STAGE_BYTES / 1024;       // 8-row groups, one load instruction each
+  constexpr int LPW = (G + NW - 1) / NW;      // load instructions per wave per stage
+  constexpr bool PADDED = G % NW != 0;        // some waves issue a load more: the others aim at a spare group
+  static_assert(STAGES >= 2 && (STAGES - 2) * LPW <= 63, "vmcnt range");
+  // the planes' epilogue turns 32 x WN pieces of both planes per wave in the same memory
+  constexpr int EPI_BYTES = epi_planes<Epi>::value && WN == 64 && TM % 2 == 0 ? NW * 2 * 32 * (2 * WN + 16) : 0;
+  constexpr int RING_BYTES = STAGES * STAGE_BYTES + (PADDED ? 1024 : 0);
+  constexpr int LDS_BYTES = RING_BYTES > EPI_BYTES ? RING_BYTES : EPI_BYTES;
+  static_assert(LDS_BYTES <= 160 * 1024, "LDS of a CU");
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[LDS_BYTES];
+
+  int tm, tn;
+  tile_of_block(d, tm, tn);
+  const int b = blockIdx.z, ks = blockIdx.y;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm0 = (wave / WC) * WM, wn0 = (wave % WC) * WN;
+  const int m0 = tm * BM, n0 = tn * BN;
+  const int kbeg = ks * d.kchunk;
+  const int kend = min(d.K, kbeg + d.kchunk);
+  const int nk = kend > kbeg ? (kend - kbeg + KSTEP - 1) / KSTEP : 0;
+  // a wave outside the matrix, or above the diagonal of a lower triangle, only loads
+  const bool active = m0 + wm0 < d.M && n0 + wn0 < d.N && !(d.lower && m0 + wm0 + WM <= n0 + wn0);
+
+  // this lane's source and first k for each of the wave's loads; rows past M / N read the last row (their
+  // results are not stored), k past the chunk reads the zero page
+  const unsigned short* zp = reinterpret_cast<const unsigned short*>(g_zero_page);
+  const unsigned short* src[LPW];
+  int kof[LPW];
+#pragma unroll
+  for (int j = 0; j < LPW; ++j) {
+    const int gi = NW * j + wave;
+    const int rr = 8 * gi + (lane >> 3);
+    const int c = lds_slot(rr, lane & 7);
+    const bool lo = SPLIT && c >= 4;
+    kof[j] = kbeg + (SPLIT ? 8 * (c & 3) : 8 * c);
+    if (PADDED && gi >= G) kof[j] = d.K;  // always the zero page
+    src[j] = (gi < BM / 8 ? (lo ? A.lo : A.p) + (long)b * A.bs + (long)min(m0 + rr, d.M - 1) * A.ld
+                          : (lo ? B.lo : B.p) + (long)b * B.bs + (long)min(n0 + rr - BM, d.N - 1) * B.ld) +
+             kof[j];
+  }
+  const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(lds_u4*)lds);
+  auto issue = [&](int stage, int dk) {  // the stage that starts dk after kbeg
+#pragma unroll
+    for (int j = 0; j < LPW; ++j) {
+      const unsigned short* g = kof[j] + dk < kend ? src[j] + dk : zp;
+      const int gi = NW * j + wave;
+      dma16(g, lds0 + (unsigned)(!PADDED || gi < G ? stage * STAGE_BYTES + gi * 1024 : STAGES * STAGE_BYTES));
+    }
+  };
+
+  f4v acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = (f4v){0.f, 0.f, 0.f, 0.f};
+
+  const int r16 = lane & 15, q = lane >> 4;
+  const unsigned char* fa = lds + (wm0 + r16) * ROWB;
+  const unsigned char* fb = lds + (BM + wn0 + r16) * ROWB;
+  // tile rows are multiples of 16, so a lane's slot depends on r16 and the chunk only
+  int slot[2];  // chunk q, chunk q + 4: the planes (SPLIT) or the 32-k halves
+#pragma unroll
+  for (int h = 0; h < 2; ++h) slot[h] = lds_slot(r16, q + 4 * h) * 16;
+
+  auto compute = [&](int stage) {
+    const unsigned char* sa = fa + stage * STAGE_BYTES;
+    const unsigned char* sb = fb + stage * STAGE_BYTES;
+#pragma unroll
+    for (int sub = 0; sub < NSUB; ++sub) {
+      bf8v bf[NP][TN], af[2][NP];
+      auto read_a = [&](int i) {
+#pragma unroll
+        for (int p = 0; p < NP; ++p)
+          af[i & 1][p] = *reinterpret_cast<const bf8v*>(sa + i * 16 * ROWB + slot[SPLIT ? p : sub]);
+      };
+      read_a(0);
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int p = 0; p < NP; ++p)
+          bf[p][j] = *reinterpret_cast<const bf8v*>(sb + j * 16 * ROWB + slot[SPLIT ? p : sub]);
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        if (i + 1 < TM) read_a(i + 1);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[0][j], af[i & 1][0], acc[i][j], 0, 0, 0);
+          if constexpr (SPLIT) {
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[1][j], af[i & 1][0], acc[i][j], 0, 0, 0);
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[0][j], af[i & 1][1], acc[i][j], 0, 0, 0);
+          }
+        }
+      }
+    }
+  };
+
+#pragma unroll
+  for (int t = 0; t < STAGES - 1; ++t)
+    if (t < nk) issue(t, t * KSTEP);
+  int cur = 0, fill = STAGES - 1;  // stage read in this step, stage filled during it
+  for (int t = 0; t < nk; ++t) {
+    // this wave's loads of step t have landed once at most the later issued steps' remain
+    if (STAGES >= 3 && t + STAGES - 2 < nk)
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((STAGES - 2) * LPW) : "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    // then every wave's have, and every wave has read the stage that the next issue fills
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (t + STAGES - 1 < nk) issue(fill, (t + STAGES - 1) * KSTEP);
+    if (active) compute(cur);
+    cur = cur + 1 == STAGES ? 0 : cur + 1;
+    fill = fill + 1 == STAGES ? 0 : fill + 1;
+  }
+  // lane: m = 16 i + lane % 16, n = 16 j + 4 (lane / 16) + r
+  if constexpr (epi_planes<Epi>::value && WN == 64 && TM % 2 == 0) {  // 16 lanes of four columns to a row
+    if (epi.planes_ok()) {
+      // A store of the fragments as they lie touches 16 rows in 32-byte pieces (70 cycles an
+      // instruction, a fifth of the whole product at K = 900), so each wave turns 32 rows at a time in
+      // LDS and stores 128-byte pieces of four rows.
+      constexpr int RS = 2 * WN + 16;  // LDS row: 36 dwords, conflict-free in both directions
+      constexpr int PLANE = 32 * RS;
+      __syncthreads();  // every wave has read the last stage
+      unsigned char* mine = lds + wave * (2 * PLANE);
+      const bool two = SPLIT && epi.planes() == 2;
+      const int gn = n0 + wn0 + 4 * r16;
+      const long co = gn < d.N ? epi.col(b, gn) : 0;
+#pragma unroll
+      for (int h = 0; h < TM / 2; ++h) {
+#pragma unroll
+        for (int i2 = 0; i2 < 2; ++i2) {
+          const int i = 2 * h + i2;
+          const float f = epi.factor(min(m0 + wm0 + 16 * i + r16, d.M - 1));
+#pragma unroll
+          for (int j = 0; j < TN; ++j) {
+            us4v vh, vl;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const float x = acc[i][j][r] * f;
+              vh[r] = bf16_bits_rn(x);
+              vl[r] = bf16_bits_rn(x - bf16_bits_to_f(vh[r]));
+            }
+            unsigned char* at = mine + (16 * i2 + r16) * RS + (16 * j + 4 * q) * 2;
+            *reinterpret_cast<us4v*>(at) = vh;
+            if (two) *reinterpret_cast<us4v*>(at + PLANE) = vl;
+          }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+        for (int it = 0; it < 8; ++it) {
+          const int row = 4 * it + q, gm = m0 + wm0 + 32 * h + row;
+          const unsigned char* at = mine + row * RS + r16 * 8;
+          const us4v vh = *reinterpret_cast<const us4v*>(at);
+          const us4v vl = *reinterpret_cast<const us4v*>(at + PLANE);
+          if (gm < d.M && gn < d.N) {
+            const long idx = epi.row(b, ks, gm).off + co;
+            __builtin_nontemporal_store(vh, reinterpret_cast<us4v*>(epi.Sh + idx));
+            if (two) __builtin_nontemporal_store(vl, reinterpret_cast<us4v*>(epi.Sl + idx));
+          }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      }
+      return;
+    }
+  }
+  if (!active) return;
+  const int mb = m0 + wm0 + r16, nb = n0 + wn0 + 4 * q;
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    const int gm = mb + 16 * i;
+    if (gm >= d.M) continue;
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int gn = nb + 16 * j + r;
+        if (gn < d.N) epi(b, ks, gm, gn, acc[i][j][r]);
+      }
+  }
+}
+
+template <int TM, int TN, int WR, int WC, int STAGES, class Epi>
+inline hipError_t launch_bf16_ring(hipStream_t st, const GemmDims& d, Opnd<unsigned short> A, Opnd<unsigned short> B,
+                                   bool split, Epi epi) {
+  const dim3 grid(gemm_tiles(d), d.ksplit, d.batch), block(64 * WR * WC);
+  if (split)
+    hipLaunchKernelGGL((gemm_bf16_ring_kernel<TM, TN, WR, WC, STAGES, true, Epi>), grid, block, 0, st, d, A, B, epi);
+  else
+    hipLaunchKernelGGL((gemm_bf16_ring_kernel<TM, TN, WR, WC, STAGES, false, Epi>), grid, block, 0, st, d, A, B, epi);
+  return hipGetLastError();
+}
+
+// Second-stage products (M rows per batch entry, N <= 128 columns, long K in d.ksplit chunks):
+// 256-row tiles where they give three quarters of the 256 CUs a workgroup, else 32-row tiles. bk: what
+// K chunks are multiples of (64 / 128, as for the 128 x 128 tiles).
+template <class Epi>
+inline hipError_t launch_bf16_tall(hipStream_t st, int M, int N, int K, int batch, int ksplit, int bk,
+                                   Opnd<unsigned short> A, Opnd<unsigned short> B, bool split, Epi epi) {
+  if ((long)((M + 255) / 256) * batch * ksplit >= 192) {
+    const int tn = (N + 15) / 16;
+#define XG_TALL(TN) \
+  return launch_bf16_ring<2, TN, 8, 1, 3>(st, make_dims<256, 16 * TN>(M, N, K, batch, ksplit, bk, false), A, B, split, epi)
+    if (tn <= 2) XG_TALL(2);
+    if (tn <= 4) XG_TALL(4);
+    if (tn <= 6) XG_TALL(6);
+    if (tn == 7) XG_TALL(7);
+    XG_TALL(8);
+#undef XG_TALL
+  }
+  if (N <= 32) return launch_bf16_ring<1, 1, 2, 2, 4>(st, make_dims<32, 32>(M, N, K, batch, ksplit, bk, false), A, B, split, epi);
+  if (N <= 64) return launch_bf16_ring<1, 2, 2, 2, 4>(st, make_dims<32, 64>(M, N, K, batch, ksplit, bk, false), A, B, split, epi);
+  return launch_bf16_ring<1, 4, 2, 2, 4>(st, make_dims<32, 128>(M, N, K, batch, ksplit, bk, false), A, B, split, epi);
+}
+
+}  // namespace xg

@@ -18,8 +18,7 @@
 // in steps of a wave tile. HAS_S: the weights of a K step are one more 128-byte LDS row and multiply
 // the B fragment after its read (TN multiplies against TM TN MFMAs), so no scaled copy of B is written.
 #pragma once
-#include "gemm_kernels.h"
-#include "gemm_lds.h"
+#include "lds_dma.h"
 
 namespace xg {
 

@@ -626,74 +626,6 @@ inline bool bf16_vec(const Opnd<unsigned short>& A, const Opnd<unsigned short>& 
   return vec_ok(A, K, 8) && vec_ok(B, K, 8) && (s_bs % 8 == 0);
 }
 
-// 256 x 256 block tile (wave tile 128 x 128, one wave per SIMD), K step 32, vector loads:
-// half the operand bytes per MFMA of the 128 x 128 tile. The caller checks bf16_vec().
-template <bool AK, bool BK_, class Epi>
-inline hipError_t launch_gemm_bf16_big(hipStream_t st, const GemmDims& d, Opnd<unsigned short> A,
-                                       Opnd<unsigned short> B, const float* s, long s_bs, bool split, Epi epi) {
-  static_assert(AK && BK_, "K-contiguous operands only");
-  dim3 grid(gemm_tiles(d), d.ksplit, d.batch);
-  if (split) {
-    if (s) hipLaunchKernelGGL((gemm_bf16_kernel<256, 256, AK, BK_, true, true, true, Epi, 32>), grid, dim3(256), 0, st, d, A, B, s, s_bs, epi);
-    else hipLaunchKernelGGL((gemm_bf16_kernel<256, 256, AK, BK_, true, false, true, Epi, 32>), grid, dim3(256), 0, st, d, A, B, s, s_bs, epi);
-  } else {
-    if (s) hipLaunchKernelGGL((gemm_bf16_kernel<256, 256, AK, BK_, false, true, true, Epi, 32>), grid, dim3(256), 0, st, d, A, B, s, s_bs, epi);
-    else hipLaunchKernelGGL((gemm_bf16_kernel<256, 256, AK, BK_, false, false, true, Epi, 32>), grid, dim3(256), 0, st, d, A, B, s, s_bs, epi);
-  }
-  return hipGetLastError();
-}
-
-// 256 x 128 block tile with 512 threads (8 waves, wave tile 64 x 64), K step 64, vector loads:
-// a quarter fewer operand bytes per MFMA than 128 x 128 at the same per-wave register budget.
-template <bool AK, bool BK_, class Epi>
-inline hipError_t launch_gemm_bf16_tall(hipStream_t st, const GemmDims& d, Opnd<unsigned short> A,
-                                        Opnd<unsigned short> B, const float* s, long s_bs, bool split, Epi epi) {
-  static_assert(AK && BK_, "K-contiguous operands only");
-  dim3 grid(gemm_tiles(d), d.ksplit, d.batch);
-  if (split) {
-    if (s) hipLaunchKernelGGL((gemm_bf16_kernel<256, 128, AK, BK_, true, true, true, Epi, 64, 512>), grid, dim3(512), 0, st, d, A, B, s, s_bs, epi);
-    else hipLaunchKernelGGL((gemm_bf16_kernel<256, 128, AK, BK_, true, false, true, Epi, 64, 512>), grid, dim3(512), 0, st, d, A, B, s, s_bs, epi);
-  } else {
-    if (s) hipLaunchKernelGGL((gemm_bf16_kernel<256, 128, AK, BK_, false, true, true, Epi, 64, 512>), grid, dim3(512), 0, st, d, A, B, s, s_bs, epi);
-    else hipLaunchKernelGGL((gemm_bf16_kernel<256, 128, AK, BK_, false, false, true, Epi, 64, 512>), grid, dim3(512), 0, st, d, A, B, s, s_bs, epi);
-  }
-  return hipGetLastError();
-}
-
-// 256 x 128 block tile with 256 threads (wave tile 128 x 64: 32 accumulator tiles per wave),
-// K step BKT, vector loads: 1.5x the MFMAs per LDS fragment read of the 64 x 64 wave tile.
-template <int BKT, bool AK, bool BK_, class Epi>
-inline hipError_t launch_gemm_bf16_wave128(hipStream_t st, const GemmDims& d, Opnd<unsigned short> A,
-                                           Opnd<unsigned short> B, const float* s, long s_bs, bool split, Epi epi) {
-  static_assert(AK && BK_, "K-contiguous operands only");
-  dim3 grid(gemm_tiles(d), d.ksplit, d.batch);
-  if (split) {
-    if (s) hipLaunchKernelGGL((gemm_bf16_kernel<256, 128, AK, BK_, true, true, true, Epi, 64, 256>), grid, dim3(256), 0, st, d, A, B, s, s_bs, epi);
-    else hipLaunchKernelGGL((gemm_bf16_kernel<256, 128, AK, BK_, true, false, true, Epi, 64, 256>), grid, dim3(256), 0, st, d, A, B, s, s_bs, epi);
-  } else {
-    if (s) hipLaunchKernelGGL((gemm_bf16_kernel<256, 128, AK, BK_, false, true, true, Epi, BKT, 256>), grid, dim3(256), 0, st, d, A, B, s, s_bs, epi);
-    else hipLaunchKernelGGL((gemm_bf16_kernel<256, 128, AK, BK_, false, false, true, Epi, BKT, 256>), grid, dim3(256), 0, st, d, A, B, s, s_bs, epi);
-  }
-  return hipGetLastError();
-}
-
-// 128 x 128 block tile, 256 threads, two LDS stages (one barrier per K step), K step BKT
-// (64 for split operands), vector loads.
-template <int BKT, bool AK, bool BK_, class Epi>
-inline hipError_t launch_gemm_bf16_db(hipStream_t st, const GemmDims& d, Opnd<unsigned short> A,
-                                      Opnd<unsigned short> B, const float* s, long s_bs, bool split, Epi epi) {
-  static_assert(AK && BK_, "K-contiguous operands only");
-  dim3 grid(gemm_tiles(d), d.ksplit, d.batch);
-  if (split) {
-    if (s) hipLaunchKernelGGL((gemm_bf16_kernel<128, 128, AK, BK_, true, true, true, Epi, 64, 256, true>), grid, dim3(256), 0, st, d, A, B, s, s_bs, epi);
-    else hipLaunchKernelGGL((gemm_bf16_kernel<128, 128, AK, BK_, true, false, true, Epi, 64, 256, true>), grid, dim3(256), 0, st, d, A, B, s, s_bs, epi);
-  } else {
-    if (s) hipLaunchKernelGGL((gemm_bf16_kernel<128, 128, AK, BK_, false, true, true, Epi, BKT, 256, true>), grid, dim3(256), 0, st, d, A, B, s, s_bs, epi);
-    else hipLaunchKernelGGL((gemm_bf16_kernel<128, 128, AK, BK_, false, false, true, Epi, BKT, 256, true>), grid, dim3(256), 0, st, d, A, B, s, s_bs, epi);
-  }
-  return hipGetLastError();
-}
-
 // 128 x 128 block tile, 256 threads, one LDS stage, K step BKT for both forms, compiled for at
 // least MINW waves per SIMD (registers capped accordingly).
 template <int MINW, int BKT, bool AK, bool BK_, class Epi, int PAD = 8>

@@ -30,9 +30,8 @@
 #include <vector>
 
 #include "gemm_kernels.h"
-#include "gemm_pipe.h"
-#include "gemm_lds.h"
 #include "gemm_f64_lds.h"
+#include "gemm_bf16_lds.h"
 #include "host_eigen.h"
 #include "kernels_misc.h"
 #include "qp_solver.h"
@@ -136,6 +135,11 @@ struct EpiStage1 {
   // idx = outer * pc * colsp + p * colsp + j with outer = kv * rows + r (or r * kvec + kv):
   // the row (p, r) and column (kv, j) terms separate.
   static constexpr bool kSeparable = true;
+  // BF16 planes, four columns at a time where no group of four crosses a vector's end
+  static constexpr bool kPlanes = true;
+  __device__ bool planes_ok() const { return (cols & 3) == 0; }
+  __device__ int planes() const { return Sl ? 2 : 1; }
+  __device__ float factor(int m) const { return scale ? (float)scale[p0 + m / rows] : 1.0f; }
   struct Row {
     long off;
     double f;
@@ -235,127 +239,50 @@ void gemm64(hipStream_t st, int M, int N, int K, int batch, int ksplit, Opnd<dou
   XG_HIP((launch_gemm_f64<64, 64, AK, BK_>(st, d, A, B, epi)));
 }
 
-// BF16 kernel choice (XTPGPU_BF16_KERNEL, for A/B timing; anything else is the default, 1):
-// 1 = K-contiguous operands: split forms 128x128 with BK 64 (two workgroups per CU), plain BF16
-// 128x128 with BK 64 capped for three waves per SIMD; staged32 = BK 32; wide = split BK 64 /
-// plain BK 128 at two workgroups per CU; pipe = direct-to-LDS pipeline; big = 256x256; tall =
-// 256x128 with 512 threads; wave128 / wave128k128 = 256x128 with 256 threads; db64 / db128 = two
-// LDS stages; k64occ{2,3,4} / k32occ{3,4} = register caps for 2-4 waves per SIMD.
+// BF16 kernel choice (XTPGPU_BF16_KERNEL, for A/B timing; anything else is the default, 2):
+// staged32 / staged64 = the register-staged 128 x 128 tiles with 32- or 64-wide K steps throughout.
 inline int bf16_kernel_choice() {
   const char* e = std::getenv("XTPGPU_BF16_KERNEL");
   if (e && std::strcmp(e, "staged32") == 0) return 0;
-  if (e && std::strcmp(e, "pipe") == 0) return 2;
-  if (e && std::strcmp(e, "big") == 0) return 3;
-  if (e && std::strcmp(e, "tall") == 0) return 4;
-  if (e && std::strcmp(e, "wave128") == 0) return 5;
-  if (e && std::strcmp(e, "wave128k128") == 0) return 6;
-  if (e && std::strcmp(e, "db64") == 0) return 7;
-  if (e && std::strcmp(e, "db128") == 0) return 8;
-  if (e && std::strcmp(e, "k64occ2") == 0) return 9;
-  if (e && std::strcmp(e, "k64occ3") == 0) return 10;
-  if (e && std::strcmp(e, "k64occ4") == 0) return 11;
-  if (e && std::strcmp(e, "k32occ3") == 0) return 12;
-  if (e && std::strcmp(e, "k32occ4") == 0) return 13;
-  if (e && std::strcmp(e, "wide") == 0) return 14;
-  if (e && std::strcmp(e, "lds256") == 0) return 15;
-  if (e && std::strcmp(e, "lds128") == 0) return 16;
-  return 1;
+  if (e && std::strcmp(e, "staged64") == 0) return 1;
+  return 2;
+}
+
+// 256 x 256 tiles for an M x N product: enough of them for the chip's 256 CUs, and no more than a fifth
+// of padding over what 128 x 128 tiles compute (which the larger tile's rate pays for).
+inline bool bf16_big_tiles(long M, long N, long batch_ks) {
+  const long t2 = (M + 255) / 256 * ((N + 255) / 256), t1 = (M + 127) / 128 * ((N + 127) / 128);
+  return t2 * batch_ks >= 256 && 4 * t2 * 5 <= t1 * 6;
 }
 
 template <bool AK, bool BK_, class Epi>
 void gemm16(hipStream_t st, int M, int N, int K, int batch, int ksplit, Opnd<unsigned short> A,
-            Opnd<unsigned short> B, const float* s, long s_bs, bool split, bool lower, Epi epi) {
+            Opnd<unsigned short> B, bool split, bool lower, Epi epi) {
   if (M <= 0 || N <= 0 || batch <= 0) return;
   const int choice = bf16_kernel_choice();
   if constexpr (AK && BK_) {
-    // direct-to-LDS pipeline with 128-row wave tiles (256 x 256 block, 2 stages; 256 x 128, 3 stages)
-    if ((choice == 15 || choice == 16) && !s && lds_ok(A, B, K, split) && !(lower && choice == 16)) {
-      if (choice == 15) {
-        GemmDims d = make_dims<256, 256>(M, N, std::max(K, 0), batch, ksplit, split ? 32 : 64, lower);
-        d.group = lower ? lower_tile_group(d) : tile_group(d);
-        const char* sc = std::getenv("XTPGPU_LDS_SCHED");
-        const int sched = sc ? std::atoi(sc) : 0;
-        if constexpr (std::is_same<Epi, EpiStage1>::value) {
-          if (sched == 1) { XG_HIP((launch_gemm_bf16_lds<256, 256, 2, Epi, 1>(st, d, A, B, split, epi))); return; }
-          if (sched == 2) { XG_HIP((launch_gemm_bf16_lds<256, 256, 2, Epi, 2>(st, d, A, B, split, epi))); return; }
-        }
-        XG_HIP((launch_gemm_bf16_lds<256, 256, 2>(st, d, A, B, split, epi)));
-      } else {
-        GemmDims d = make_dims<256, 128>(M, N, std::max(K, 0), batch, ksplit, split ? 32 : 64, false);
-        d.group = tile_group(d);
-        XG_HIP((launch_gemm_bf16_lds<256, 128, 3>(st, d, A, B, split, epi)));
+    if (choice == 2 && !lower && lds_ok(A, B, K, split)) {
+      if (bf16_big_tiles(M, N, (long)batch * std::max(ksplit, 1))) {
+        GemmDims d = make_dims<256, 256>(M, N, std::max(K, 0), batch, ksplit, split ? 32 : 64, false);
+        d.group = d.tiles_m >= 32 && d.tiles_n >= 4 ? 4 : 0;
+        XG_HIP((launch_bf16_ring<4, 4, 4, 4, 2>(st, d, A, B, split, epi)));
+        return;
       }
-      return;
     }
-    if (choice == 3 && bf16_vec(A, B, K, s_bs) && (long)M * N >= 256L * 256 * 512) {
-      GemmDims d = make_dims<256, 256>(M, N, std::max(K, 0), batch, ksplit, 32, lower);
-      XG_HIP((launch_gemm_bf16_big<AK, BK_>(st, d, A, B, s, s_bs, split, epi)));
-      return;
-    }
-    // the lower-triangle tile walk assumes square tiles: 256 x 128 only for full outputs
-    if (choice == 4 && !lower && bf16_vec(A, B, K, s_bs) && (long)M * N >= 256L * 128 * 512) {
-      GemmDims d = make_dims<256, 128>(M, N, std::max(K, 0), batch, ksplit, 64, false);
-      d.group = tile_group(d);
-      XG_HIP((launch_gemm_bf16_tall<AK, BK_>(st, d, A, B, s, s_bs, split, epi)));
-      return;
-    }
-    if ((choice == 5 || choice == 6) && !lower && bf16_vec(A, B, K, s_bs) && (long)M * N >= 256L * 128 * 512) {
-      const int bk = split ? 64 : (choice == 6 ? 128 : 64);
-      GemmDims d = make_dims<256, 128>(M, N, std::max(K, 0), batch, ksplit, bk, false);
-      d.group = tile_group(d);
-      if (bk == 128)
-        XG_HIP((launch_gemm_bf16_wave128<128, AK, BK_>(st, d, A, B, s, s_bs, split, epi)));
-      else
-        XG_HIP((launch_gemm_bf16_wave128<64, AK, BK_>(st, d, A, B, s, s_bs, split, epi)));
-      return;
-    }
-    if ((choice == 7 || choice == 8) && bf16_vec(A, B, K, s_bs)) {
-      const int bk = split ? 64 : (choice == 8 ? 128 : 64);
-      GemmDims d = make_dims<128, 128>(M, N, std::max(K, 0), batch, ksplit, bk, lower);
-      d.group = lower ? lower_tile_group(d) : tile_group(d);
-      if (bk == 128)
-        XG_HIP((launch_gemm_bf16_db<128, AK, BK_>(st, d, A, B, s, s_bs, split, epi)));
-      else
-        XG_HIP((launch_gemm_bf16_db<64, AK, BK_>(st, d, A, B, s, s_bs, split, epi)));
-      return;
-    }
-    // default for plain BF16: 64-wide K steps with the registers capped for three waves per SIMD
-    // (148 VGPRs, 37 KB LDS: three workgroups per CU) -- latency hiding by occupancy
-    if (choice == 1 && !split && bf16_vec(A, B, K, s_bs)) {
+    if (choice >= 1 && bf16_vec(A, B, K, 0)) {
       GemmDims d = make_dims<128, 128>(M, N, std::max(K, 0), batch, ksplit, 64, lower);
       d.group = lower ? lower_tile_group(d) : tile_group(d);
-      XG_HIP((launch_gemm_bf16_occ<3, 64, AK, BK_>(st, d, A, B, s, s_bs, split, epi)));
-      return;
-    }
-    if (choice >= 9 && choice <= 13 && bf16_vec(A, B, K, s_bs)) {
-      GemmDims d = make_dims<128, 128>(M, N, std::max(K, 0), batch, ksplit, choice >= 12 ? 32 : 64, lower);
-      d.group = lower ? lower_tile_group(d) : tile_group(d);
-      if (choice == 9) XG_HIP((launch_gemm_bf16_occ<2, 64, AK, BK_>(st, d, A, B, s, s_bs, split, epi)));
-      else if (choice == 10) XG_HIP((launch_gemm_bf16_occ<3, 64, AK, BK_>(st, d, A, B, s, s_bs, split, epi)));
-      else if (choice == 11) XG_HIP((launch_gemm_bf16_occ<4, 64, AK, BK_>(st, d, A, B, s, s_bs, split, epi)));
-      else if (choice == 12) XG_HIP((launch_gemm_bf16_occ<3, 32, AK, BK_>(st, d, A, B, s, s_bs, split, epi)));
-      else XG_HIP((launch_gemm_bf16_occ<4, 32, AK, BK_>(st, d, A, B, s, s_bs, split, epi)));
-      return;
-    }
-    if ((choice == 1 || choice >= 3) && bf16_vec(A, B, K, s_bs)) {
-      GemmDims d = make_dims<128, 128>(M, N, std::max(K, 0), batch, ksplit, bf16_wide_kstep(split), lower);
-      d.group = lower ? lower_tile_group(d) : tile_group(d);
-      XG_HIP((launch_gemm_bf16<128, 128, AK, BK_>(st, d, A, B, s, s_bs, split, epi, true)));
-      return;
-    }
-    if (choice == 2 && split && !s && !lower && pipe_ok(A, B, K)) {
-      if ((long)M * N >= 256L * 128 * 512) {
-        GemmDims d = make_dims<256, 128>(M, N, std::max(K, 0), batch, ksplit, 32, false);
-        XG_HIP((launch_gemm_bf16x3_pipe<256, 128, 3>(st, d, A, B, epi)));
-      } else {
-        GemmDims d = make_dims<128, 128>(M, N, std::max(K, 0), batch, ksplit, 32, false);
-        XG_HIP((launch_gemm_bf16x3_pipe<128, 128, 4>(st, d, A, B, epi)));
-      }
+      // plain BF16: registers capped for three waves per SIMD (148 VGPRs, 37 KB LDS: three workgroups
+      // per CU) -- latency hiding by occupancy; split: two workgroups per CU
+      if (split)
+        XG_HIP((launch_gemm_bf16<128, 128, AK, BK_>(st, d, A, B, nullptr, 0, split, epi, true)));
+      else
+        XG_HIP((launch_gemm_bf16_occ<3, 64, AK, BK_>(st, d, A, B, nullptr, 0, split, epi)));
       return;
     }
   }
   GemmDims d = make_dims<128, 128>(M, N, std::max(K, 0), batch, ksplit, 32, lower);
-  XG_HIP((launch_gemm_bf16<128, 128, AK, BK_>(st, d, A, B, s, s_bs, split, epi)));
+  XG_HIP((launch_gemm_bf16<128, 128, AK, BK_>(st, d, A, B, nullptr, 0, split, epi)));
 }
 
 // Number of K splits so that tiles*splits gives about four workgroups per CU, with K chunks
@@ -981,23 +908,18 @@ void rpa_epsilon_impl(xtpgpu_ctx ctx, xtpgpu_mmn mmn, const double* energies, in
       const Opnd<unsigned short> Bo{Bh, Bl, Kp, (long)plane};
       const long tl = (P + 127) / 128;
       // the default kernels keep 2 (split) or 3 (plain) 128 x 128 workgroups per CU resident
-      const int ks = (P >= 256 && bf16_kernel_choice() == 1 && bf16_vec(A, Bo, (int)Kp, 0))
+      const int ks = (P >= 256 && bf16_kernel_choice() >= 1 && bf16_vec(A, Bo, (int)Kp, 0))
                          ? eps_ksplit(tl * (tl + 1) / 2 * nw_g, (split ? 2L : 3L) * cus, Kp, 64) : 1;
-      // split form from P = 1536: 256 x 256 tiles whose operands go straight to LDS (one
-      // workgroup per CU), K split to fill its rounds -- half the panel traffic per FLOP of
-      // 128 x 128 tiles, which is what bounds this GEMM (220 against 206 TFLOP/s at P = 2000, 280
-      // against 229 at P = 6000); below, the 128 x 128 tiles fill the chip better (a loop of the
-      // 256 uneven segments' builds, P 248-2100, took 532 ms with the large tiles from P = 512
-      // against 480 ms). XTPGPU_EPS_BF16_KERNEL=wide keeps the 128 x 128 tiles throughout.
-      const char* ek = std::getenv("XTPGPU_EPS_BF16_KERNEL");
-      const bool wide = ek && std::strcmp(ek, "wide") == 0;
-      if (!wide && bf16_kernel_choice() == 1 && split && P >= 1536 && lds_ok(A, Bo, (int)Kp, true)) {
+      // split form from P = 1536: 256 x 256 tiles (one workgroup per CU), K split to fill their rounds;
+      // below, the 128 x 128 tiles fill the chip better (a loop of the 256 uneven segments' builds,
+      // P 248-2100, took 532 ms with large tiles from P = 512 against 480 ms)
+      if (bf16_kernel_choice() == 2 && split && P >= 1536 && lds_ok(A, Bo, (int)Kp, true)) {
         const long t2 = (P + 255) / 256;
         const int k2 = eps_ksplit(t2 * (t2 + 1) / 2 * nw_g, (long)cus, Kp, 32);
         GemmDims d = make_dims<256, 256>((int)P, (int)P, (int)Kp, (int)nw_g, k2, 32, true);
         DevBuf& pb = ctx->ws[2];
         pb.ensure((size_t)d.ksplit * nw_g * P * P * 4);
-        XG_HIP((launch_gemm_bf16_lds<256, 256, 2>(st, d, A, Bo, true, EpiPart32{pb.as<float>(), P, P, nw_g})));
+        XG_HIP((launch_bf16_ring<4, 4, 4, 4, 2>(st, d, A, Bo, true, EpiPart32{pb.as<float>(), P, P, nw_g})));
         eps_reduce_splits(st, pb.as<float>(), d.ksplit, nw_g, P, out_dev + w0 * P * P);
       } else if (ks > 1) {  // the default tiles over K splits, FP32 partials, one reduction
         GemmDims d = make_dims<128, 128>((int)P, (int)P, (int)Kp, (int)nw_g, ks, 64, true);
@@ -1011,7 +933,7 @@ void rpa_epsilon_impl(xtpgpu_ctx ctx, xtpgpu_mmn mmn, const double* energies, in
           XG_HIP((launch_gemm_bf16_occ<3, 64, true, true>(st, d, A, Bo, nullptr, 0, false, ep)));
         eps_reduce_splits(st, pb.as<float>(), d.ksplit, nw_g, P, out_dev + w0 * P * P);
       } else {
-        gemm16<true, true>(st, (int)P, (int)P, (int)Kp, (int)nw_g, 1, A, Bo, nullptr, 0, split, true, eg);
+        gemm16<true, true>(st, (int)P, (int)P, (int)Kp, (int)nw_g, 1, A, Bo, split, true, eg);
       }
     }
   }
@@ -1175,6 +1097,7 @@ MatmulPlan plan_matmul(const xtpgpu_bseop_s* op, int precision, long k) {
   if ((op->cd || op->cd2) && !m16)
     pl.part_more = std::max(pl.part_more,
                             (size_t)f64_ksplit(f64_narrow_tiles(ct, vt) * k, P * op->vtp) * ct * vt * k * 8);
+  if (op->cd2 && m16) pl.part_more = std::max(pl.part_more, (size_t)k * ct * vt * 4);  // one split
   pl.part_more = std::max(pl.part_more, pl.part);
   return pl;
 }
@@ -1333,6 +1256,25 @@ void bse_matmul_impl(xtpgpu_bseop op, int precision, const double* X, long ldx, 
     }
   };
 
+  // the same in BF16 with ks K splits (FP32 partials, added in order)
+  auto stage2_bf16 = [&](Opnd<unsigned short> A, Opnd<unsigned short> B, long np, int ks, double alpha) {
+    const long K2 = np * vtp;
+    const int bk = bf16_wide_kstep(split);
+    const GemmDims dd = make_dims<128, 128>((int)ct, (int)vt, (int)K2, (int)k, ks, bk, false);
+    float* pt = static_cast<float*>(part_p);
+    const EpiPart32 ep{pt, ct, vt, k};
+    const bool fits = (size_t)dd.ksplit * k * ct * vt * 4 <= part_bytes;
+    if (fits && vt <= 128 && bf16_kernel_choice() == 2 && lds_ok(A, B, (int)K2, split)) {
+      XG_HIP(launch_bf16_tall(st, (int)ct, (int)vt, (int)K2, (int)k, ks, bk, A, B, split, ep));
+    } else if (fits && ks > 1 && bf16_vec(A, B, (int)K2, 0)) {
+      XG_HIP((launch_gemm_bf16<128, 128, true, true>(st, dd, A, B, nullptr, 0, split, ep, true)));
+    } else {
+      gemm16<true, true>(st, (int)ct, (int)vt, (int)K2, (int)k, 1, A, B, split, false, EpiStore{Y, 1, ct, ldy, alpha, 1.0});
+      return;
+    }
+    add_partials(st, pt, dd.ksplit, ct * vt, k, Y, ldy, alpha);
+  };
+
   // ---------------- Hd (bse_operator.cc:70-89, PrepareMatrix1/2): -cd sum_P eps_P M^P_cc' X M^P_vv'^T
   if (op->cd) {
     const double alpha = -(double)op->cd;
@@ -1383,7 +1325,7 @@ void bse_matmul_impl(xtpgpu_bseop op, int precision, const double* X, long ldx, 
                              Opnd<unsigned short>{op->Mcc_h.as<unsigned short>() + p0 * ct * ctp,
                                                   split ? op->Mcc_l.as<unsigned short>() + p0 * ct * ctp : nullptr,
                                                   ctp, 0},
-                             Opnd<unsigned short>{Xh, Xl, ctp, 0}, nullptr, 0, split, false, e1);
+                             Opnd<unsigned short>{Xh, Xl, ctp, 0}, split, false, e1);
         }
         ProfScope prof(pctx, split ? "hd_stage2" : "hd_stage2_bf16", f2, b2);
         const Opnd<unsigned short> s2a{Sh, Sl, k * np * vtp, np * vtp};
@@ -1394,18 +1336,7 @@ void bse_matmul_impl(xtpgpu_bseop op, int precision, const double* X, long ldx, 
         const long tiles2 = ((ct + 127) / 128) * ((vt + 127) / 128) * k;
         const int ks2 = (int)std::max<long>(1, std::min<long>(4, std::min<long>(512 / std::max<long>(1, tiles2),
                                                                                (np * vtp) / 2048)));
-        if (ks2 > 1 && bf16_vec(s2a, s2b, (int)(np * vtp), 0)) {
-          // launched directly so the partial count is exactly dd.ksplit (<= 4, within pl.part)
-          const GemmDims dd = make_dims<128, 128>((int)ct, (int)vt, (int)(np * vtp), (int)k, ks2,
-                                                  bf16_wide_kstep(split), false);
-          float* pt = static_cast<float*>(part_p);
-          XG_HIP((launch_gemm_bf16<128, 128, true, true>(st, dd, s2a, s2b, nullptr, 0, split, EpiPart32{pt, ct, vt, k},
-                                                         true)));
-          add_partials(st, pt, dd.ksplit, ct * vt, k, Y, ldy, alpha);
-        } else {
-          gemm16<true, true>(st, (int)ct, (int)vt, (int)(np * vtp), (int)k, 1, s2a, s2b, nullptr, 0, split, false,
-                             EpiStore{Y, 1, ct, ldy, alpha, 1.0});
-        }
+        stage2_bf16(s2a, s2b, np, ks2, alpha);
       }
     }
   }
@@ -1435,12 +1366,10 @@ void bse_matmul_impl(xtpgpu_bseop op, int precision, const double* X, long ldx, 
         gemm16<true, true>(st, (int)M1, (int)N1, (int)round8(ct), 1, 1,
                            Opnd<unsigned short>{op->Mvc_h.as<unsigned short>() + p0 * Np,
                                                 split ? op->Mvc_l.as<unsigned short>() + p0 * Np : nullptr, ctp, 0},
-                           Opnd<unsigned short>{Xh, Xl, ctp, 0}, nullptr, 0, split, false, e1);
-        gemm16<true, true>(st, (int)ct, (int)vt, (int)(np * vtp), (int)k, 1,
-                           Opnd<unsigned short>{op->McvT_h.as<unsigned short>() + p0 * vtp,
-                                                split ? op->McvT_l.as<unsigned short>() + p0 * vtp : nullptr, P * vtp, 0},
-                           Opnd<unsigned short>{Sh, Sl, np * vtp, vt * np * vtp}, nullptr, 0, split, false,
-                           EpiStore{Y, 1, ct, ldy, alpha, 1.0});
+                           Opnd<unsigned short>{Xh, Xl, ctp, 0}, split, false, e1);
+        stage2_bf16(Opnd<unsigned short>{op->McvT_h.as<unsigned short>() + p0 * vtp,
+                                         split ? op->McvT_l.as<unsigned short>() + p0 * vtp : nullptr, P * vtp, 0},
+                    Opnd<unsigned short>{Sh, Sl, np * vtp, vt * np * vtp}, np, 1, alpha);
       }
     }
   }
