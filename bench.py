@@ -39,9 +39,9 @@ PEAK = {"fp64": 78.6e12, "bf16": 2.5e15, "hbm": 8.0e12}
 # WRITE_SIZE 1.0 GiB -> x1.0); FETCH_SIZE 4.462e6 / 3.159e6 KiB, WRITE_SIZE 3.450e6 / 3.490e6 KiB
 # per dispatch. The P-chunk keeps the stage-1 intermediate under 3 GiB: 286 levels for the split
 # form (two output planes), 573 for plain BF16.
-HD_STAGE1_TRAFFIC = {"bf16x3": {"read": 2.745e6 * 2.0 * 1024, "write": 4.090e6 * 1.0 * 1024,
+HD_STAGE1_TRAFFIC = {"bf16x3": {"read": 2.745e6 * 2.0 * 1024, "write": 3.440e6 * 1.0 * 1024,
                                 "launch": "30-column H X stage-1 launch, split BF16 (P-chunk 286)"},
-                     "bf16": {"read": 2.371e6 * 2.0 * 1024, "write": 4.060e6 * 1.0 * 1024,
+                     "bf16": {"read": 2.371e6 * 2.0 * 1024, "write": 3.448e6 * 1.0 * 1024,
                               "launch": "30-column H X stage-1 launch, plain BF16 (P-chunk 573)"}}
 
 
