@@ -34,6 +34,7 @@
 #include "gemm_bf16_lds.h"
 #include "host_eigen.h"
 #include "kernels_misc.h"
+#include "pack_kernels.h"
 #include "qp_solver.h"
 #include "xtpgpu_internal.h"
 
@@ -1514,41 +1515,28 @@ void pack_transitions(xtpgpu_bseop op, xtpgpu_mmn mmn) {
   const int cx = op->cx, cd2 = op->cd2;
   const bool need16 = ((op->mask >> XTPGPU_BF16) & 1u) || ((op->mask >> XTPGPU_BF16X3) & 1u);
   const double* D = mmn->d();
-  auto el = [=] __device__(long p, long slice, long row) { return D[p * ps + slice * nt + row]; };
+  const double* vc = D + vmin_r * nt + cmin_r;  // (p, v, c) at p ps + v nt + c
+  const double* cv = D + cmin_r * nt + vmin_r;
   if (cx || cd2) {
     op->Mvc.ensure((size_t)P * Np * 8);
-    double* A = op->Mvc.as<double>();
-    launch_map(st, (size_t)P * Np, [=] __device__(size_t i) {
-      long p = (long)(i / (size_t)Np), r = (long)(i % (size_t)Np);
-      long v = r / ctp, c = r % ctp;
-      A[i] = c < ct ? el(p, vmin_r + v, cmin_r + c) : 0.0;
-    });
     if (need16 && cd2) {
       op->Mvc_h.ensure((size_t)P * Np * 2); op->Mvc_l.ensure((size_t)P * Np * 2);
-      split_to_bf16(st, A, op->Mvc_h.as<unsigned short>(), op->Mvc_l.as<unsigned short>(), (size_t)P * Np);
     }
+    const bool planes = need16 && cd2;
+    pack_rows(st, vc, ps, nt, P, vt, (int)ct, (int)ctp, nullptr, op->Mvc.as<double>(),
+              planes ? op->Mvc_h.as<unsigned short>() : nullptr, planes ? op->Mvc_l.as<unsigned short>() : nullptr);
   }
   if (cx) {
     op->MvcT.ensure((size_t)N * Pp * 8);
-    double* A = op->MvcT.as<double>();
-    launch_map(st, (size_t)N * Pp, [=] __device__(size_t i) {
-      long r = (long)(i / (size_t)Pp), p = (long)(i % (size_t)Pp);
-      long v = r / ct, c = r % ct;
-      A[i] = p < P ? el(p, vmin_r + v, cmin_r + c) : 0.0;
-    });
+    pack_turned(st, vc, ps, nt, vt, ct, P, Pp, op->MvcT.as<double>());
   }
   if (cd2) {
     op->McvT.ensure((size_t)ct * P * vtp * 8);
-    double* A = op->McvT.as<double>();
-    launch_map(st, (size_t)ct * P * vtp, [=] __device__(size_t i) {
-      long c1 = (long)(i / (size_t)(P * vtp)), r = (long)(i % (size_t)(P * vtp));
-      long p = r / vtp, v2 = r % vtp;
-      A[i] = v2 < vt ? el(p, cmin_r + c1, vmin_r + v2) : 0.0;
-    });
     if (need16) {
       op->McvT_h.ensure((size_t)ct * P * vtp * 2); op->McvT_l.ensure((size_t)ct * P * vtp * 2);
-      split_to_bf16(st, A, op->McvT_h.as<unsigned short>(), op->McvT_l.as<unsigned short>(), (size_t)ct * P * vtp);
     }
+    pack_rows(st, cv, nt, ps, ct, P, (int)vt, (int)vtp, nullptr, op->McvT.as<double>(),
+              need16 ? op->McvT_h.as<unsigned short>() : nullptr, need16 ? op->McvT_l.as<unsigned short>() : nullptr);
   }
 }
 
@@ -1558,33 +1546,24 @@ void build_diag(xtpgpu_bseop op, xtpgpu_mmn mmn) {
   hipStream_t st = op->ctx->stream;
   const long ct = op->ct, P = op->P, N = op->N, nt = mmn->ntotal, ps = (long)mmn->pstride();
   const long vmin_r = op->vmin_r, cmin_r = op->cmin_r;
-  const double* D = mmn->d();
-  const double* E = op->eps.as<double>();
-  auto el = [=] __device__(long p, long slice, long row) { return D[p * ps + slice * nt + row]; };
   op->diag.ensure((size_t)N * 8);
   op->diag0.ensure((size_t)N * 8);
   double* d0 = op->diag0.as<double>();
-  const double fx = op->cx, fd = op->cd, fd2 = op->cd2;
-  launch_map(st, (size_t)N, [=] __device__(size_t i) {
-    long v = (long)i / ct, c = (long)i % ct;
-    double e = 0.0;
-    if (fx != 0.0) {
-      double s = 0.0;
-      for (long p = 0; p < P; ++p) { double m = el(p, vmin_r + v, cmin_r + c); s += m * m; }
-      e += fx * s;
-    }
-    if (fd != 0.0) {
-      double s = 0.0;
-      for (long p = 0; p < P; ++p) s += el(p, cmin_r + c, cmin_r + c) * E[p] * el(p, vmin_r + v, vmin_r + v);
-      e -= fd * s;
-    }
-    if (fd2 != 0.0) {
-      double s = 0.0;
-      for (long p = 0; p < P; ++p) s += el(p, cmin_r + c, vmin_r + v) * E[p] * el(p, vmin_r + v, cmin_r + c);
-      e -= fd2 * s;
-    }
-    d0[i] = e;
-  });
+  const long shares = diag_shares(op->vt, ct, P);
+  double* part = d0;
+  if (shares > 1) {
+    DevBuf& ws = op->ctx->ws[4];
+    ws.ensure((size_t)shares * N * 8);
+    part = ws.as<double>();
+  }
+  diag_sums(st, mmn->d(), ps, nt, vmin_r, cmin_r, op->vt, ct, P, op->eps.as<double>(), op->cx, op->cd, op->cd2, shares,
+            part);
+  if (shares > 1)
+    launch_map(st, (size_t)N, [=] __device__(size_t i) {
+      double t = 0.0;
+      for (long z = 0; z < shares; ++z) t += part[z * N + i];
+      d0[i] = t;
+    });
   finish_diag(op);
 }
 
@@ -1618,34 +1597,20 @@ extern "C" int xtpgpu_bse_create(xtpgpu_ctx ctx, xtpgpu_mmn mmn, const double* e
     const long ctp = op->ctp, vtp = op->vtp, Pp = op->Pp, Np = vt * ctp;
     XG_HIP(hipSetDevice(ctx->device));
     hipStream_t st = ctx->stream;
-    const double* D = mmn->d();
-
     setup_hqp_eps(op.get(), Hqp, ldhqp, eps0inv);
-    const double* E = op->eps.as<double>();
     const bool need16 = ((op->mask >> XTPGPU_BF16) & 1u) || ((op->mask >> XTPGPU_BF16X3) & 1u);
-
-    auto el = [=] __device__(long p, long slice, long row) { return D[p * ps + slice * nt + row]; };
     if (cd) {
       op->Mcc.alloc((size_t)P * ct * ctp * 8);
-      double* A = op->Mcc.as<double>();
-      launch_map(st, (size_t)P * ct * ctp, [=] __device__(size_t i) {
-        long p = (long)(i / (size_t)(ct * ctp)), r = (long)(i % (size_t)(ct * ctp));
-        long c1 = r / ctp, c2 = r % ctp;
-        A[i] = c2 < ct ? el(p, cmin_r + c1, cmin_r + c2) : 0.0;
-      });
       op->Bvv.alloc((size_t)vt * P * vtp * 8);
-      double* B = op->Bvv.as<double>();
-      launch_map(st, (size_t)vt * P * vtp, [=] __device__(size_t i) {
-        long v1 = (long)(i / (size_t)(P * vtp)), r = (long)(i % (size_t)(P * vtp));
-        long p = r / vtp, v2 = r % vtp;
-        B[i] = v2 < vt ? E[p] * el(p, vmin_r + v1, vmin_r + v2) : 0.0;
-      });
       if (need16) {
         op->Mcc_h.alloc((size_t)P * ct * ctp * 2); op->Mcc_l.alloc((size_t)P * ct * ctp * 2);
-        split_to_bf16(st, A, op->Mcc_h.as<unsigned short>(), op->Mcc_l.as<unsigned short>(), (size_t)P * ct * ctp);
         op->Bvv_h.alloc((size_t)vt * P * vtp * 2); op->Bvv_l.alloc((size_t)vt * P * vtp * 2);
-        split_to_bf16(st, B, op->Bvv_h.as<unsigned short>(), op->Bvv_l.as<unsigned short>(), (size_t)vt * P * vtp);
       }
+      auto u16 = [&](DevBuf& b) { return need16 ? b.as<unsigned short>() : nullptr; };
+      pack_rows(st, mmn->d() + cmin_r * nt + cmin_r, ps, nt, P, ct, (int)ct, (int)ctp, nullptr, op->Mcc.as<double>(),
+                u16(op->Mcc_h), u16(op->Mcc_l));
+      pack_rows(st, mmn->d() + vmin_r * nt + vmin_r, nt, ps, vt, P, (int)vt, (int)vtp, op->eps.as<double>(),
+                op->Bvv.as<double>(), u16(op->Bvv_h), u16(op->Bvv_l));
     }
     op->vmin_r = vmin_r;
     op->cmin_r = cmin_r;
