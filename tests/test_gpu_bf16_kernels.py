@@ -29,7 +29,8 @@ def operator(c, o, v, P, seed):
 @pytest.mark.parametrize("o,v,P,k", [(1, 33, 9, 3), (16, 31, 40, 1), (17, 32, 33, 16), (32, 65, 20, 2), (33, 256, 24, 9),
                                      (64, 257, 24, 9), (65, 129, 40, 3), (112, 96, 12, 5), (113, 64, 16, 5),
                                      (128, 520, 70, 9), (129, 260, 33, 4), (30, 300, 600, 19), (31, 301, 600, 19),
-                                     (100, 255, 257, 12), (8, 1030, 130, 31)])
+                                     (100, 255, 257, 12), (8, 1030, 130, 31), (33, 390, 60, 31),
+                                     (64, 388, 60, 12), (30, 400, 100, 17)])
 @pytest.mark.parametrize("c", [(0, 0, 1, 0), (0, 0, 0, 1)])
 @pytest.mark.parametrize("prec", ["bf16", "bf16x3"])
 def test_first_and_second_stage(o, v, P, k, c, prec, monkeypatch):

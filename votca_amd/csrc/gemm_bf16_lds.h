@@ -26,15 +26,21 @@
 
 namespace xg {
 
-// Epilogues whose rows are BF16 planes (kPlanes): the kernel rounds to hi (and lo, planes() == 2) and
-// stores four consecutive columns of a row at once, which planes_ok() allows: 4 columns from a
-// multiple of four are adjacent in memory, 8-byte aligned. Row m carries factor(m).
+// Epilogues whose rows are BF16 planes (kPlanes): the kernel rounds to hi (and lo, planes() == 2). Row m
+// carries factor(m). by_four(): 4 columns from a multiple of four are adjacent in memory, 8-byte aligned.
 template <class E, class = void>
 struct epi_planes { static constexpr bool value = false; };
 template <class E>
 struct epi_planes<E, decltype((void)E::kPlanes)> { static constexpr bool value = E::kPlanes; };
 
 typedef unsigned short us4v __attribute__((ext_vector_type(4)));
+
+// lane `from`'s value, the same in every lane
+__device__ __forceinline__ long lane_value(long x, int from) {
+  const unsigned lo = __builtin_amdgcn_readlane((unsigned)x, from);
+  const unsigned hi = __builtin_amdgcn_readlane((unsigned)((unsigned long)x >> 32), from);
+  return (long)((unsigned long)hi << 32 | lo);
+}
 
 template <int TM, int TN, int WR, int WC, int STAGES, bool SPLIT, class Epi>
 __global__ __launch_bounds__(64 * WR * WC) void gemm_bf16_ring_kernel(
@@ -164,42 +170,46 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_bf16_ring_kernel(
     fill = fill + 1 == STAGES ? 0 : fill + 1;
   }
   // lane: m = 16 i + lane % 16, n = 16 j + 4 (lane / 16) + r
-  if constexpr (epi_planes<Epi>::value && WN == 64 && TM % 2 == 0) {  // 16 lanes of four columns to a row
-    if (epi.planes_ok()) {
-      // A store of the fragments as they lie touches 16 rows in 32-byte pieces (70 cycles an
-      // instruction, a fifth of the whole product at K = 900), so each wave turns 32 rows at a time in
-      // LDS and stores 128-byte pieces of four rows. The pieces straddle cache lines (a vector's rows
-      // are not multiples of 128 bytes), so the stores stay in the L2 until their lines are whole:
-      // non-temporal ones wrote 4.2 GB instead of 3.5 per 3.2 GB and took 4.24 / 1.84 ms instead of
-      // 4.04 / 1.64 (split / plain, 257400 x 3000 x 900).
-      constexpr int RS = 2 * WN + 16;  // LDS row: 36 dwords, conflict-free in both directions
-      constexpr int PLANE = 32 * RS;
-      __syncthreads();  // every wave has read the last stage
-      unsigned char* mine = lds + wave * (2 * PLANE);
-      const bool two = SPLIT && epi.planes() == 2;
-      const int gn = n0 + wn0 + 4 * r16;
-      const long co = gn < d.N ? epi.col(b, gn) : 0;
+  if constexpr (epi_planes<Epi>::value && WN == 64 && TM % 2 == 0) {
+    // A store of the fragments as they lie touches 16 rows in 32-byte pieces (70 cycles an
+    // instruction, a fifth of the whole product at K = 900), so each wave turns 32 rows at a time in
+    // LDS and stores 128-byte pieces of four rows. The pieces straddle cache lines (a vector's rows
+    // are not multiples of 128 bytes), so the stores stay in the L2 until their lines are whole:
+    // non-temporal ones wrote 4.2 GB instead of 3.5 per 3.2 GB and took 4.24 / 1.84 ms instead of
+    // 4.04 / 1.64 (split / plain, 257400 x 3000 x 900).
+    constexpr int RS = 2 * WN + 16;  // LDS row: 36 dwords, conflict-free in both directions
+    constexpr int PLANE = 32 * RS;
+    __syncthreads();  // every wave has read the last stage
+    unsigned char* mine = lds + wave * (2 * PLANE);
+    const bool two = SPLIT && epi.planes() == 2;
+    // 16 lanes of four columns to a row, or 64 of one: 2-byte stores, four times as many, where
+    // vectors end inside a group of four (31 columns, 900 x 250 rows, K = 250, split / plain: 173 / 81 us;
+    // 8-byte stores at odd 2-byte offsets, with the cut groups one by one: 190 / 88)
+    const bool four = epi.by_four();
+    const int gn = n0 + wn0 + (four ? 4 * r16 : lane);
+    const long co = gn < d.N ? epi.col(b, gn) : 0;
 #pragma unroll
-      for (int h = 0; h < TM / 2; ++h) {
+    for (int h = 0; h < TM / 2; ++h) {
 #pragma unroll
-        for (int i2 = 0; i2 < 2; ++i2) {
-          const int i = 2 * h + i2;
-          const float f = epi.factor(min(m0 + wm0 + 16 * i + r16, d.M - 1));
+      for (int i2 = 0; i2 < 2; ++i2) {
+        const int i = 2 * h + i2;
+        const float f = epi.factor(min(m0 + wm0 + 16 * i + r16, d.M - 1));
 #pragma unroll
-          for (int j = 0; j < TN; ++j) {
-            us4v vh, vl;
+        for (int j = 0; j < TN; ++j) {
+          us4v vh, vl;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              const float x = acc[i][j][r] * f;
-              vh[r] = bf16_bits_rn(x);
-              vl[r] = bf16_bits_rn(x - bf16_bits_to_f(vh[r]));
-            }
-            unsigned char* at = mine + (16 * i2 + r16) * RS + (16 * j + 4 * q) * 2;
-            *reinterpret_cast<us4v*>(at) = vh;
-            if (two) *reinterpret_cast<us4v*>(at + PLANE) = vl;
+          for (int r = 0; r < 4; ++r) {
+            const float x = acc[i][j][r] * f;
+            vh[r] = bf16_bits_rn(x);
+            vl[r] = bf16_bits_rn(x - bf16_bits_to_f(vh[r]));
           }
+          unsigned char* at = mine + (16 * i2 + r16) * RS + (16 * j + 4 * q) * 2;
+          *reinterpret_cast<us4v*>(at) = vh;
+          if (two) *reinterpret_cast<us4v*>(at + PLANE) = vl;
         }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      if (four) {
 #pragma unroll
         for (int it = 0; it < 8; ++it) {
           const int row = 4 * it + q, gm = m0 + wm0 + 32 * h + row;
@@ -212,10 +222,25 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_bf16_ring_kernel(
             if (two) *reinterpret_cast<us4v*>(epi.Sl + idx) = vl;
           }
         }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      } else {
+        const int mh = m0 + wm0 + 32 * h;
+        const long ro = epi.row(b, ks, min(mh + (lane & 31), d.M - 1)).off;
+#pragma unroll 8
+        for (int row = 0; row < 32; ++row) {
+          if (mh + row >= d.M) break;
+          const unsigned char* at = mine + row * RS + lane * 2;
+          const unsigned short vh = *reinterpret_cast<const unsigned short*>(at);
+          const unsigned short vl = *reinterpret_cast<const unsigned short*>(at + PLANE);
+          const long idx = lane_value(ro, row) + co;
+          if (gn < d.N) {
+            epi.Sh[idx] = vh;
+            if (two) epi.Sl[idx] = vl;
+          }
+        }
       }
-      return;
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
+    return;
   }
   if (!active) return;
   const int mb = m0 + wm0 + r16, nb = n0 + wn0 + 4 * q;

@@ -136,9 +136,9 @@ struct EpiStage1 {
   // idx = outer * pc * colsp + p * colsp + j with outer = kv * rows + r (or r * kvec + kv):
   // the row (p, r) and column (kv, j) terms separate.
   static constexpr bool kSeparable = true;
-  // BF16 planes, four columns at a time where no group of four crosses a vector's end
+  // BF16 planes; no group of four columns crosses a vector's end
   static constexpr bool kPlanes = true;
-  __device__ bool planes_ok() const { return (cols & 3) == 0; }
+  __device__ bool by_four() const { return (cols & 3) == 0; }
   __device__ int planes() const { return Sl ? 2 : 1; }
   __device__ float factor(int m) const { return scale ? (float)scale[p0 + m / rows] : 1.0f; }
   struct Row {
@@ -249,11 +249,15 @@ inline int bf16_kernel_choice() {
   return 2;
 }
 
-// 256 x 256 tiles for an M x N product: enough of them for the chip's 256 CUs, and no more than a fifth
-// of padding over what 128 x 128 tiles compute (which the larger tile's rate pays for).
-inline bool bf16_big_tiles(long M, long N, long batch_ks) {
+// 256 x 256 tiles for an M x N product: enough of them for the chip's 256 CUs, at most a tenth of padding
+// over what 128 x 128 tiles compute, and a K that pays for filling and emptying the larger tile.
+// First stage of H X, 256 / 128 tiles, split and plain, us: (30 vectors of 100, 900 virtual, 700 aux)
+// 1872 / 2157, 744 / 892; (12 of 61, 430, 1200) 1408 / 1528, 725 / 748; (7 of 32, 250, 900)
+// 137 / 160, 70 / 69; (8 of 31, 250, 900) 173 / 177, 81 / 73; (26 of 33, 189, 485: a seventh of
+// padding) 249 / 234, 102 / 87.
+inline bool bf16_big_tiles(long M, long N, long K, long batch_ks, bool split) {
   const long t2 = (M + 255) / 256 * ((N + 255) / 256), t1 = (M + 127) / 128 * ((N + 127) / 128);
-  return t2 * batch_ks >= 256 && 4 * t2 * 5 <= t1 * 6;
+  return t2 * batch_ks >= 256 && 4 * t2 * 10 <= t1 * 11 && K >= (split ? 192 : 384);
 }
 
 template <bool AK, bool BK_, class Epi>
@@ -263,7 +267,7 @@ void gemm16(hipStream_t st, int M, int N, int K, int batch, int ksplit, Opnd<uns
   const int choice = bf16_kernel_choice();
   if constexpr (AK && BK_) {
     if (choice == 2 && !lower && lds_ok(A, B, K, split)) {
-      if (bf16_big_tiles(M, N, (long)batch * std::max(ksplit, 1))) {
+      if (bf16_big_tiles(M, N, K / std::max(ksplit, 1), (long)batch * std::max(ksplit, 1), split)) {
         GemmDims d = make_dims<256, 256>(M, N, std::max(K, 0), batch, ksplit, split ? 32 : 64, false);
         d.group = d.tiles_m >= 32 && d.tiles_n >= 4 ? 4 : 0;
         XG_HIP((launch_bf16_ring<4, 4, 4, 4, 2>(st, d, A, B, split, epi)));
