@@ -311,6 +311,103 @@ void split_to_bf16(hipStream_t st, const double* src, unsigned short* hi, unsign
   });
 }
 
+// Columns of `rows` doubles between a host array (leading dimension ld) and a contiguous device one. A
+// whole array is one copy: a 2D copy to pageable memory goes row by row, some 50 us each.
+void copy_cols(hipStream_t st, double* dev, double* host, long ld, long rows, long cols, hipMemcpyKind kind) {
+  const bool up = kind == hipMemcpyHostToDevice, whole = ld == rows || cols == 1;
+  const size_t n = (size_t)rows * (whole ? cols : 1);
+  for (long c = 0; c < (whole ? std::min<long>(cols, 1) : cols) && n > 0; ++c) {
+    double *d = dev + c * rows, *h = host + c * ld;
+    XG_HIP(hipMemcpyAsync(up ? d : h, up ? h : d, n * 8, kind, st));
+  }
+}
+
+// The host arrays of one call. Up to kPinBytes each way pass through the context's pinned memory, which
+// a small kernel reads or writes as part of the stream's work; a copy of the runtime costs 15-25 us
+// at a few KB and 130 at 64 KB of pageable memory, the kernel 3-5. One call at a time has the context's
+// pinned memory and its ws[5], ws[6]; a second one at the same time (another thread, a chunk source that
+// makes a product) has not, and copies and allocates for itself.
+class HostIo {
+ public:
+  explicit HostIo(xtpgpu_ctx c) : ctx_(c), st_(c->stream), kept_(!c->io_busy.exchange(true)) {
+    if (kept_ && !c->pin) {
+      void* p = nullptr;
+      void* q = nullptr;
+      if (hipHostMalloc(&p, 2 * c->kPinBytes, hipHostMallocMapped | hipHostMallocCoherent) == hipSuccess) {
+        if (hipHostGetDevicePointer(&q, p, 0) == hipSuccess) {
+          c->pin = static_cast<unsigned char*>(p);
+          c->pin_dev = static_cast<unsigned char*>(q);
+        } else {
+          (void)hipHostFree(p);
+        }
+      }
+      (void)hipGetLastError();  // without pinned memory the copies below do
+    }
+  }
+  ~HostIo() {
+    if (busy_) (void)hipStreamSynchronize(st_);
+    if (kept_) ctx_->io_busy.store(false);
+  }
+  // `keep`, or `own` for a call that has not got it or needs more than the context keeps
+  DevBuf& buffer(DevBuf& keep, DevBuf& own, size_t bytes) const {
+    DevBuf& b = kept_ && bytes <= ctx_->kKeepBytes ? keep : own;
+    b.ensure(bytes);
+    return b;
+  }
+  HostIo(const HostIo&) = delete;
+  HostIo& operator=(const HostIo&) = delete;
+
+  void up(double* dev, const double* host, long ld, long rows, long cols) {
+    const size_t n = (size_t)rows * cols;
+    if (n == 0) return;
+    busy_ = true;
+    if (!kept_ || !ctx_->pin || up_ + n * 8 > ctx_->kPinBytes) {
+      copy_cols(st_, dev, const_cast<double*>(host), ld, rows, cols, hipMemcpyHostToDevice);
+      return;
+    }
+    double* p = reinterpret_cast<double*>(ctx_->pin + up_);
+    const double* q = reinterpret_cast<const double*>(ctx_->pin_dev + up_);
+    for (long c = 0; c < cols; ++c) std::memcpy(p + c * rows, host + c * ld, rows * 8);
+    up_ += n * 8;
+    launch_map(st_, n, [=] __device__(size_t i) { dev[i] = q[i]; });
+  }
+  void down(double* host, long ld, const double* dev, long rows, long cols) {
+    const size_t n = (size_t)rows * cols;
+    if (n == 0) return;
+    busy_ = true;
+    if (!kept_ || !ctx_->pin || down_ + n * 8 > ctx_->kPinBytes) {
+      copy_cols(st_, const_cast<double*>(dev), host, ld, rows, cols, hipMemcpyDeviceToHost);
+      return;
+    }
+    double* q = reinterpret_cast<double*>(ctx_->pin_dev + ctx_->kPinBytes + down_);
+    out_.push_back({host, ctx_->pin + ctx_->kPinBytes + down_, ld, rows, cols});
+    down_ += n * 8;
+    launch_map(st_, n, [=] __device__(size_t i) { q[i] = dev[i]; });
+  }
+  // waits for the stream; the downloads are in their arrays afterwards
+  void finish() {
+    XG_HIP(hipStreamSynchronize(st_));
+    busy_ = false;
+    for (const Out& o : out_)
+      for (long c = 0; c < o.cols; ++c)
+        std::memcpy(o.host + c * o.ld, reinterpret_cast<const double*>(o.from) + c * o.rows, o.rows * 8);
+    out_.clear();
+    up_ = down_ = 0;
+  }
+
+ private:
+  struct Out {
+    double* host;
+    const unsigned char* from;
+    long ld, rows, cols;
+  };
+  xtpgpu_ctx ctx_;
+  hipStream_t st_;
+  bool kept_, busy_ = false;
+  size_t up_ = 0, down_ = 0;
+  std::vector<Out> out_;
+};
+
 }  // namespace
 
 // =================================================================== context / memory
@@ -364,6 +461,8 @@ extern "C" int xtpgpu_ctx_create(int device, unsigned flags, xtpgpu_ctx* out) {
     resolve_scratch(device);
     auto c = std::make_unique<xtpgpu_ctx_s>();
     c->device = device;
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && cus > 0) c->cus = cus;
     XG_HIP(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
     *out = c.release();
   });
@@ -378,7 +477,9 @@ extern "C" int xtpgpu_ctx_destroy(xtpgpu_ctx ctx) {
     ctx->collect();
     for (hipEvent_t e : ctx->event_pool) (void)hipEventDestroy(e);
     if (ctx->blas) (void)rocblas_destroy_handle((rocblas_handle)ctx->blas);
+    if (ctx->pin) (void)hipHostFree(ctx->pin);
     delete ctx;
+    DevBuf::drain_current();
   });
 }
 
@@ -396,7 +497,15 @@ extern "C" int xtpgpu_ctx_release_scratch(xtpgpu_ctx ctx) {
     XG_REQUIRE(ctx, XTPGPU_ERR_ARG, "null ctx");
     XG_HIP(hipSetDevice(ctx->device));
     XG_HIP(hipStreamSynchronize(ctx->stream));
-    for (auto& b : ctx->ws) b.release();
+    for (int i = 0; i < 5; ++i) ctx->ws[i].release();
+    if (!ctx->io_busy.exchange(true)) {  // else in use by a call on another thread
+      ctx->ws[5].release();
+      ctx->ws[6].release();
+      if (ctx->pin) (void)hipHostFree(ctx->pin);
+      ctx->pin = ctx->pin_dev = nullptr;
+      ctx->io_busy.store(false);
+    }
+    DevBuf::drain_current();
   });
 }
 
@@ -437,6 +546,10 @@ extern "C" int xtpgpu_malloc(xtpgpu_ctx ctx, int64_t bytes, void** dptr) {
     XG_HIP(hipSetDevice(ctx->device));
     size_t fr = 0, tot = 0;
     XG_HIP(hipMemGetInfo(&fr, &tot));
+    if ((size_t)bytes > fr) {
+      DevBuf::drain_current();
+      XG_HIP(hipMemGetInfo(&fr, &tot));
+    }
     XG_REQUIRE((size_t)bytes <= fr, XTPGPU_ERR_OOM, "xtpgpu_malloc: request exceeds free device memory");
     XG_HIP(hipMalloc(dptr, (size_t)std::max<int64_t>(bytes, 1)));
   });
@@ -700,23 +813,25 @@ extern "C" int xtpgpu_mmn_set_block(xtpgpu_mmn mmn, int64_t vmin, int64_t vtotal
 namespace {
 
 struct RpaPacked {
-  DevBuf A64;          // [P][Kp] FP64
-  DevBuf Ah, Al;       // [P][Kp] bf16 hi / lo
+  double* A64 = nullptr;                           // [P][Kp] FP64
+  unsigned short *Ah = nullptr, *Al = nullptr;     // [P][Kp] bf16 hi / lo
   long K = 0;          // transitions n_occ * n_unocc
   long Kp = 0;         // row length: K rounded up to 64 (8 below 64) for line-aligned rows, zero pads
 };
 
-void rpa_pack(xtpgpu_mmn mmn, long n_occ, long n_unocc, bool need64, bool need16, RpaPacked& pk) {
+long rpa_row_length(long K) { return K >= 64 ? (K + 63) / 64 * 64 : (K + 7) / 8 * 8; }  // 128-byte aligned rows
+
+// the packed transitions at `to` (P Kp doubles, or as many BF16 hi and then lo)
+void rpa_pack(xtpgpu_mmn mmn, long n_occ, long n_unocc, bool need16, void* to, RpaPacked& pk) {
   hipStream_t st = mmn->ctx->stream;
   const long P = mmn->aux, K = n_occ * n_unocc, nt = mmn->ntotal, ps = (long)mmn->pstride();
-  const long Kp = K >= 64 ? (K + 63) / 64 * 64 : (K + 7) / 8 * 8;  // 128-byte aligned rows
+  const long Kp = rpa_row_length(K);
   const long r0 = nt - n_unocc;
   pk.K = K;
   pk.Kp = Kp;
   const double* D = mmn->d();
-  if (need64) {
-    pk.A64.alloc((size_t)P * Kp * sizeof(double));
-    double* A = pk.A64.as<double>();
+  if (!need16) {
+    double* A = pk.A64 = static_cast<double*>(to);
     launch_map(st, (size_t)P * Kp, [=] __device__(size_t i) {
       long p = (long)(i / Kp), k = (long)(i % Kp);
       long v = k / n_unocc, c = k % n_unocc;
@@ -724,10 +839,8 @@ void rpa_pack(xtpgpu_mmn mmn, long n_occ, long n_unocc, bool need64, bool need16
     });
   }
   if (need16) {
-    pk.Ah.alloc((size_t)P * Kp * 2);
-    pk.Al.alloc((size_t)P * Kp * 2);
-    unsigned short* H = pk.Ah.as<unsigned short>();
-    unsigned short* L = pk.Al.as<unsigned short>();
+    unsigned short* H = pk.Ah = static_cast<unsigned short*>(to);
+    unsigned short* L = pk.Al = H + (size_t)P * Kp;
     launch_map(st, (size_t)P * Kp, [=] __device__(size_t i) {
       long p = (long)(i / Kp), k = (long)(i % Kp);
       long v = k / n_unocc, c = k % n_unocc;
@@ -786,10 +899,11 @@ void eps_reduce_splits(hipStream_t st, const T* part, int ks, long nb, long P, d
   });
 }
 
+// to out_dev, or to the host array out_host
 void rpa_epsilon_impl(xtpgpu_ctx ctx, xtpgpu_mmn mmn, const double* energies, int64_t homo, int64_t rpamin,
                       int64_t rpamax, int kind, const double* omega_re, const double* omega_im, int n_omega,
-                      double eta, int precision, double* out_dev) {
-  XG_REQUIRE(ctx && mmn && energies && omega_re && out_dev, XTPGPU_ERR_ARG, "xtpgpu_rpa_epsilon: null argument");
+                      double eta, int precision, double* out_dev, double* out_host = nullptr) {
+  XG_REQUIRE(ctx && mmn && energies && omega_re && (out_dev || out_host), XTPGPU_ERR_ARG, "xtpgpu_rpa_epsilon: null argument");
   XG_REQUIRE(n_omega > 0, XTPGPU_ERR_ARG, "xtpgpu_rpa_epsilon: n_omega must be positive");
   XG_REQUIRE(kind >= 0 && kind <= 2, XTPGPU_ERR_ARG, "xtpgpu_rpa_epsilon: unknown kind");
   XG_REQUIRE(precision == XTPGPU_FP64 || precision == XTPGPU_BF16 || precision == XTPGPU_BF16X3,
@@ -805,25 +919,34 @@ void rpa_epsilon_impl(xtpgpu_ctx ctx, xtpgpu_mmn mmn, const double* energies, in
   const long P = mmn->aux;
   const long rpatotal = rpamax - rpamin + 1;
   const long K = n_occ * n_unocc;
-  RpaPacked pk;
   const bool use16 = precision != XTPGPU_FP64;
-  rpa_pack(mmn, n_occ, n_unocc, !use16, use16, pk);
+  const long Kp = rpa_row_length(K);
+  // one buffer: energies and frequencies, weights, packed transitions, and the matrices if they go to the
+  // host; kept by the context up to kKeepBytes
+  auto up256 = [](size_t n) { return (n + 255) / 256 * 256; };
+  const size_t n_in = (size_t)rpatotal + 2 * n_omega, n_out = out_host ? (size_t)n_omega * P * P : 0;
+  const size_t o_d = up256(n_in * 8), o_a = o_d + up256((size_t)n_omega * Kp * (use16 ? 4 : 8));
+  const size_t o_o = o_a + up256((size_t)P * Kp * (use16 ? 4 : 8)), total = o_o + n_out * 8;
+  HostIo io(ctx);
+  DevBuf own;
+  unsigned char* base = io.buffer(ctx->ws[5], own, total).as<unsigned char>();
+  if (out_host) out_dev = reinterpret_cast<double*>(base + o_o);
+  RpaPacked pk;
+  rpa_pack(mmn, n_occ, n_unocc, use16, base + o_a, pk);
 
   // weights d[w][K] (rpa.cc:110-125, 178-190; the complex kind carries the -2 of rpa.cc:197)
-  DevBuf de(rpatotal * sizeof(double)), dw(2 * n_omega * sizeof(double));
-  XG_HIP(hipMemcpyAsync(de.p, energies, rpatotal * sizeof(double), hipMemcpyHostToDevice, st));
-  std::vector<double> w(2 * n_omega, 0.0);
+  std::vector<double> w(n_in, 0.0);
+  std::copy(energies, energies + rpatotal, w.begin());
   for (int i = 0; i < n_omega; ++i) {
-    w[i] = omega_re[i];
-    w[n_omega + i] = omega_im ? omega_im[i] : 0.0;
+    w[rpatotal + i] = omega_re[i];
+    w[rpatotal + n_omega + i] = omega_im ? omega_im[i] : 0.0;
   }
-  XG_HIP(hipMemcpyAsync(dw.p, w.data(), w.size() * sizeof(double), hipMemcpyHostToDevice, st));
-  const long Kp = pk.Kp;
-  DevBuf dd((size_t)n_omega * Kp * (use16 ? sizeof(float) : sizeof(double)));
-  const double* E = de.as<double>();
-  const double* W = dw.as<double>();
-  double* d64 = use16 ? nullptr : dd.as<double>();
-  float* d32 = use16 ? dd.as<float>() : nullptr;
+  double* in = reinterpret_cast<double*>(base);
+  io.up(in, w.data(), (long)n_in, (long)n_in, 1);
+  const double* E = in;
+  const double* W = in + rpatotal;
+  double* d64 = use16 ? nullptr : reinterpret_cast<double*>(base + o_d);
+  float* d32 = use16 ? reinterpret_cast<float*>(base + o_d) : nullptr;
   const int nw = n_omega;
   launch_map(st, (size_t)n_omega * Kp, [=] __device__(size_t i) {
     long f = (long)(i / Kp), k = (long)(i % Kp);
@@ -849,17 +972,13 @@ void rpa_epsilon_impl(xtpgpu_ctx ctx, xtpgpu_mmn mmn, const double* energies, in
   });
 
   EpiEpsSym epi{out_dev, P};
-  int cus = 256;
-  {
-    hipDeviceProp_t prop;
-    if (hipGetDeviceProperties(&prop, ctx->device) == hipSuccess) cus = prop.multiProcessorCount;
-  }
+  const int cus = ctx->cus;
   // algorithmic FLOPs: n_omega * K * P * (P+1) (symmetric rank-K update); bytes: M read once + eps written
   ProfScope prof(ctx, "rpa_eps_gemm", (double)n_omega * K * P * (P + 1),
                  (double)P * K * (use16 ? (precision == XTPGPU_BF16X3 ? 4 : 2) : 8) + (double)n_omega * P * P * 8);
   if (!use16) {
     // both operands are the packed transitions; the kernel applies the weights to the B fragments
-    const Opnd<double> A{pk.A64.as<double>(), nullptr, Kp, 0};
+    const Opnd<double> A{pk.A64, nullptr, Kp, 0};
     const EvenPlan pl = f64_even_plan(P, Kp, n_omega, cus);
     DevBuf& pb = ctx->ws[2];
     pb.ensure(pl.part_bytes());
@@ -878,8 +997,8 @@ void rpa_epsilon_impl(xtpgpu_ctx ctx, xtpgpu_mmn mmn, const double* energies, in
     sc.ensure(per_w * gsz);
     unsigned short* Bh = sc.as<unsigned short>();
     unsigned short* Bl = split ? Bh + plane * gsz : nullptr;
-    const unsigned short* Ah = pk.Ah.as<unsigned short>();
-    const unsigned short* Al = pk.Al.as<unsigned short>();
+    const unsigned short* Ah = pk.Ah;
+    const unsigned short* Al = pk.Al;
     const Opnd<unsigned short> A{Ah, Al, Kp, 0};
     for (long w0 = 0; w0 < n_omega; w0 += gsz) {
       const long nw_g = std::min<long>(gsz, n_omega - w0);
@@ -942,7 +1061,8 @@ void rpa_epsilon_impl(xtpgpu_ctx ctx, xtpgpu_mmn mmn, const double* energies, in
       }
     }
   }
-  XG_HIP(hipStreamSynchronize(st));
+  if (out_host) io.down(out_host, (long)n_out, out_dev, (long)n_out, 1);
+  io.finish();
 }
 
 }  // namespace
@@ -952,6 +1072,7 @@ extern "C" int xtpgpu_rpa_epsilon_device(xtpgpu_ctx ctx, xtpgpu_mmn mmn, const d
                                          const double* omega_im, int n_omega, double eta, int precision,
                                          double* out_dev) {
   return guarded([&] {
+    XG_REQUIRE(out_dev, XTPGPU_ERR_ARG, "xtpgpu_rpa_epsilon: null argument");
     rpa_epsilon_impl(ctx, mmn, energies, homo, rpamin, rpamax, kind, omega_re, omega_im, n_omega, eta, precision,
                      out_dev);
   });
@@ -962,12 +1083,8 @@ extern "C" int xtpgpu_rpa_epsilon(xtpgpu_ctx ctx, xtpgpu_mmn mmn, const double* 
                                   const double* omega_im, int n_omega, double eta, int precision, double* out) {
   return guarded([&] {
     XG_REQUIRE(ctx && mmn && out, XTPGPU_ERR_ARG, "xtpgpu_rpa_epsilon: null argument");
-    const size_t n = (size_t)mmn->aux * mmn->aux * std::max(n_omega, 0);
-    DevBuf o(n * sizeof(double));
     rpa_epsilon_impl(ctx, mmn, energies, homo, rpamin, rpamax, kind, omega_re, omega_im, n_omega, eta, precision,
-                     o.as<double>());
-    XG_HIP(hipMemcpyAsync(out, o.p, n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    XG_HIP(hipStreamSynchronize(ctx->stream));
+                     nullptr, out);
   });
 }
 
@@ -1957,14 +2074,17 @@ extern "C" int xtpgpu_bse_matmul(xtpgpu_bseop op, int precision, const double* X
     XG_HIP(hipSetDevice(op->ctx->device));
     hipStream_t st = op->ctx->stream;
     const size_t n = (size_t)op->N * k;
-    DevBuf dx(n * 8), dy(n * 8);
-    XG_HIP(hipMemcpy2DAsync(dx.p, op->N * 8, X, ldx * 8, op->N * 8, k, hipMemcpyHostToDevice, st));
+    HostIo io(op->ctx);
+    DevBuf own;
+    double* dx = io.buffer(op->ctx->ws[6], own, 2 * n * 8).as<double>();
+    double* dy = dx + n;
+    io.up(dx, X, ldx, op->N, k);
     if (grouped_matmul_env())
-      grouped_matmul_one(op, precision, dx.as<double>(), k, dy.as<double>(), st);
+      grouped_matmul_one(op, precision, dx, k, dy, st);
     else
-      bse_matmul_impl(op, precision, dx.as<double>(), op->N, k, dy.as<double>(), op->N);
-    XG_HIP(hipMemcpy2DAsync(Y, ldy * 8, dy.p, op->N * 8, op->N * 8, k, hipMemcpyDeviceToHost, st));
-    XG_HIP(hipStreamSynchronize(st));
+      bse_matmul_impl(op, precision, dx, op->N, k, dy, op->N);
+    io.down(Y, ldy, dy, op->N, k);
+    io.finish();
   });
 }
 

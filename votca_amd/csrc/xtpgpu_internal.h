@@ -3,10 +3,13 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
 #include <stdexcept>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/xtpgpu.h"
@@ -33,38 +36,141 @@ struct Error : public std::runtime_error {
     if (!(cond)) throw ::xg::Error((code), std::string(msg)); \
   } while (0)
 
+// Large blocks (kMinBlock and more) that DevBufs of one device have given up, at most kBound bytes of them,
+// the oldest freed first. Mapping and clearing device memory costs 0.3-10 ms per GiB and giving it back
+// about as much, which is most of an operator's set-up (2.1 GB at 40 x 280 x 1280: 4.5 ms with, 2.0 without). A
+// block enters once the device is idle, as hipFree would have waited, so whichever thread or stream
+// takes it finds nothing still using it. drain() returns them: when a context lets go of its scratch or
+// ends, and before any allocation is refused.
+class BlockPool {
+ public:
+  static constexpr size_t kMinBlock = (size_t)16 << 20, kBound = (size_t)4 << 30;
+  static BlockPool& of(int device) {
+    static BlockPool* pools = new BlockPool[kDevices];  // not destroyed: buffers may outlive it at exit
+    return pools[device];
+  }
+  BlockPool() { kept_.reserve(kBound / kMinBlock + 1); }  // give() runs in destructors: no allocation there
+  static bool serves(int device) { return device >= 0 && device < kDevices; }
+  // the smallest kept block of n to n + n / 8 bytes, or null
+  void* take(size_t n, size_t& cap) {
+    std::lock_guard<std::mutex> lk(mu_);
+    size_t best = kept_.size();
+    for (size_t i = 0; i < kept_.size(); ++i)
+      if (kept_[i].cap >= n && kept_[i].cap <= n + n / 8 && (best == kept_.size() || kept_[i].cap < kept_[best].cap))
+        best = i;
+    if (best == kept_.size()) return nullptr;
+    void* p = kept_[best].p;
+    cap = kept_[best].cap;
+    total_ -= cap;
+    kept_.erase(kept_.begin() + best);
+    return p;
+  }
+  // false: not taken in, the caller frees it
+  bool give(int device, void* p, size_t cap) {
+    if (cap > kBound) return false;
+    int cur = device;
+    if (hipGetDevice(&cur) != hipSuccess) return false;
+    if (cur != device && hipSetDevice(device) != hipSuccess) return false;
+    const bool idle = hipDeviceSynchronize() == hipSuccess;
+    if (cur != device) (void)hipSetDevice(cur);
+    if (!idle) return false;
+    std::lock_guard<std::mutex> lk(mu_);
+    while (!kept_.empty() && total_ + cap > kBound) free_oldest();
+    kept_.push_back({p, cap});
+    total_ += cap;
+    return true;
+  }
+  void drain() {
+    std::lock_guard<std::mutex> lk(mu_);
+    while (!kept_.empty()) free_oldest();
+  }
+
+ private:
+  static constexpr int kDevices = 64;
+  struct Block {
+    void* p;
+    size_t cap;
+  };
+  void free_oldest() {
+    (void)hipFree(kept_.front().p);
+    total_ -= kept_.front().cap;
+    kept_.erase(kept_.begin());
+  }
+  std::mutex mu_;
+  std::vector<Block> kept_;
+  size_t total_ = 0;
+};
+
 // Owning device allocation. The allocation checks free memory first, mirroring the
 // reference's guard in CudaMatrix (xtp/src/libxtp/cudamatrix.cc:97-113).
 struct DevBuf {
   void* p = nullptr;
   size_t bytes = 0;
+  size_t cap = 0;   // bytes of the block, at least `bytes`
+  int device = -1;  // of a block that the pool takes back
   DevBuf() = default;
   explicit DevBuf(size_t n) { alloc(n); }
   DevBuf(const DevBuf&) = delete;
   DevBuf& operator=(const DevBuf&) = delete;
-  DevBuf(DevBuf&& o) noexcept : p(o.p), bytes(o.bytes) { o.p = nullptr; o.bytes = 0; }
+  DevBuf(DevBuf&& o) noexcept { swap(o); }
   DevBuf& operator=(DevBuf&& o) noexcept {
-    if (this != &o) { release(); p = o.p; bytes = o.bytes; o.p = nullptr; o.bytes = 0; }
+    if (this != &o) { release(); swap(o); }
     return *this;
+  }
+  void swap(DevBuf& o) noexcept {
+    std::swap(p, o.p); std::swap(bytes, o.bytes); std::swap(cap, o.cap); std::swap(device, o.device);
   }
   ~DevBuf() { release(); }
   void alloc(size_t n) {
     release();
     if (n == 0) return;
+    // a query of the free memory costs 5-10 us, ten times a small allocation: below 1 MiB, where the
+    // runtime mostly carves from a block that it holds, the allocation itself tells
+    int dev = -1;
+    if (n >= BlockPool::kMinBlock && hipGetDevice(&dev) == hipSuccess && BlockPool::serves(dev)) {
+      p = BlockPool::of(dev).take(n, cap);
+      if (p) {
+        bytes = n;
+        device = dev;
+        return;
+      }
+    } else {
+      dev = -1;
+    }
+    if (n >= ((size_t)1 << 20)) require_free(n);
+    hipError_t rc = hipMalloc(&p, n);
+    if (rc == hipErrorOutOfMemory) {
+      (void)hipGetLastError();
+      drain_current();
+      require_free(n);
+      rc = hipMalloc(&p, n);
+    }
+    if (rc != hipSuccess) p = nullptr;
+    XG_HIP(rc);
+    bytes = cap = n;
+    device = dev;
+  }
+  static void drain_current() {
+    int dev = -1;
+    if (hipGetDevice(&dev) == hipSuccess && BlockPool::serves(dev)) BlockPool::of(dev).drain();
+  }
+  // throws when the device has not got n bytes, kept blocks given back
+  static void require_free(size_t n) {
     size_t fr = 0, tot = 0;
+    if (hipMemGetInfo(&fr, &tot) != hipSuccess || n <= fr) return;
+    drain_current();
     if (hipMemGetInfo(&fr, &tot) == hipSuccess && n > fr)
       throw Error(XTPGPU_ERR_OOM, "device allocation of " + std::to_string(n) +
                                       " bytes exceeds free device memory (" + std::to_string(fr) + ")");
-    XG_HIP(hipMalloc(&p, n));
-    bytes = n;
   }
   void ensure(size_t n) {
     if (n > bytes) alloc(n);
   }
   void release() {
-    if (p) (void)hipFree(p);
+    if (p && !(device >= 0 && BlockPool::of(device).give(device, p, cap))) (void)hipFree(p);
     p = nullptr;
-    bytes = 0;
+    bytes = cap = 0;
+    device = -1;
   }
   template <typename T> T* as() const { return reinterpret_cast<T*>(p); }
 };
@@ -86,8 +192,17 @@ struct xtpgpu_ctx_s {
   int device = 0;
   hipStream_t stream = nullptr;
   // grow-only scratch buffers, reused across calls on this context (ws[1]: the eps builds' scaled
-  // transition copies, at most the scale budget)
-  xg::DevBuf ws[6];
+  // transition copies, at most the scale budget; ws[5], ws[6]: what calls on host arrays and the eps
+  // builds stage, at most kKeepBytes each)
+  xg::DevBuf ws[7];
+  static constexpr size_t kKeepBytes = (size_t)256 << 20;
+  int cus = 256;  // compute units of the device
+  // pinned memory for small host transfers (HostIo), allocated at the first one. It, ws[5] and ws[6] are
+  // used by the call that set io_busy, until its end; a call that finds it set does without them
+  static constexpr size_t kPinBytes = (size_t)1 << 20;  // each way
+  std::atomic<bool> io_busy{false};
+  unsigned char* pin = nullptr;
+  unsigned char* pin_dev = nullptr;  // as the device sees it
   bool profiling = false;
   void* blas = nullptr;  // rocblas_handle for the rocSOLVER calls, bound to `stream`
   std::vector<std::pair<std::string, xg::KTimer>> timers;
