@@ -43,8 +43,8 @@ def test_first_and_second_stage(o, v, P, k, c, prec, monkeypatch):
     assert np.array_equal(op.matmul(x, prec), got)
 
 
-@pytest.mark.parametrize("o,v,P,nw", [(3, 11, 1535, 2), (3, 11, 1536, 2), (4, 16, 1601, 3), (2, 67, 1793, 1)])
-def test_eps_large_aux(o, v, P, nw, monkeypatch):
+@pytest.mark.parametrize("o,v,P,nw", [(3, 40, 256, 3), (7, 60, 300, 12), (5, 130, 513, 1), (9, 70, 1100, 4), (3, 11, 1535, 2), (3, 11, 1536, 2), (4, 16, 1601, 3), (2, 67, 1793, 1)])
+def test_eps_lower_triangle(o, v, P, nw, monkeypatch):
     rng = np.random.default_rng(P + nw)
     M = rng.normal(scale=0.1, size=(o, o + v, P))
     e = np.concatenate([np.sort(rng.uniform(-1, -0.3, o)), np.sort(rng.uniform(0.1, 2.0, v))])

@@ -4,7 +4,7 @@
 //   SPLIT:   operands a = a_hi + a_lo, products hi*hi + hi*lo + lo*hi (FP32 accumulation)
 //
 // WR x WC waves, wave tile 16 TM x 16 TN of v_mfma_f32_16x16x32_bf16 tiles, a ring of STAGES LDS
-// stages (64 k, or 32 k of both planes), one barrier per stage. Three forms are used:
+// stages (64 k, or 32 k of both planes), one barrier per stage. Four forms are used:
 //   256 x 256, 16 waves of 64 x 64, 2 stages: large products. What bounds the 128 x 128
 //     register-staged tiles of gemm_bf16_kernel is LDS traffic (fragment reads plus staged writes
 //     come to the 128 bytes a CU moves per cycle at half of the MFMA rate); twice the tile edge halves
@@ -12,6 +12,8 @@
 //     of the Hd contraction at 128700 x 3000 x 900, split / plain: 2.64 / 0.98 ms with 128 x 128
 //     tiles, 2.00 / 0.83 here (347 / 840 TFLOP/s); eight waves of 128 x 64 2.11 / 0.85, of 64 x 128
 //     2.12 / 0.84, 256 x 128 tiles 2.42 / 1.01; the same without the stores 1.65 / 0.60.
+//   128 x 128, 8 waves of 32 x 64, 2 stages: products with fewer columns or a shorter K; two workgroups
+//     per CU, one's epilogue under the other's products (three stages leave room for one: 20-30% slower).
 //   256 rows x (16 TN) columns, 8 waves of 32 rows, 3 stages: second-stage products with enough of
 //     them (900 x 100 per vector, K = 29744, 30 vectors: 1193 -> 1054 us split, 440 -> 410 plain).
 //   32 rows x (32, 64, 128) columns, 2 x 2 waves, 4 stages: the same with few outputs, where each

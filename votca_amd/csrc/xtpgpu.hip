@@ -138,7 +138,7 @@ struct EpiStage1 {
   static constexpr bool kSeparable = true;
   // BF16 planes; no group of four columns crosses a vector's end
   static constexpr bool kPlanes = true;
-  __device__ bool by_four() const { return (cols & 3) == 0; }
+  __host__ __device__ bool by_four() const { return (cols & 3) == 0; }
   __device__ int planes() const { return Sl ? 2 : 1; }
   __device__ float factor(int m) const { return scale ? (float)scale[p0 + m / rows] : 1.0f; }
   struct Row {
@@ -249,15 +249,23 @@ inline int bf16_kernel_choice() {
   return 2;
 }
 
-// 256 x 256 tiles for an M x N product: enough of them for the chip's 256 CUs, at most a tenth of padding
-// over what 128 x 128 tiles compute, and a K that pays for filling and emptying the larger tile.
-// First stage of H X, 256 / 128 tiles, split and plain, us: (30 vectors of 100, 900 virtual, 700 aux)
-// 1872 / 2157, 744 / 892; (12 of 61, 430, 1200) 1408 / 1528, 725 / 748; (7 of 32, 250, 900)
-// 137 / 160, 70 / 69; (8 of 31, 250, 900) 173 / 177, 81 / 73; (26 of 33, 189, 485: a seventh of
-// padding) 249 / 234, 102 / 87.
-inline bool bf16_big_tiles(long M, long N, long K, long batch_ks, bool split) {
+// Direct-to-LDS tiles of a BF16 product, 256 x 256 (one workgroup per CU) or 128 x 128 (8 waves of
+// 32 x 64, two per CU, so that one's stores run under the other's products). The large ones need enough of
+// them for the chip's 256 CUs, at most a tenth of padding over the smaller, and a K that pays for filling
+// and emptying them. First stage of H X, 256 / 128 / register-staged 128, us:
+//                                                      split                 plain
+//   30 vectors of 100, 900 virtual levels, 143 aux   1998 / 2330 / 2520     851 /  909 /  978
+//    6 vectors of 100, 900, 286                       994 /  966 / 1104     421 /  420 /  441
+//   12 vectors of  61, 430, 600                       700 /  690 /  769     316 /  349 /  328
+//    7 vectors of  32, 250, 900                       139 /  144 /  164      66 /   59 /   66
+//   26 vectors of  33, 189, 485                       258 /  207 /  247      95 /   85 /   81
+//   12 vectors of  30, 210, 960                       272 /  213 /  247     119 /   90 /   87
+//    4 vectors of  30, 210, 960                       129 /   89 /   95      72 /   45 /   45
+// The register-staged ones remain for plain products of vectors that are not multiples of four long,
+// whose 2-byte stores the three workgroups per CU of theirs hide better.
+inline bool bf16_big_tiles(long M, long N, long K, long batch_ks) {
   const long t2 = (M + 255) / 256 * ((N + 255) / 256), t1 = (M + 127) / 128 * ((N + 127) / 128);
-  return t2 * batch_ks >= 256 && 4 * t2 * 10 <= t1 * 11 && K >= (split ? 192 : 384);
+  return t2 * batch_ks >= 256 && 4 * t2 * 10 <= t1 * 11 && K >= 384;
 }
 
 template <bool AK, bool BK_, class Epi>
@@ -267,11 +275,19 @@ void gemm16(hipStream_t st, int M, int N, int K, int batch, int ksplit, Opnd<uns
   const int choice = bf16_kernel_choice();
   if constexpr (AK && BK_) {
     if (choice == 2 && !lower && lds_ok(A, B, K, split)) {
-      if (bf16_big_tiles(M, N, K / std::max(ksplit, 1), (long)batch * std::max(ksplit, 1), split)) {
+      if (bf16_big_tiles(M, N, K / std::max(ksplit, 1), (long)batch * std::max(ksplit, 1))) {
         GemmDims d = make_dims<256, 256>(M, N, std::max(K, 0), batch, ksplit, split ? 32 : 64, false);
         d.group = d.tiles_m >= 32 && d.tiles_n >= 4 ? 4 : 0;
         XG_HIP((launch_bf16_ring<4, 4, 4, 4, 2>(st, d, A, B, split, epi)));
         return;
+      }
+      if constexpr (epi_planes<Epi>::value) {
+        if (split || epi.by_four()) {
+          GemmDims d = make_dims<128, 128>(M, N, std::max(K, 0), batch, ksplit, 64, false);
+          d.group = d.tiles_m >= 32 && d.tiles_n >= 2 ? 4 : 0;
+          XG_HIP((launch_bf16_ring<2, 4, 4, 2, 2>(st, d, A, B, split, epi)));
+          return;
+        }
       }
     }
     if (choice >= 1 && bf16_vec(A, B, K, 0)) {
@@ -1051,7 +1067,9 @@ void rpa_epsilon_impl(xtpgpu_ctx ctx, xtpgpu_mmn mmn, const double* energies, in
         DevBuf& pb = ctx->ws[2];
         pb.ensure((size_t)d.ksplit * nw_g * P * P * 4);
         const EpiPart32 ep{pb.as<float>(), P, P, nw_g};
-        if (split)
+        if (split && bf16_kernel_choice() == 2 && lds_ok(A, Bo, (int)Kp, true))
+          XG_HIP((launch_bf16_ring<2, 4, 4, 2, 2>(st, d, A, Bo, true, ep)));
+        else if (split)
           XG_HIP((launch_gemm_bf16<128, 128, true, true>(st, d, A, Bo, nullptr, 0, true, ep, true)));
         else
           XG_HIP((launch_gemm_bf16_occ<3, 64, true, true>(st, d, A, Bo, nullptr, 0, false, ep)));
