@@ -29,20 +29,14 @@
 namespace xg {
 
 // Epilogues whose rows are BF16 planes (kPlanes): the kernel rounds to hi (and lo, planes() == 2). Row m
-// carries factor(m). by_four(): 4 columns from a multiple of four are adjacent in memory, 8-byte aligned.
+// carries factor(m). width(): w = 4, 2 or 1 columns from a multiple of w are adjacent in memory, 2w-byte aligned.
 template <class E, class = void>
 struct epi_planes { static constexpr bool value = false; };
 template <class E>
 struct epi_planes<E, decltype((void)E::kPlanes)> { static constexpr bool value = E::kPlanes; };
 
 typedef unsigned short us4v __attribute__((ext_vector_type(4)));
-
-// lane `from`'s value, the same in every lane
-__device__ __forceinline__ long lane_value(long x, int from) {
-  const unsigned lo = __builtin_amdgcn_readlane((unsigned)x, from);
-  const unsigned hi = __builtin_amdgcn_readlane((unsigned)((unsigned long)x >> 32), from);
-  return (long)((unsigned long)hi << 32 | lo);
-}
+typedef unsigned short us2v __attribute__((ext_vector_type(2)));
 
 template <int TM, int TN, int WR, int WC, int STAGES, bool SPLIT, class Epi>
 __global__ __launch_bounds__(64 * WR * WC) void gemm_bf16_ring_kernel(
@@ -184,11 +178,10 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_bf16_ring_kernel(
     __syncthreads();  // every wave has read the last stage
     unsigned char* mine = lds + wave * (2 * PLANE);
     const bool two = SPLIT && epi.planes() == 2;
-    // 16 lanes of four columns to a row, or 64 of one: 2-byte stores, four times as many, where
-    // vectors end inside a group of four (31 columns, 900 x 250 rows, K = 250, split / plain: 173 / 81 us;
+    // 16 lanes of four columns to a row, 32 of two or 64 of one, as vectors end (31 columns, 900 x 250 rows, K = 250, split / plain: 173 / 81 us;
     // 8-byte stores at odd 2-byte offsets, with the cut groups one by one: 190 / 88)
-    const bool four = epi.by_four();
-    const int gn = n0 + wn0 + (four ? 4 * r16 : lane);
+    const int width = epi.width();
+    const int gn = n0 + wn0 + (width == 4 ? 4 * r16 : width == 2 ? 2 * (lane & 31) : lane);
     const long co = gn < d.N ? epi.col(b, gn) : 0;
 #pragma unroll
     for (int h = 0; h < TM / 2; ++h) {
@@ -211,7 +204,7 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_bf16_ring_kernel(
         }
       }
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      if (four) {
+      if (width == 4) {
 #pragma unroll
         for (int it = 0; it < 8; ++it) {
           const int row = 4 * it + q, gm = m0 + wm0 + 32 * h + row;
@@ -227,6 +220,21 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_bf16_ring_kernel(
       } else {
         const int mh = m0 + wm0 + 32 * h;
         const long ro = epi.row(b, ks, min(mh + (lane & 31), d.M - 1)).off;
+        if (width == 2) {
+#pragma unroll 8
+          for (int it = 0; it < 16; ++it) {
+            const int row = 2 * it + (lane >> 5);
+            const unsigned char* at = mine + row * RS + (lane & 31) * 4;
+            const us2v vh = *reinterpret_cast<const us2v*>(at);
+            const us2v vl = *reinterpret_cast<const us2v*>(at + PLANE);
+            const long r0 = lane_value(ro, 2 * it), r1 = lane_value(ro, 2 * it + 1);
+            const long idx = (lane < 32 ? r0 : r1) + co;
+            if (mh + row < d.M && gn < d.N) {
+              *reinterpret_cast<us2v*>(epi.Sh + idx) = vh;
+              if (two) *reinterpret_cast<us2v*>(epi.Sl + idx) = vl;
+            }
+          }
+        } else
 #pragma unroll 8
         for (int row = 0; row < 32; ++row) {
           if (mh + row >= d.M) break;

@@ -109,6 +109,13 @@ __device__ __forceinline__ void tile_of_block(const GemmDims& d, int& tm, int& t
   }
 }
 
+// lane `from`'s value, the same in every lane
+__device__ __forceinline__ long lane_value(long x, int from) {
+  const unsigned lo = __builtin_amdgcn_readlane((unsigned)x, from);
+  const unsigned hi = __builtin_amdgcn_readlane((unsigned)((unsigned long)x >> 32), from);
+  return (long)((unsigned long)hi << 32 | lo);
+}
+
 __device__ __forceinline__ unsigned short bf16_bits_rn(float f) {
   // round-to-nearest-even float -> bf16 (finite inputs)
   unsigned int u = __float_as_uint(f);

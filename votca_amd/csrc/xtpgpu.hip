@@ -136,9 +136,9 @@ struct EpiStage1 {
   // idx = outer * pc * colsp + p * colsp + j with outer = kv * rows + r (or r * kvec + kv):
   // the row (p, r) and column (kv, j) terms separate.
   static constexpr bool kSeparable = true;
-  // BF16 planes; no group of four columns crosses a vector's end
+  // BF16 planes; no group of `width` columns crosses a vector's end
   static constexpr bool kPlanes = true;
-  __host__ __device__ bool by_four() const { return (cols & 3) == 0; }
+  __host__ __device__ int width() const { return (cols & 3) == 0 ? 4 : (cols & 1) == 0 ? 2 : 1; }
   __device__ int planes() const { return Sl ? 2 : 1; }
   __device__ float factor(int m) const { return scale ? (float)scale[p0 + m / rows] : 1.0f; }
   struct Row {
@@ -259,10 +259,11 @@ inline int bf16_kernel_choice() {
 //   12 vectors of  61, 430, 600                       700 /  690 /  769     316 /  349 /  328
 //    7 vectors of  32, 250, 900                       139 /  144 /  164      66 /   59 /   66
 //   26 vectors of  33, 189, 485                       258 /  207 /  247      95 /   85 /   81
-//   12 vectors of  30, 210, 960                       272 /  213 /  247     119 /   90 /   87
-//    4 vectors of  30, 210, 960                       129 /   89 /   95      72 /   45 /   45
-// The register-staged ones remain for plain products of vectors that are not multiples of four long,
-// whose 2-byte stores the three workgroups per CU of theirs hide better.
+//   26 vectors of  34, 190, 485                       259 /  216 /  249      91 /   79 /   91
+//   12 vectors of  30, 210, 960                       268 /  212 /  244     114 /   86 /   95
+//    4 vectors of  30, 210, 960                       127 /   90 /   94      70 /   42 /   47
+// The register-staged ones remain for plain products of vectors of odd length, whose 2-byte stores the three
+// workgroups per CU of theirs hide better.
 inline bool bf16_big_tiles(long M, long N, long K, long batch_ks) {
   const long t2 = (M + 255) / 256 * ((N + 255) / 256), t1 = (M + 127) / 128 * ((N + 127) / 128);
   return t2 * batch_ks >= 256 && 4 * t2 * 10 <= t1 * 11 && K >= 384;
@@ -282,7 +283,7 @@ void gemm16(hipStream_t st, int M, int N, int K, int batch, int ksplit, Opnd<uns
         return;
       }
       if constexpr (epi_planes<Epi>::value) {
-        if (split || epi.by_four()) {
+        if (split || epi.width() > 1) {
           GemmDims d = make_dims<128, 128>(M, N, std::max(K, 0), batch, ksplit, 64, false);
           d.group = d.tiles_m >= 32 && d.tiles_n >= 2 ? 4 : 0;
           XG_HIP((launch_bf16_ring<2, 4, 4, 2, 2>(st, d, A, B, split, epi)));
