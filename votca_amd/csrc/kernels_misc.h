@@ -93,6 +93,12 @@ __global__ __launch_bounds__(256) void colnorm_partial_kernel(const double* __re
   if (threadIdx.x == 0) part[(long)blockIdx.y * nb + blockIdx.x] = red[0];
 }
 
+// lane `from`'s value, in every lane
+__device__ __forceinline__ double lane_value(double x, int from) {
+  const unsigned long u = lane_value((long)__double_as_longlong(x), from);
+  return __longlong_as_double((long long)u);
+}
+
 __device__ __forceinline__ double wave_sum(double s) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
@@ -111,17 +117,30 @@ __global__ __launch_bounds__(256) void colnorm_finish_kernel(const double* __res
   if (lane == 0) out[c] = sqrt(s);
 }
 
-// Sum of split-K partials, one wave per output (4 per block): lanes stride over the splits and
-// a fixed butterfly combines them, so the order is deterministic.
-__global__ __launch_bounds__(256) void reduce_partials_wave_kernel(const double* __restrict__ part, long stride,
-                                                                   int nsplit, long n, double* __restrict__ out) {
-  const long i = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (i >= n) return;
+// Sum of split-K partials for few outputs and many splits: a workgroup takes 64 outputs (lanes), its 16 waves
+// every sixteenth split each, and their sums are added in order. Output i goes to row i / len of out, ld apart.
+__global__ __launch_bounds__(1024) void reduce_partials_wave_kernel(const double* __restrict__ part, long stride,
+                                                                    int nsplit, long n, double* __restrict__ out,
+                                                                    long len, long ld) {
+  __shared__ double red[16][64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const long i = (long)blockIdx.x * 64 + lane;
   double s = 0.0;
-  for (int k = lane; k < nsplit; k += 64) s += part[(long)k * stride + i];
-  s = wave_sum(s);
-  if (lane == 0) out[i] = s;
+  if (i < n)
+    for (int k = w; k < nsplit; k += 16) s += part[(long)k * stride + i];
+  red[w][lane] = s;
+  __syncthreads();
+  if (w > 0 || i >= n) return;
+#pragma unroll
+  for (int k = 1; k < 16; ++k) s += red[k][lane];
+  const long r = i / len;
+  out[r * ld + (i - r * len)] = s;
+}
+
+inline void reduce_partials_wave(hipStream_t st, const double* part, int nsplit, long n, double* out, long len, long ld) {
+  hipLaunchKernelGGL(reduce_partials_wave_kernel, dim3((unsigned)((n + 63) / 64)), dim3(1024), 0, st, part, n, nsplit, n,
+                     out, len, ld);
+  XG_HIP(hipGetLastError());
 }
 
 // Sum of split-K partials: out[i] = sum_s part[s*stride + i] (fixed order).

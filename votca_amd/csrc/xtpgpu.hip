@@ -1233,7 +1233,8 @@ MatmulPlan plan_matmul(const xtpgpu_bseop_s* op, int precision, long k) {
     const GemmDims dd = make_dims<64, 64>((int)P, (int)k, (int)Np, 1, pick_ksplit(tiles, Np, 16), 16, false);
     pl.part = std::max(pl.part, (size_t)dd.ksplit * P * k * 8);
     pl.wbuf = (size_t)op->Pp * k * 8;
-    pl.part_more = (size_t)f64_ksplit(f64_narrow_tiles(op->N, k), op->Pp) * op->N * k * 8;
+    pl.part_more = std::max((size_t)f64_ksplit(f64_narrow_tiles(op->N, k), op->Pp) * op->N,
+                            (size_t)f64_ksplit(f64_narrow_tiles(P, k), Np) * P) * k * 8;
   }
   if ((op->cd || op->cd2) && !m16)
     pl.part_more = std::max(pl.part_more,
@@ -1519,19 +1520,14 @@ void bse_matmul_impl(xtpgpu_bseop op, int precision, const double* X, long ldx, 
   if (op->cx) {
     ProfScope prof(pctx, "hx", 4.0 * N * P * k, 8.0 * (2.0 * N * P + 2.0 * N * k));
     const int tiles = (int)(((P + 63) / 64) * ((k + 63) / 64));
-    const int ks = pick_ksplit(tiles, Np, 16);
+    // at least 128 k to a split where the buffer has room (30 x 210 x 960, 12 vectors: 15 splits 30 us)
+    const int ks = std::max(pick_ksplit(tiles, Np, 16), splits64(f64_narrow_tiles(P, k), Np, (size_t)P * k));
     GemmDims dd = make_dims<64, 64>((int)P, (int)k, (int)Np, 1, ks, 16, false);
     double* part = static_cast<double*>(part_p);
     gemm64<true, true>(st, (int)P, (int)k, (int)Np, 1, ks, Opnd<double>{op->Mvc.as<double>(), nullptr, Np, 0},
                        Opnd<double>{Xp, nullptr, Np, 0}, false, EpiPartial{part, (int)P, (int)k, 1});
     // W[kv][Pp] (pads stay zero)
-    const int nsp = dd.ksplit;
-    launch_map(st, (size_t)P * k, [=] __device__(size_t i) {
-      long kv = (long)(i / P), p = (long)(i % P);
-      double acc = 0.0;
-      for (int q = 0; q < nsp; ++q) acc += part[(long)q * P * k + i];
-      Wb[kv * Pp + p] = acc;
-    });
+    reduce_partials_wave(st, part, dd.ksplit, P * k, Wb, P, Pp);
     const Opnd<double> vt_op{op->MvcT.as<double>(), nullptr, Pp, 0}, w_op{Wb, nullptr, Pp, 0};
     const int ksb = splits64(f64_narrow_tiles(N, k), Pp, (size_t)N * k);
     if (ksb > 1 && f64_lds_ok(vt_op, w_op, (int)Pp, nullptr, 0)) {
