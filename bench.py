@@ -39,9 +39,9 @@ PEAK = {"fp64": 78.6e12, "bf16": 2.5e15, "hbm": 8.0e12}
 # WRITE_SIZE 1.0 GiB -> x1.0); FETCH_SIZE 4.462e6 / 3.159e6 KiB, WRITE_SIZE 3.450e6 / 3.490e6 KiB
 # per dispatch. The P-chunk keeps the stage-1 intermediate under 3 GiB: 286 levels for the split
 # form (two output planes), 573 for plain BF16.
-HD_STAGE1_TRAFFIC = {"bf16x3": {"read": 2.745e6 * 2.0 * 1024, "write": 3.440e6 * 1.0 * 1024,
+HD_STAGE1_TRAFFIC = {"bf16x3": {"read": 2.750e6 * 2.0 * 1024, "write": 3.440e6 * 1.0 * 1024,
                                 "launch": "30-column H X stage-1 launch, split BF16 (P-chunk 286)"},
-                     "bf16": {"read": 2.371e6 * 2.0 * 1024, "write": 3.448e6 * 1.0 * 1024,
+                     "bf16": {"read": 2.520e6 * 2.0 * 1024, "write": 3.448e6 * 1.0 * 1024,
                               "launch": "30-column H X stage-1 launch, plain BF16 (P-chunk 573)"}}
 
 
@@ -49,10 +49,10 @@ HD_STAGE1_TRAFFIC = {"bf16x3": {"read": 2.745e6 * 2.0 * 1024, "write": 3.440e6 *
 # the clock the chip holds under the load (GRBM_GUI_ACTIVE / 8 XCDs / duration), MFMA busy
 # (SQ_VALU_MFMA_BUSY_CYCLES / cycles / 1024 SIMDs) and the share of cycles the L1 waits on L2 data
 # (TCP_PENDING_STALL_CYCLES_sum / 256 CUs / cycles).
-HD_STAGE1_COUNTERS = {"bf16x3": {"clock_GHz": 1.98, "peak_at_clock_tflops": 2500.0 * 1.98 / 2.4,
-                                 "mfma_busy": 0.476, "tcp_pending_stall": 0.487},
-                      "bf16": {"clock_GHz": 2.13, "peak_at_clock_tflops": 2500.0 * 2.13 / 2.4,
-                               "mfma_busy": 0.337, "tcp_pending_stall": 0.560}}
+HD_STAGE1_COUNTERS = {"bf16x3": {"clock_GHz": 1.94, "peak_at_clock_tflops": 2500.0 * 1.94 / 2.4,
+                                 "mfma_busy": 0.518, "tcp_pending_stall": 0.453},
+                      "bf16": {"clock_GHz": 2.08, "peak_at_clock_tflops": 2500.0 * 2.08 / 2.4,
+                               "mfma_busy": 0.389, "tcp_pending_stall": 0.520}}
 
 
 def log(*a):
