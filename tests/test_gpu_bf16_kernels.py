@@ -30,7 +30,8 @@ def operator(c, o, v, P, seed):
                                      (64, 257, 24, 9), (65, 129, 40, 3), (112, 96, 12, 5), (113, 64, 16, 5),
                                      (128, 520, 70, 9), (129, 260, 33, 4), (30, 300, 600, 19), (31, 301, 600, 19),
                                      (100, 255, 257, 12), (8, 1030, 130, 31), (33, 390, 60, 31),
-                                     (64, 388, 60, 12), (30, 400, 100, 17)])
+                                     (64, 388, 60, 12), (30, 400, 100, 17), (97, 360, 90, 17), (64, 380, 130, 17),
+                                     (65, 380, 130, 15)])
 @pytest.mark.parametrize("c", [(0, 0, 1, 0), (0, 0, 0, 1)])
 @pytest.mark.parametrize("prec", ["bf16", "bf16x3"])
 def test_first_and_second_stage(o, v, P, k, c, prec, monkeypatch):

@@ -279,6 +279,17 @@ inline hipError_t launch_bf16_ring(hipStream_t st, const GemmDims& d, Opnd<unsig
   return hipGetLastError();
 }
 
+// Second-stage products for which launch_bf16_tall's tiles are the faster: where its 256-row tiles give three
+// quarters of the 256 CUs a workgroup, and else where 128 x 128 tiles would not, or with few plain columns. Narrow
+// / register-staged 128 x 128 tiles, us (4 K splits): (80 columns, 300 rows, 700 x 80 long, 4 vectors: 48
+// workgroups of the latter) split 238 / 407, plain 102 / 183; (100, 900, 500, 4 vectors: 128) 420 / 529,
+// 202 / 240; (97, 513, 996, 14: 280) 2157 / 1577, 720 / 668; (97, 360, 996, 16: 192) split 1669 / 1086; (61,
+// 430, 1000, 12: 192) 541 / 512, 227 / 261; (33, 189, 485, 26: 208) 207 / 190, 45 / 69.
+inline bool bf16_tall_pays(int M, int N, int batch, int ksplit, bool split) {
+  if ((long)((M + 255) / 256) * batch * ksplit >= 192) return true;
+  return (long)((M + 127) / 128) * batch * ksplit < 192 || (N <= 64 && !split);
+}
+
 // Second-stage products (M rows per batch entry, N <= 128 columns, long K in d.ksplit chunks):
 // 256-row tiles where they give three quarters of the 256 CUs a workgroup, else 32-row tiles. bk: what
 // K chunks are multiples of (64 / 128, as for the 128 x 128 tiles).
