@@ -263,10 +263,11 @@ inline int bf16_kernel_choice() {
 //   12 vectors of  30, 210, 960                       268 /  212 /  244     114 /   86 /   95
 //    4 vectors of  30, 210, 960                       127 /   90 /   94      70 /   42 /   47
 // The register-staged ones remain for plain products of vectors of odd length, whose 2-byte stores the three
-// workgroups per CU of theirs hide better.
-inline bool bf16_big_tiles(long M, long N, long K, long batch_ks) {
+// workgroups per CU of theirs hide better; for these the large tiles pay without padding only (14, 15
+// vectors of 97, 513, 996: 9 and 0 % of it, 1320 / 1311 and 1369 / 1501).
+inline bool bf16_big_tiles(long M, long N, long K, long batch_ks, int padding) {
   const long t2 = (M + 255) / 256 * ((N + 255) / 256), t1 = (M + 127) / 128 * ((N + 127) / 128);
-  return t2 * batch_ks >= 256 && 4 * t2 * 10 <= t1 * 11 && K >= 384;
+  return t2 * batch_ks >= 256 && 4 * t2 * 100 <= t1 * (100 + padding) && K >= 384;
 }
 
 template <bool AK, bool BK_, class Epi>
@@ -276,7 +277,10 @@ void gemm16(hipStream_t st, int M, int N, int K, int batch, int ksplit, Opnd<uns
   const int choice = bf16_kernel_choice();
   if constexpr (AK && BK_) {
     if (choice == 2 && !lower && lds_ok(A, B, K, split)) {
-      if (bf16_big_tiles(M, N, K / std::max(ksplit, 1), (long)batch * std::max(ksplit, 1))) {
+      int padding = 10;
+      if constexpr (epi_planes<Epi>::value)
+        if (!split && epi.width() == 1) padding = 2;
+      if (bf16_big_tiles(M, N, K / std::max(ksplit, 1), (long)batch * std::max(ksplit, 1), padding)) {
         GemmDims d = make_dims<256, 256>(M, N, std::max(K, 0), batch, ksplit, split ? 32 : 64, false);
         d.group = d.tiles_m >= 32 && d.tiles_n >= 4 ? 4 : 0;
         XG_HIP((launch_bf16_ring<4, 4, 4, 4, 2>(st, d, A, B, split, epi)));
