@@ -55,11 +55,12 @@ int xtpgpu_ctx_create(int device, unsigned flags, xtpgpu_ctx* out);
 int xtpgpu_ctx_destroy(xtpgpu_ctx ctx);
 int xtpgpu_ctx_synchronize(xtpgpu_ctx ctx);
 /* Free the context's grow-only scratch, kept between calls: the eps builds' scaled transition
- * copies (up to XTPGPU_EPS_SCALE_BYTES) and their partials, the adjoint's intermediates (about 1 GiB at
- * most beside its input vectors), the self-energy's partial sums, what the eps builds and the products of
- * host vectors stage (at most 256 MiB each and 2 MiB pinned); and the device blocks that destroyed
- * objects have left for reuse (at most 4 GiB per device, kept also until any context of the device ends or
- * memory runs short). The next call that needs it allocates it again. No counterpart in the reference (its GPU buffers live per call). */
+ * copies (up to XTPGPU_EPS_SCALE_BYTES) and their partials; the adjoint's intermediates, the partial sums of
+ * the self-energy and of operator diagonals, what the eps builds and the products of host vectors stage (at
+ * most 256 MiB each, and 2 MiB pinned; not those that a call on another thread is using); and the device
+ * blocks that destroyed objects have left for reuse (at most 4 GiB per device, kept also until any context
+ * of the device ends or memory runs short). The next call that needs it allocates it again. No
+ * counterpart in the reference (its GPU buffers live per call). */
 int xtpgpu_ctx_release_scratch(xtpgpu_ctx ctx);
 /* Live kernel timing: when enabled, HIP events are recorded on the context's stream around
  * the dominant launches (names: "rpa_eps_gemm", "hd_stage1" / "hd_stage2" for the split BF16x3

@@ -346,7 +346,7 @@ void copy_cols(hipStream_t st, double* dev, double* host, long ld, long rows, lo
 // The host arrays of one call. Up to kPinBytes each way pass through the context's pinned memory, which
 // a small kernel reads or writes as part of the stream's work; a copy of the runtime costs 15-25 us
 // at a few KB and 130 at 64 KB of pageable memory, the kernel 3-5. One call at a time has the context's
-// pinned memory and its ws[5], ws[6]; a second one at the same time (another thread, a chunk source that
+// pinned memory and its ws[3], ws[4]; a second one at the same time (another thread, a chunk source that
 // makes a product) has not, and copies and allocates for itself.
 class HostIo {
  public:
@@ -518,10 +518,15 @@ extern "C" int xtpgpu_ctx_release_scratch(xtpgpu_ctx ctx) {
     XG_REQUIRE(ctx, XTPGPU_ERR_ARG, "null ctx");
     XG_HIP(hipSetDevice(ctx->device));
     XG_HIP(hipStreamSynchronize(ctx->stream));
-    for (int i = 0; i < 5; ++i) ctx->ws[i].release();
-    if (!ctx->io_busy.exchange(true)) {  // else in use by a call on another thread
-      ctx->ws[5].release();
-      ctx->ws[6].release();
+    for (int i = 0; i < 3; ++i) ctx->ws[i].release();
+    for (KeptBuf* k : {&ctx->adjoint_ws, &ctx->sum_ws})
+      if (!k->busy.exchange(true)) {  // else in use by a call on another thread, as below
+        k->buf.release();
+        k->busy.store(false);
+      }
+    if (!ctx->io_busy.exchange(true)) {
+      ctx->ws[3].release();
+      ctx->ws[4].release();
       if (ctx->pin) (void)hipHostFree(ctx->pin);
       ctx->pin = ctx->pin_dev = nullptr;
       ctx->io_busy.store(false);
@@ -950,7 +955,7 @@ void rpa_epsilon_impl(xtpgpu_ctx ctx, xtpgpu_mmn mmn, const double* energies, in
   const size_t o_o = o_a + up256((size_t)P * Kp * (use16 ? 4 : 8)), total = o_o + n_out * 8;
   HostIo io(ctx);
   DevBuf own;
-  unsigned char* base = io.buffer(ctx->ws[5], own, total).as<unsigned char>();
+  unsigned char* base = io.buffer(ctx->ws[3], own, total).as<unsigned char>();
   if (out_host) out_dev = reinterpret_cast<double*>(base + o_o);
   RpaPacked pk;
   rpa_pack(mmn, n_occ, n_unocc, use16, base + o_a, pk);
@@ -1691,12 +1696,8 @@ void build_diag(xtpgpu_bseop op, xtpgpu_mmn mmn) {
   op->diag0.ensure((size_t)N * 8);
   double* d0 = op->diag0.as<double>();
   const long shares = diag_shares(op->vt, ct, P);
-  double* part = d0;
-  if (shares > 1) {
-    DevBuf& ws = op->ctx->ws[4];
-    ws.ensure((size_t)shares * N * 8);
-    part = ws.as<double>();
-  }
+  Scratch ws(op->ctx->sum_ws);
+  double* part = shares > 1 ? reinterpret_cast<double*>(ws.get((size_t)shares * N * 8)) : d0;
   diag_sums(st, mmn->d(), ps, nt, vmin_r, cmin_r, op->vt, ct, P, op->eps.as<double>(), op->cx, op->cd, op->cd2, shares,
             part);
   if (shares > 1)
@@ -2096,7 +2097,7 @@ extern "C" int xtpgpu_bse_matmul(xtpgpu_bseop op, int precision, const double* X
     const size_t n = (size_t)op->N * k;
     HostIo io(op->ctx);
     DevBuf own;
-    double* dx = io.buffer(op->ctx->ws[6], own, 2 * n * 8).as<double>();
+    double* dx = io.buffer(op->ctx->ws[4], own, 2 * n * 8).as<double>();
     double* dy = dx + n;
     io.up(dx, X, ldx, op->N, k);
     if (grouped_matmul_env())

@@ -180,6 +180,35 @@ struct DevBuf {
   template <typename T> T* as() const { return reinterpret_cast<T*>(p); }
 };
 
+// Scratch that a context keeps between calls and that one call at a time uses.
+struct KeptBuf {
+  static constexpr size_t kKeepBytes = (size_t)256 << 20;
+  DevBuf buf;
+  std::atomic<bool> busy{false};
+};
+
+// A call's scratch, for work on the context's stream only: the kept buffer, which the next call's work follows in
+// the stream; or one of its own, for a call that finds the kept one in use (another thread) or needs more than
+// is kept.
+class Scratch {
+ public:
+  explicit Scratch(KeptBuf& k) : kept_(k.busy.exchange(true) ? nullptr : &k) {}
+  ~Scratch() {
+    if (kept_) kept_->busy.store(false);
+  }
+  Scratch(const Scratch&) = delete;
+  Scratch& operator=(const Scratch&) = delete;
+  unsigned char* get(size_t bytes) {
+    DevBuf& b = kept_ && bytes <= KeptBuf::kKeepBytes ? kept_->buf : own_;
+    b.ensure(bytes);
+    return b.as<unsigned char>();
+  }
+
+ private:
+  KeptBuf* kept_;
+  DevBuf own_;
+};
+
 }  // namespace xg
 
 namespace xg {
@@ -197,12 +226,13 @@ struct xtpgpu_ctx_s {
   int device = 0;
   hipStream_t stream = nullptr;
   // grow-only scratch buffers, reused across calls on this context (ws[1]: the eps builds' scaled
-  // transition copies, at most the scale budget; ws[5], ws[6]: what calls on host arrays and the eps
+  // transition copies, at most the scale budget; ws[3], ws[4]: what calls on host arrays and the eps
   // builds stage, at most kKeepBytes each)
-  xg::DevBuf ws[7];
-  static constexpr size_t kKeepBytes = (size_t)256 << 20;
+  xg::DevBuf ws[5];
+  static constexpr size_t kKeepBytes = xg::KeptBuf::kKeepBytes;
+  xg::KeptBuf adjoint_ws, sum_ws;  // the adjoint's intermediates; partial sums of the self-energy and of operator diagonals
   int cus = 256;  // compute units of the device
-  // pinned memory for small host transfers (HostIo), allocated at the first one. It, ws[5] and ws[6] are
+  // pinned memory for small host transfers (HostIo), allocated at the first one. It, ws[3] and ws[4] are
   // used by the call that set io_busy, until its end; a call that finds it set does without them
   static constexpr size_t kPinBytes = (size_t)1 << 20;  // each way
   std::atomic<bool> io_busy{false};
