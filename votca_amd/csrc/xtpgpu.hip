@@ -346,8 +346,8 @@ void copy_cols(hipStream_t st, double* dev, double* host, long ld, long rows, lo
 // The host arrays of one call. Up to kPinBytes each way pass through the context's pinned memory, which
 // a small kernel reads or writes as part of the stream's work; a copy of the runtime costs 15-25 us
 // at a few KB and 130 at 64 KB of pageable memory, the kernel 3-5. One call at a time has the context's
-// pinned memory and its ws[3], ws[4]; a second one at the same time (another thread, a chunk source that
-// makes a product) has not, and copies and allocates for itself.
+// pinned memory; a second one at the same time (another thread, a chunk source that makes a product) has
+// not, and copies.
 class HostIo {
  public:
   explicit HostIo(xtpgpu_ctx c) : ctx_(c), st_(c->stream), kept_(!c->io_busy.exchange(true)) {
@@ -368,12 +368,6 @@ class HostIo {
   ~HostIo() {
     if (busy_) (void)hipStreamSynchronize(st_);
     if (kept_) ctx_->io_busy.store(false);
-  }
-  // `keep`, or `own` for a call that has not got it or needs more than the context keeps
-  DevBuf& buffer(DevBuf& keep, DevBuf& own, size_t bytes) const {
-    DevBuf& b = kept_ && bytes <= ctx_->kKeepBytes ? keep : own;
-    b.ensure(bytes);
-    return b;
   }
   HostIo(const HostIo&) = delete;
   HostIo& operator=(const HostIo&) = delete;
@@ -485,6 +479,7 @@ extern "C" int xtpgpu_ctx_create(int device, unsigned flags, xtpgpu_ctx* out) {
     int cus = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && cus > 0) c->cus = cus;
     XG_HIP(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
+    for (KeptBuf* k : c->kept()) KeptList::get().add(device, k);
     *out = c.release();
   });
 }
@@ -518,15 +513,9 @@ extern "C" int xtpgpu_ctx_release_scratch(xtpgpu_ctx ctx) {
     XG_REQUIRE(ctx, XTPGPU_ERR_ARG, "null ctx");
     XG_HIP(hipSetDevice(ctx->device));
     XG_HIP(hipStreamSynchronize(ctx->stream));
-    for (int i = 0; i < 3; ++i) ctx->ws[i].release();
-    for (KeptBuf* k : {&ctx->adjoint_ws, &ctx->sum_ws})
-      if (!k->busy.exchange(true)) {  // else in use by a call on another thread, as below
-        k->buf.release();
-        k->busy.store(false);
-      }
-    if (!ctx->io_busy.exchange(true)) {
-      ctx->ws[3].release();
-      ctx->ws[4].release();
+    for (auto& b : ctx->ws) b.release();
+    for (KeptBuf* k : ctx->kept()) k->release();
+    if (!ctx->io_busy.exchange(true)) {  // else in use by a call on another thread
       if (ctx->pin) (void)hipHostFree(ctx->pin);
       ctx->pin = ctx->pin_dev = nullptr;
       ctx->io_busy.store(false);
@@ -573,7 +562,7 @@ extern "C" int xtpgpu_malloc(xtpgpu_ctx ctx, int64_t bytes, void** dptr) {
     size_t fr = 0, tot = 0;
     XG_HIP(hipMemGetInfo(&fr, &tot));
     if ((size_t)bytes > fr) {
-      DevBuf::drain_current();
+      DevBuf::reclaim_current();
       XG_HIP(hipMemGetInfo(&fr, &tot));
     }
     XG_REQUIRE((size_t)bytes <= fr, XTPGPU_ERR_OOM, "xtpgpu_malloc: request exceeds free device memory");
@@ -948,14 +937,14 @@ void rpa_epsilon_impl(xtpgpu_ctx ctx, xtpgpu_mmn mmn, const double* energies, in
   const bool use16 = precision != XTPGPU_FP64;
   const long Kp = rpa_row_length(K);
   // one buffer: energies and frequencies, weights, packed transitions, and the matrices if they go to the
-  // host; kept by the context up to kKeepBytes
+  // host
   auto up256 = [](size_t n) { return (n + 255) / 256 * 256; };
   const size_t n_in = (size_t)rpatotal + 2 * n_omega, n_out = out_host ? (size_t)n_omega * P * P : 0;
   const size_t o_d = up256(n_in * 8), o_a = o_d + up256((size_t)n_omega * Kp * (use16 ? 4 : 8));
   const size_t o_o = o_a + up256((size_t)P * Kp * (use16 ? 4 : 8)), total = o_o + n_out * 8;
   HostIo io(ctx);
-  DevBuf own;
-  unsigned char* base = io.buffer(ctx->ws[3], own, total).as<unsigned char>();
+  Scratch ws(ctx->eps_ws);
+  unsigned char* base = ws.get(total);
   if (out_host) out_dev = reinterpret_cast<double*>(base + o_o);
   RpaPacked pk;
   rpa_pack(mmn, n_occ, n_unocc, use16, base + o_a, pk);
@@ -2096,8 +2085,8 @@ extern "C" int xtpgpu_bse_matmul(xtpgpu_bseop op, int precision, const double* X
     hipStream_t st = op->ctx->stream;
     const size_t n = (size_t)op->N * k;
     HostIo io(op->ctx);
-    DevBuf own;
-    double* dx = io.buffer(op->ctx->ws[4], own, 2 * n * 8).as<double>();
+    Scratch ws(op->ctx->host_ws);
+    double* dx = reinterpret_cast<double*>(ws.get(2 * n * 8));
     double* dy = dx + n;
     io.up(dx, X, ldx, op->N, k);
     if (grouped_matmul_env())

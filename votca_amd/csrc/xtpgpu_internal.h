@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <array>
 #include <atomic>
 #include <cstdio>
 #include <cstring>
@@ -41,7 +42,7 @@ struct Error : public std::runtime_error {
 // about as much, which is most of an operator's set-up (2.1 GB at 40 x 280 x 1280: 4.5 ms with, 2.0 without). A
 // block enters once the device is idle, as hipFree would have waited, so whichever thread or stream
 // takes it finds nothing still using it. drain() returns them: when a context lets go of its scratch or
-// ends, and before any allocation is refused.
+// ends, and before an allocation of this library is refused (reclaim_current).
 class BlockPool {
  public:
   static constexpr size_t kMinBlock = (size_t)16 << 20, kBound = (size_t)4 << 30;
@@ -146,7 +147,7 @@ struct DevBuf {
     hipError_t rc = hipMalloc(&p, n);
     if (rc == hipErrorOutOfMemory) {
       (void)hipGetLastError();
-      drain_current();
+      reclaim_current();
       require_free(n);
       rc = hipMalloc(&p, n);
     }
@@ -159,11 +160,13 @@ struct DevBuf {
     int dev = -1;
     if (hipGetDevice(&dev) == hipSuccess && BlockPool::serves(dev)) BlockPool::of(dev).drain();
   }
-  // throws when the device has not got n bytes, kept blocks given back
+  // what calls and destroyed objects have left for reuse on the current device goes back to it
+  static void reclaim_current();
+  // throws when the device has not got n bytes, what is kept given back
   static void require_free(size_t n) {
     size_t fr = 0, tot = 0;
     if (hipMemGetInfo(&fr, &tot) != hipSuccess || n <= fr) return;
-    drain_current();
+    reclaim_current();
     if (hipMemGetInfo(&fr, &tot) == hipSuccess && n > fr)
       throw Error(XTPGPU_ERR_OOM, "device allocation of " + std::to_string(n) +
                                       " bytes exceeds free device memory (" + std::to_string(fr) + ")");
@@ -185,7 +188,61 @@ struct KeptBuf {
   static constexpr size_t kKeepBytes = (size_t)256 << 20;
   DevBuf buf;
   std::atomic<bool> busy{false};
+  void release() {
+    if (busy.exchange(true)) return;  // in use by a call on another thread
+    buf.release();
+    busy.store(false);
+  }
 };
+
+// The kept scratch of the living contexts, by device.
+class KeptList {
+ public:
+  static KeptList& get() {
+    static KeptList* list = new KeptList;  // not destroyed: contexts may outlive it at exit
+    return *list;
+  }
+  void add(int device, KeptBuf* k) {
+    std::lock_guard<std::mutex> lk(mu_);
+    all_.push_back({device, k});
+  }
+  void remove(KeptBuf* k) {
+    std::lock_guard<std::mutex> lk(mu_);
+    for (size_t i = 0; i < all_.size(); ++i)
+      if (all_[i].second == k) {
+        all_.erase(all_.begin() + i);
+        return;
+      }
+  }
+  void release(int device) {
+    std::lock_guard<std::mutex> lk(mu_);
+    for (auto& e : all_)
+      if (e.first == device) e.second->release();
+  }
+
+ private:
+  std::mutex mu_;
+  std::vector<std::pair<int, KeptBuf*>> all_;
+};
+
+inline void DevBuf::reclaim_current() {
+  int dev = -1;
+  if (hipGetDevice(&dev) != hipSuccess) return;
+  KeptList::get().release(dev);
+  drain_current();
+}
+
+// f() of another library that allocates for itself: once more with what is kept given back when it reports
+// `no_memory` (before it has touched its operands)
+template <class S, class F>
+S with_reclaim(S no_memory, F f) {
+  S s = f();
+  if (s == no_memory) {
+    DevBuf::reclaim_current();
+    s = f();
+  }
+  return s;
+}
 
 // A call's scratch, for work on the context's stream only: the kept buffer, which the next call's work follows in
 // the stream; or one of its own, for a call that finds the kept one in use (another thread) or needs more than
@@ -226,14 +283,18 @@ struct xtpgpu_ctx_s {
   int device = 0;
   hipStream_t stream = nullptr;
   // grow-only scratch buffers, reused across calls on this context (ws[1]: the eps builds' scaled
-  // transition copies, at most the scale budget; ws[3], ws[4]: what calls on host arrays and the eps
-  // builds stage, at most kKeepBytes each)
-  xg::DevBuf ws[5];
-  static constexpr size_t kKeepBytes = xg::KeptBuf::kKeepBytes;
-  xg::KeptBuf adjoint_ws, sum_ws;  // the adjoint's intermediates; partial sums of the self-energy and of operator diagonals
+  // transition copies, at most the scale budget)
+  xg::DevBuf ws[3];
+  // the adjoint's intermediates; partial sums of the self-energy and of operator diagonals; what eps builds
+  // stage; vectors of products on host arrays
+  xg::KeptBuf adjoint_ws, sum_ws, eps_ws, host_ws;
+  std::array<xg::KeptBuf*, 4> kept() { return {&adjoint_ws, &sum_ws, &eps_ws, &host_ws}; }
+  ~xtpgpu_ctx_s() {
+    for (xg::KeptBuf* k : kept()) xg::KeptList::get().remove(k);
+  }
   int cus = 256;  // compute units of the device
-  // pinned memory for small host transfers (HostIo), allocated at the first one. It, ws[3] and ws[4] are
-  // used by the call that set io_busy, until its end; a call that finds it set does without them
+  // pinned memory for small host transfers (HostIo), allocated at the first one. It is used by the call
+  // that set io_busy, until its end; a call that finds it set does without
   static constexpr size_t kPinBytes = (size_t)1 << 20;  // each way
   std::atomic<bool> io_busy{false};
   unsigned char* pin = nullptr;
