@@ -1263,11 +1263,11 @@ void add_partials(hipStream_t st, const T* part, int nsp, long n, long batch, do
 
 // Padded copies of the k input vectors (FP64, and BF16 hi / lo when Xh / Xl are given) and the start
 // of the result: Y = cqp (H_c - H_v) X for a diagonal Hqp (hc given), else 0. One thread per padded
-// element, grid (k * vt, row length / 256).
-__global__ __launch_bounds__(256) void prep_vectors_kernel(const double* __restrict__ X, long ldx, int vt, int ct, int ctp,
-                                                           double* __restrict__ Xp, unsigned short* __restrict__ Xh,
-                                                           unsigned short* __restrict__ Xl, double* __restrict__ Y,
-                                                           long ldy, const double* __restrict__ hc,
+// element, grid (k * vt, row length / 256). Y may be X with its leading dimension: a thread reads its element
+// first; null: left alone.
+__global__ __launch_bounds__(256) void prep_vectors_kernel(const double* X, long ldx, int vt, int ct, int ctp, double* Xp,
+                                                           unsigned short* __restrict__ Xh,
+                                                           unsigned short* __restrict__ Xl, double* Y, long ldy, const double* __restrict__ hc,
                                                            const double* __restrict__ hv, double cqp) {
   const int c = blockIdx.y * 256 + threadIdx.x;
   if (c >= ctp) return;
@@ -1281,7 +1281,7 @@ __global__ __launch_bounds__(256) void prep_vectors_kernel(const double* __restr
     Xh[i] = h;
     if (Xl) Xl[i] = l;
   }
-  if (c < ct) Y[kv * ldy + (long)v * ct + c] = hc ? cqp * (hc[c] - hv[v]) * x : 0.0;
+  if (Y && c < ct) Y[kv * ldy + (long)v * ct + c] = hc ? cqp * (hc[c] - hv[v]) * x : 0.0;
 }
 
 // BSE_OPERATOR::matmul (bse_operator.cc:39-119) on device buffers. Scratch comes from the
@@ -1341,10 +1341,18 @@ void bse_matmul_impl(xtpgpu_bseop op, int precision, const double* X, long ldx, 
   const bool diag_qp = op->cqp && op->hqp_diag;
   {
     ProfScope prof(pctx, diag_qp ? "hqp" : nullptr, 2.0 * N * k, 8.0 * 3.0 * N * k);
+    const double *hc = diag_qp ? op->hcd.as<double>() : nullptr, *hv = diag_qp ? op->hvd.as<double>() : nullptr;
+    const double cqp = op->cqp;
+    // a result that lies over other vectors or elements than its own starts once all of X is copied
+    const bool apart = X + (k - 1) * ldx + N <= Y || Y + (k - 1) * ldy + N <= X || (X == Y && (ldx == ldy || k == 1));
     hipLaunchKernelGGL(prep_vectors_kernel, dim3((unsigned)(k * vt), (unsigned)((ctp + 255) / 256)), dim3(256), 0, st, X,
-                       ldx, (int)vt, (int)ct, (int)ctp, Xp, Xh, Xl, Y, ldy, diag_qp ? op->hcd.as<double>() : nullptr,
-                       diag_qp ? op->hvd.as<double>() : nullptr, (double)op->cqp);
+                       ldx, (int)vt, (int)ct, (int)ctp, Xp, Xh, Xl, apart ? Y : nullptr, ldy, hc, hv, cqp);
     XG_HIP(hipGetLastError());
+    if (!apart)
+      launch_map(st, (size_t)N * k, [=] __device__(size_t i) {
+        const long kv = (long)(i / N), r = (long)(i % N), v = r / ct, c = r % ct;
+        Y[kv * ldy + r] = hc ? cqp * (hc[c] - hv[v]) * Xp[(kv * vt + v) * ctp + c] : 0.0;
+      });
   }
 
   // ---------------- Hqp (bse_operator.cc:121-132): cqp (H_c^T X - X H_v) per vector
