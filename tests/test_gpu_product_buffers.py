@@ -1,4 +1,4 @@
-"""H X on device buffers that share memory."""
+"""H X on device buffers that share memory, and with more vectors than a grid's second dimension holds."""
 import ctypes as C
 
 import numpy as np
@@ -50,3 +50,25 @@ def test_result_over_the_vectors(shift, dx, dy, o, v, diagonal, prec):
     px._check(fn(op.h, px._PREC[prec], ptr(x0), ldx, k, ptr(y0), ldy))
     got = buf.download((size,))[y0:y0 + ldy * k].reshape((ldy, k), order="F")[:N]
     assert np.array_equal(got, want)
+
+
+def test_more_vectors_than_a_grid_dimension():
+    """The exchange product of 70000 vectors, whose second half is summed from K splits."""
+    P, k = 4096, 70000
+    op, _, M, rng = operator((0, 2, 0, 0), 1, 2, P, 5)
+    x = rng.normal(size=(2, k))
+    A = M[0, 1:, :]
+    want = 2.0 * A @ (A.T @ x)
+    # two sums of 2 and 4096 products of either sign
+    assert np.linalg.norm(op.matmul(x) - want) <= 1e-12 * np.linalg.norm(want)
+
+
+def test_more_auxiliary_functions_than_a_grid_dimension():
+    """The exchange part of the adjoint over 70000 auxiliary functions."""
+    P = 70000
+    op, _, M, rng = operator((1, 2, 0, 0), 1, 2, P, 6)
+    x = rng.normal(size=(2, 1))
+    m = M[0, 1:, :]  # (c, P)
+    want = 4.0 * (m.T @ x)[:, :, None] * x[:, 0]  # (P, 1, c)
+    got = px.bse_adjoint(op, x)[1][0]
+    assert np.linalg.norm(got - want) <= 1e-13 * np.linalg.norm(want)

@@ -117,29 +117,34 @@ __global__ __launch_bounds__(256) void colnorm_finish_kernel(const double* __res
   if (lane == 0) out[c] = sqrt(s);
 }
 
-// Sum of split-K partials for few outputs and many splits: a workgroup takes 64 outputs (lanes), its 16 waves
-// every sixteenth split each, and their sums are added in order. Output i goes to row i / len of out, ld apart.
+// Sum of split-K partials for few outputs and many splits: a workgroup takes 64 outputs (lanes) at a time, its 16
+// waves every sixteenth split each, and their sums are added in order. Output i goes to row i / len of out, ld apart.
+// The grid stays below 2^32 threads, beyond which a launch is cut short without an error.
 __global__ __launch_bounds__(1024) void reduce_partials_wave_kernel(const double* __restrict__ part, long stride,
                                                                     int nsplit, long n, double* __restrict__ out,
                                                                     long len, long ld) {
   __shared__ double red[16][64];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const long i = (long)blockIdx.x * 64 + lane;
-  double s = 0.0;
-  if (i < n)
-    for (int k = w; k < nsplit; k += 16) s += part[(long)k * stride + i];
-  red[w][lane] = s;
-  __syncthreads();
-  if (w > 0 || i >= n) return;
+  for (long i0 = (long)blockIdx.x * 64; i0 < n; i0 += (long)gridDim.x * 64) {
+    const long i = i0 + lane;
+    double s = 0.0;
+    if (i < n)
+      for (int k = w; k < nsplit; k += 16) s += part[(long)k * stride + i];
+    red[w][lane] = s;
+    __syncthreads();
+    if (w == 0 && i < n) {
 #pragma unroll
-  for (int k = 1; k < 16; ++k) s += red[k][lane];
-  const long r = i / len;
-  out[r * ld + (i - r * len)] = s;
+      for (int k = 1; k < 16; ++k) s += red[k][lane];
+      const long r = i / len;
+      out[r * ld + (i - r * len)] = s;
+    }
+    __syncthreads();
+  }
 }
 
 inline void reduce_partials_wave(hipStream_t st, const double* part, int nsplit, long n, double* out, long len, long ld) {
-  hipLaunchKernelGGL(reduce_partials_wave_kernel, dim3((unsigned)((n + 63) / 64)), dim3(1024), 0, st, part, n, nsplit, n,
-                     out, len, ld);
+  hipLaunchKernelGGL(reduce_partials_wave_kernel, dim3((unsigned)std::min<long>((n + 63) / 64, 1 << 20)), dim3(1024), 0, st,
+                     part, n, nsplit, n, out, len, ld);
   XG_HIP(hipGetLastError());
 }
 

@@ -1242,46 +1242,50 @@ MatmulPlan plan_matmul(const xtpgpu_bseop_s* op, int precision, long k) {
   return pl;
 }
 
-// Y[b][r] += alpha * (sum over the K splits of part[q][b][r], in order); grid (rows of n / 256, batch)
+// Y[b][r] += alpha * (sum over the K splits of part[q][b][r], in order); grid (rows of n / 256, batch or less)
 template <typename T>
-__global__ __launch_bounds__(256) void add_partials_kernel(const T* __restrict__ part, int nsp, long n,
+__global__ __launch_bounds__(256) void add_partials_kernel(const T* __restrict__ part, int nsp, long n, long batch,
                                                            double* __restrict__ Y, long ldy, double alpha) {
   const long r = (long)blockIdx.x * 256 + threadIdx.x;
   if (r >= n) return;
-  const long b = blockIdx.y, stride = n * gridDim.y;
-  const T* p = part + b * n + r;
-  double acc = 0.0;
-  for (int q = 0; q < nsp; ++q) acc += (double)p[q * stride];
-  Y[b * ldy + r] += alpha * acc;
+  for (long b = blockIdx.y; b < batch; b += gridDim.y) {
+    const T* p = part + b * n + r;
+    double acc = 0.0;
+    for (int q = 0; q < nsp; ++q) acc += (double)p[q * (n * batch)];
+    Y[b * ldy + r] += alpha * acc;
+  }
 }
 template <typename T>
 void add_partials(hipStream_t st, const T* part, int nsp, long n, long batch, double* Y, long ldy, double alpha) {
-  hipLaunchKernelGGL(add_partials_kernel<T>, dim3((unsigned)((n + 255) / 256), (unsigned)batch), dim3(256), 0, st, part,
-                     nsp, n, Y, ldy, alpha);
+  hipLaunchKernelGGL(add_partials_kernel<T>, dim3((unsigned)((n + 255) / 256), (unsigned)std::min<long>(batch, 65535)),
+                     dim3(256), 0, st, part, nsp, n, batch, Y, ldy, alpha);
   XG_HIP(hipGetLastError());
 }
 
 // Padded copies of the k input vectors (FP64, and BF16 hi / lo when Xh / Xl are given) and the start
 // of the result: Y = cqp (H_c - H_v) X for a diagonal Hqp (hc given), else 0. One thread per padded
-// element, grid (k * vt, row length / 256). Y may be X with its leading dimension: a thread reads its element
+// element, grid (k * vt or less, row length / 256). Y may be X with its leading dimension: a thread reads its element
 // first; null: left alone.
-__global__ __launch_bounds__(256) void prep_vectors_kernel(const double* X, long ldx, int vt, int ct, int ctp, double* Xp,
-                                                           unsigned short* __restrict__ Xh,
-                                                           unsigned short* __restrict__ Xl, double* Y, long ldy, const double* __restrict__ hc,
+__global__ __launch_bounds__(256) void prep_vectors_kernel(const double* X, long ldx, long cols, int vt, int ct, int ctp,
+                                                           double* Xp, unsigned short* __restrict__ Xh,
+                                                           unsigned short* __restrict__ Xl, double* Y, long ldy,
+                                                           const double* __restrict__ hc,
                                                            const double* __restrict__ hv, double cqp) {
   const int c = blockIdx.y * 256 + threadIdx.x;
   if (c >= ctp) return;
-  const int col = blockIdx.x, kv = col / vt, v = col - kv * vt;
-  const double x = c < ct ? X[kv * ldx + (long)v * ct + c] : 0.0;
-  const long i = (long)col * ctp + c;
-  Xp[i] = x;
-  if (Xh) {
-    unsigned short h, l;
-    split_bf16(x, h, l);
-    Xh[i] = h;
-    if (Xl) Xl[i] = l;
+  for (long col = blockIdx.x; col < cols; col += gridDim.x) {
+    const long kv = col / vt, v = col - kv * vt;
+    const double x = c < ct ? X[kv * ldx + v * ct + c] : 0.0;
+    const long i = col * ctp + c;
+    Xp[i] = x;
+    if (Xh) {
+      unsigned short h, l;
+      split_bf16(x, h, l);
+      Xh[i] = h;
+      if (Xl) Xl[i] = l;
+    }
+    if (Y && c < ct) Y[kv * ldy + v * ct + c] = hc ? cqp * (hc[c] - hv[v]) * x : 0.0;
   }
-  if (Y && c < ct) Y[kv * ldy + (long)v * ct + c] = hc ? cqp * (hc[c] - hv[v]) * x : 0.0;
 }
 
 // BSE_OPERATOR::matmul (bse_operator.cc:39-119) on device buffers. Scratch comes from the
@@ -1345,8 +1349,9 @@ void bse_matmul_impl(xtpgpu_bseop op, int precision, const double* X, long ldx, 
     const double cqp = op->cqp;
     // a result that lies over other vectors or elements than its own starts once all of X is copied
     const bool apart = X + (k - 1) * ldx + N <= Y || Y + (k - 1) * ldy + N <= X || (X == Y && (ldx == ldy || k == 1));
-    hipLaunchKernelGGL(prep_vectors_kernel, dim3((unsigned)(k * vt), (unsigned)((ctp + 255) / 256)), dim3(256), 0, st, X,
-                       ldx, (int)vt, (int)ct, (int)ctp, Xp, Xh, Xl, apart ? Y : nullptr, ldy, hc, hv, cqp);
+    hipLaunchKernelGGL(prep_vectors_kernel,
+                       dim3((unsigned)std::min<long>(k * vt, 1 << 20), (unsigned)((ctp + 255) / 256)), dim3(256), 0, st, X,
+                       ldx, k * vt, (int)vt, (int)ct, (int)ctp, Xp, Xh, Xl, apart ? Y : nullptr, ldy, hc, hv, cqp);
     XG_HIP(hipGetLastError());
     if (!apart)
       launch_map(st, (size_t)N * k, [=] __device__(size_t i) {
