@@ -165,7 +165,13 @@ __global__ __launch_bounds__(64 * WR * WC) __attribute__((amdgpu_waves_per_eu(4)
 // with two.) The workgroups of a flock walk the same k of the same operand panels on one XCD, so
 // one of them misses its L2 and the others hit. A (unit, batch) that one workgroup covers goes to
 // the epilogue; parts go to part[(2 wg + slot) BM BN], slot 0 for a unit an earlier workgroup began,
-// slot 1 for one begun here and not finished, and even_reduce_kernel adds them in order.
+// slot 1 for one begun here and not finished, and even_reduce_kernel adds them in order. A part holds the
+// fragments as the lanes do, value by value.
+// One accumulator takes at most 4096 k; the sums of longer shares are added up in the slot. The rounding
+// of a sum of K products grows with the partial sums it passes through, and with one accumulator over all of K
+// the error of eps (2-norm, against 80 bits) was 6.2e-15 at P = 2000, K = 90000, 12 frequencies and 1.3e-15 at 937,
+// 6293; it is 3.3e-16 and 7.2e-16. The slot's traffic costs 0.4-2 % (74.5 -> 75.1 and 1.347 -> 1.351 ms; P = 1535,
+// K = 27000: 14.1 -> 14.4); 1024 k give 2.4e-16 at P = 937, for 6 % at 1535.
 struct EvenShare {
   long units, steps, groups;  // groups: flocks
   int flock, bgroups;         // workgroups of a flock; batch groups (units = tiles * bgroups)
@@ -194,45 +200,59 @@ template <int TM, int TN, int WR, int WC, class Epi>
 __global__ __launch_bounds__(64 * WR * WC) __attribute__((amdgpu_waves_per_eu(4))) void gemm_f64_even_kernel(
     GemmDims d, EvenShare sh, Opnd<double> A, Opnd<double> B, const double* __restrict__ s, long s_bs, Epi epi,
     double* __restrict__ part) {
-  constexpr int BM = 16 * TM * WR, BN = 16 * TN * WC, BK = 16;
+  constexpr int BM = 16 * TM * WR, BN = 16 * TN * WC, BK = 16, NT = 64 * WR * WC;
   // consecutive workgroups on one XCD (block b runs on XCD b % 8)
   const long nb = sh.groups * sh.flock, q = nb >> 3, rem = nb & 7, x = blockIdx.x & 7;
   const long wg = x * q + (x < rem ? x : rem) + (blockIdx.x >> 3);
-  const long g = wg / sh.flock;
+  // 64-bit divisions leave their results in vector registers, of which the products need all 128
+  const long g = lane_value(wg / sh.flock, 0);
   const int member = (int)(wg - g * sh.flock);
-  const long end = sh.begin(g + 1);
-  for (long pos = sh.begin(g); pos < end;) {
-    const long u = pos / sh.steps, t0 = pos - u * sh.steps;
+  const long end = lane_value(sh.begin(g + 1), 0);
+  constexpr long kChain = 4096 / BK;
+  for (long pos = lane_value(sh.begin(g), 0); pos < end;) {
+    const long u = lane_value(pos / sh.steps, 0), t0 = pos - u * sh.steps;
     const long t1 = min(sh.steps, t0 + (end - pos));
     pos += t1 - t0;
-    const int tile = (int)(u / sh.bgroups), b = (int)(u - (long)tile * sh.bgroups) * sh.flock + member;
+    const int tile = (int)lane_value(u / sh.bgroups, 0), b = (int)(u - (long)tile * sh.bgroups) * sh.flock + member;
     if (b >= d.batch) continue;
     int tm, tn;
     lower_tile(tile, tm, tn);
+    tm = __builtin_amdgcn_readfirstlane(tm);
+    tn = __builtin_amdgcn_readfirstlane(tn);
     const bool whole = t0 == 0 && t1 == sh.steps;
     double* out = part + (2 * wg + (t0 == 0 ? 1 : 0)) * BM * BN;
-    f64_lds_tile<TM, TN, WR, WC, 2, true>(
-        d, A, B, s, s_bs, tm, tn, b, (int)t0 * BK, min(d.K, (int)t1 * BK),
-        [&](const auto& acc, auto row_of, auto col_of) {
-          if (whole) {
-            epilogue_store<TM, TN, 4>(d, epi, b, 0, acc, row_of, col_of);
-            return;
-          }
+    for (long t = t0; t < t1; t += kChain) {
+      const long te = min(t1, t + kChain);
+      f64_lds_tile<TM, TN, WR, WC, 2, true>(
+          d, A, B, s, s_bs, tm, tn, b, (int)t * BK, min(d.K, (int)te * BK),
+          [&](auto& acc, auto row_of, auto col_of) {
+            auto each = [&](auto f) {
 #pragma unroll
-          for (int i = 0; i < TM; ++i)
+              for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
+                for (int j = 0; j < TN; ++j) {
+                  unsigned at = threadIdx.x + (i * TN + j) * 4 * NT;
+                  asm volatile("" : "+v"(at)::"memory");  // else every address is computed ahead and held
 #pragma unroll
-              for (int j = 0; j < TN; ++j) out[(row_of(i, r) - tm * BM) * BN + col_of(j) - tn * BN] = acc[i][j][r];
-        });
-    __syncthreads();  // the next unit refills the LDS stages
+                  for (int r = 0; r < 4; ++r) f(acc[i][j], r, out[at + r * NT]);
+                }
+            };
+            if (t > t0) each([](d4v& v, int r, const double& o) { v[r] += o; });
+            if (whole && te == t1)
+              epilogue_store<TM, TN, 4>(d, epi, b, 0, acc, row_of, col_of);
+            else
+              each([](const d4v& v, int r, double& o) { o = v[r]; });
+          });
+      __syncthreads();  // the next piece refills the LDS stages
+    }
   }
 }
 
 // The units that several workgroups share: their parts added in order, then the epilogue.
-template <int BM, int BN, class Epi>
+template <int TM, int TN, int WR, int WC, class Epi>
 __global__ __launch_bounds__(256) void even_reduce_kernel(GemmDims d, EvenShare sh, const double* __restrict__ part,
                                                           Epi epi) {
+  constexpr int BM = 16 * TM * WR, BN = 16 * TN * WC, NT = 64 * WR * WC;
   const long u = blockIdx.x;
   const int member = blockIdx.y;
   const long g0 = sh.owner(u * sh.steps), g1 = sh.owner(u * sh.steps + sh.steps - 1);
@@ -241,10 +261,13 @@ __global__ __launch_bounds__(256) void even_reduce_kernel(GemmDims d, EvenShare 
   int tm, tn;
   lower_tile(tile, tm, tn);
   for (int e = threadIdx.x; e < BM * BN; e += 256) {
-    const int m = tm * BM + e / BN, n = tn * BN + e % BN;
+    const int row = e / BN, col = e % BN, m = tm * BM + row, n = tn * BN + col;
     if (m >= d.M || n >= d.N || m < n) continue;
-    double acc = part[(2 * (g0 * sh.flock + member) + 1) * BM * BN + e];
-    for (long g = g0 + 1; g <= g1; ++g) acc += part[2 * (g * sh.flock + member) * BM * BN + e];
+    const int value = ((row / 16 % TM) * TN + col / 16 % TN) * 4 + (row & 15) / 4;
+    const int wave = row / (16 * TM) * WC + col / (16 * TN);
+    const double* q = part + value * NT + 64 * wave + 16 * (row & 3) + (col & 15);
+    double acc = q[(2 * (g0 * sh.flock + member) + 1) * BM * BN];
+    for (long g = g0 + 1; g <= g1; ++g) acc += q[2 * (g * sh.flock + member) * BM * BN];
     epi(b, 0, m, n, acc);
   }
 }
@@ -317,12 +340,12 @@ inline hipError_t launch_f64_even(hipStream_t st, const EvenPlan& p, int P, int 
     const GemmDims d = make_dims<128, 128>(P, P, K, batch, 1, 16, true);
     hipLaunchKernelGGL((gemm_f64_even_kernel<4, 2, 2, 4, Epi>), grid, dim3(512), 0, st, d, p.sh, A, B, s, s_bs, epi, part);
     if (p.sh.groups > 1)
-      hipLaunchKernelGGL((even_reduce_kernel<128, 128, Epi>), red, dim3(256), 0, st, d, p.sh, part, epi);
+      hipLaunchKernelGGL((even_reduce_kernel<4, 2, 2, 4, Epi>), red, dim3(256), 0, st, d, p.sh, part, epi);
   } else {
     const GemmDims d = make_dims<64, 64>(P, P, K, batch, 1, 16, true);
     hipLaunchKernelGGL((gemm_f64_even_kernel<4, 1, 1, 4, Epi>), grid, dim3(256), 0, st, d, p.sh, A, B, s, s_bs, epi, part);
     if (p.sh.groups > 1)
-      hipLaunchKernelGGL((even_reduce_kernel<64, 64, Epi>), red, dim3(256), 0, st, d, p.sh, part, epi);
+      hipLaunchKernelGGL((even_reduce_kernel<4, 1, 1, 4, Epi>), red, dim3(256), 0, st, d, p.sh, part, epi);
   }
   return hipGetLastError();
 }
