@@ -1,4 +1,5 @@
-"""Dielectric builds with a long K: the sums' rounding."""
+"""Dielectric builds with a long K: the sums' rounding, K splits of the BF16 form, and the FP64 form against kernels
+that share nothing with it."""
 import numpy as np
 import pytest
 
@@ -26,3 +27,44 @@ def test_fp64_sums_in_pieces():
     x = np.longdouble(m) ** 2 * (o * v) * 4 / (1 + w.astype(np.longdouble) ** 2)
     for i in range(nw):
         assert np.abs(got[:, :, i] / (x[i] + np.eye(P)) - 1).max() <= (4096 + 24 + 8) * 2.0**-53
+
+
+def problem(o, v, P, seed):
+    rng = np.random.default_rng(seed)
+    e = np.concatenate([np.sort(rng.uniform(-1, -0.3, o)), np.sort(rng.uniform(0.1, 2.0, v))])
+    return rpa_of(rng.normal(scale=0.1, size=(o, o + v, P)), e, o)
+
+
+# K of 2048 and more is split: 128 x 128 tiles below P = 1536, 256 x 256 from there; the register-staged tiles split
+# these K in the same places, so the bits are the same
+@pytest.mark.parametrize("o,v,P,nw", [(20, 120, 257, 2), (12, 180, 300, 1), (12, 180, 384, 5), (31, 203, 937, 3),
+                                      (40, 110, 1535, 1), (31, 203, 1536, 1), (16, 300, 1800, 1)])
+def test_split_bf16_tiles(o, v, P, nw, monkeypatch):
+    rpa = problem(o, v, P, P + nw)
+    w = np.linspace(0.0, 3.0, nw)
+    got = rpa.calculate_epsilon(px.EPS_IMAG, w, "bf16x3")
+    ref = rpa.calculate_epsilon(px.EPS_IMAG, w)
+    # both operands of a product rounded to 16 bits, weights in one: 4 2^-17, times 2 for sums of either sign
+    assert np.linalg.norm(got - ref) <= 2 * 4 * 2.0**-17 * np.linalg.norm(ref)
+    monkeypatch.setenv("XTPGPU_BF16_KERNEL", "staged64")
+    assert np.array_equal(rpa.calculate_epsilon(px.EPS_IMAG, w, "bf16x3"), got)
+
+
+# tiles shared by several workgroups, and workgroups that walk several tiles in pieces of K, at both tile sizes
+@pytest.mark.parametrize("o,v,P,nw", [(3, 40, 130, 1), (31, 203, 937, 3), (31, 203, 937, 12), (20, 210, 1600, 1),
+                                      (30, 210, 1540, 8)])
+def test_fp64_against_the_batch(o, v, P, nw, monkeypatch):
+    """The many-segment build with the weights on the operand load: 64 x 64 tiles, one sum over all of K."""
+    rpa = problem(o, v, P, P + nw)
+    w = np.linspace(0.0, 3.0, nw)
+    got = rpa.calculate_epsilon(px.EPS_IMAG, w)
+    monkeypatch.setenv("XTPGPU_EPSBATCH_SCALED", "0")
+    b = px.EpsBatch([rpa], w)
+    b.run()
+    ref = b.result(0)
+    b.close()
+    for i in range(nw):
+        # sums of K products of magnitudes |sum| <= sqrt(eps_ii eps_jj), the weights being positive
+        d = np.sqrt(np.diagonal(ref[:, :, i]))
+        assert (np.abs(got[:, :, i] - ref[:, :, i]) <= 2 * (o * v + 8) * 2.0**-53 * d[:, None] * d).all()
+        assert np.array_equal(got[:, :, i], got[:, :, i].T)
