@@ -26,7 +26,7 @@ typedef double d2v __attribute__((ext_vector_type(2)));
 
 // One output tile over k in [kbeg, kend): store(acc, row_of, col_of) receives the wave's result
 // fragments (row_of(i, r), col_of(j): global row and column); called by active waves only.
-template <int TM, int TN, int WR, int WC, int STAGES, bool HAS_S, class Store>
+template <int TM, int TN, int WR, int WC, bool HAS_S, class Store>
 __device__ __forceinline__ void f64_lds_tile(const GemmDims& d, const Opnd<double>& A, const Opnd<double>& B,
                                              const double* __restrict__ s, long s_bs, int tm, int tn, int b, int kbeg,
                                              int kend, const Store& store) {
@@ -37,9 +37,7 @@ __device__ __forceinline__ void f64_lds_tile(const GemmDims& d, const Opnd<doubl
   constexpr int G = RG + (HAS_S ? 1 : 0);    // + the weights
   constexpr int LPW = (G + NW - 1) / NW;     // load instructions per wave per stage
   constexpr int STAGE_BYTES = G * 1024;
-  constexpr bool PADDED = G % NW != 0;       // some waves issue a load more: the others aim at a spare group
-    static_assert(STAGES >= 2 && (STAGES - 2) * LPW <= 63, "vmcnt range");
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[STAGES * STAGE_BYTES + (PADDED && STAGES > 2 ? 1024 : 0)];
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * STAGE_BYTES];
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -78,9 +76,9 @@ __device__ __forceinline__ void f64_lds_tile(const GemmDims& d, const Opnd<doubl
 #pragma unroll
     for (int j = 0; j < LPW; ++j) {
       const int gi = NW * j + wave;
-      if (PADDED && STAGES == 2 && gi >= G) continue;  // deeper pipelines count every wave's loads alike
+      if (G % NW != 0 && gi >= G) continue;
       const double* g = kof[j] + dk < kend ? src[j] + dk : zp;
-      dma16(g, lds0 + (unsigned)((!PADDED || gi < G) ? stage * STAGE_BYTES + gi * 1024 : STAGES * STAGE_BYTES));
+      dma16(g, lds0 + (unsigned)(stage * STAGE_BYTES + gi * 1024));
     }
   };
 
@@ -123,38 +121,29 @@ __device__ __forceinline__ void f64_lds_tile(const GemmDims& d, const Opnd<doubl
     }
   };
 
-#pragma unroll
-  for (int t = 0; t < STAGES - 1; ++t)
-    if (t < nk) issue(t, t * BK);
-  int cur = 0, fill = STAGES - 1;  // stage read in this step, stage filled during it
+  if (nk > 0) issue(0, 0);
   for (int t = 0; t < nk; ++t) {
-    // the loads of step t have landed once at most those of the later issued steps remain
-    if (STAGES >= 3 && t + STAGES - 2 < nk)
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((STAGES - 2) * LPW) : "memory");
-    else
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     // every wave's loads of step t are in LDS, and every wave has read the stage the next issue fills
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    if (t + STAGES - 1 < nk) issue(fill, (t + STAGES - 1) * BK);
-    if (active) compute(cur);
-    cur = cur + 1 == STAGES ? 0 : cur + 1;
-    fill = fill + 1 == STAGES ? 0 : fill + 1;
+    if (t + 1 < nk) issue((t + 1) & 1, (t + 1) * BK);
+    if (active) compute(t & 1);
   }
   if (active)
     store(acc, [&](int i, int r) { return m0 + wm0 + i * 16 + (lane >> 4) + 4 * r; },
           [&](int j) { return n0 + wn0 + j * 16 + (lane & 15); });
 }
 
-template <int TM, int TN, int WR, int WC, int STAGES, bool HAS_S, class Epi>
+template <int TM, int TN, int WR, int WC, class Epi>
 __global__ __launch_bounds__(64 * WR * WC) __attribute__((amdgpu_waves_per_eu(4))) void gemm_f64_lds_kernel(
-    GemmDims d, Opnd<double> A, Opnd<double> B, const double* __restrict__ s, long s_bs, Epi epi) {
+    GemmDims d, Opnd<double> A, Opnd<double> B, Epi epi) {
   int tm, tn;
   tile_of_block(d, tm, tn);
   const int b = blockIdx.z, ks = blockIdx.y;
-  f64_lds_tile<TM, TN, WR, WC, STAGES, HAS_S>(
-      d, A, B, s, s_bs, tm, tn, b, ks * d.kchunk, min(d.K, (ks + 1) * d.kchunk),
+  f64_lds_tile<TM, TN, WR, WC, false>(
+      d, A, B, nullptr, 0, tm, tn, b, ks * d.kchunk, min(d.K, (ks + 1) * d.kchunk),
       [&](const auto& acc, auto row_of, auto col_of) { epilogue_store<TM, TN, 4>(d, epi, b, ks, acc, row_of, col_of); });
 }
 
@@ -223,7 +212,7 @@ __global__ __launch_bounds__(64 * WR * WC) __attribute__((amdgpu_waves_per_eu(4)
     double* out = part + (2 * wg + (t0 == 0 ? 1 : 0)) * BM * BN;
     for (long t = t0; t < t1; t += kChain) {
       const long te = min(t1, t + kChain);
-      f64_lds_tile<TM, TN, WR, WC, 2, true>(
+      f64_lds_tile<TM, TN, WR, WC, true>(
           d, A, B, s, s_bs, tm, tn, b, (int)t * BK, min(d.K, (int)te * BK),
           [&](auto& acc, auto row_of, auto col_of) {
             auto each = [&](auto f) {
@@ -272,10 +261,9 @@ __global__ __launch_bounds__(256) void even_reduce_kernel(GemmDims d, EvenShare 
   }
 }
 
-// Both operands K-contiguous with 16-byte aligned rows, K even; weights 16-byte aligned.
-inline bool f64_lds_ok(const Opnd<double>& A, const Opnd<double>& B, int K, const double* s, long s_bs) {
-  return A.p && B.p && vec_ok(A, K, 2) && vec_ok(B, K, 2) &&
-         (!s || ((reinterpret_cast<uintptr_t>(s) % 16) == 0 && s_bs % 2 == 0));
+// Both operands K-contiguous with 16-byte aligned rows, K even.
+inline bool f64_lds_ok(const Opnd<double>& A, const Opnd<double>& B, int K) {
+  return A.p && B.p && vec_ok(A, K, 2) && vec_ok(B, K, 2);
 }
 
 // Full outputs, 128 x 64 tiles, eight waves of 32 x 32 (at 16384 x 3072, K = 896 / 4096: 67.8 / 69.1
@@ -283,7 +271,7 @@ inline bool f64_lds_ok(const Opnd<double>& A, const Opnd<double>& B, int K, cons
 template <class Epi>
 inline hipError_t launch_f64_big(hipStream_t st, const GemmDims& d, Opnd<double> A, Opnd<double> B, Epi epi) {
   const dim3 grid(gemm_tiles(d), d.ksplit, d.batch);
-  hipLaunchKernelGGL((gemm_f64_lds_kernel<2, 2, 4, 2, 2, false, Epi>), grid, dim3(512), 0, st, d, A, B, nullptr, 0L, epi);
+  hipLaunchKernelGGL((gemm_f64_lds_kernel<2, 2, 4, 2, Epi>), grid, dim3(512), 0, st, d, A, B, epi);
   return hipGetLastError();
 }
 
@@ -291,7 +279,7 @@ inline hipError_t launch_f64_big(hipStream_t st, const GemmDims& d, Opnd<double>
 template <class Epi>
 inline hipError_t launch_f64_mid(hipStream_t st, const GemmDims& d, Opnd<double> A, Opnd<double> B, Epi epi) {
   const dim3 grid(gemm_tiles(d), d.ksplit, d.batch);
-  hipLaunchKernelGGL((gemm_f64_lds_kernel<2, 2, 2, 2, 2, false, Epi>), grid, dim3(256), 0, st, d, A, B, nullptr, 0L, epi);
+  hipLaunchKernelGGL((gemm_f64_lds_kernel<2, 2, 2, 2, Epi>), grid, dim3(256), 0, st, d, A, B, epi);
   return hipGetLastError();
 }
 
@@ -302,8 +290,7 @@ inline hipError_t launch_f64_narrow_tn(hipStream_t st, int M, int N, int K, int 
                                        Opnd<double> B, Epi epi) {
   const GemmDims d = make_dims<128, 16 * TN>(M, N, K, batch, ksplit, 16, false);
   const dim3 grid(gemm_tiles(d), d.ksplit, d.batch);
-  hipLaunchKernelGGL((gemm_f64_lds_kernel<1, TN, 8, 1, 2, false, Epi>), grid, dim3(512), 0, st, d, A, B,
-                     nullptr, 0L, epi);
+  hipLaunchKernelGGL((gemm_f64_lds_kernel<1, TN, 8, 1, Epi>), grid, dim3(512), 0, st, d, A, B, epi);
   return hipGetLastError();
 }
 

@@ -345,10 +345,9 @@ __global__ __launch_bounds__(256) void gemm_f64_kernel(GemmDims d, Opnd<double> 
 // Operands are bf16 bit patterns (unsigned short). SPLIT: use hi/lo parts of both
 // operands (3 MFMAs per fragment pair). HAS_S: B(k,n) is rescaled by s[k] (float)
 // on load and re-split into hi/lo, so the weight costs no extra precision.
-// Block tile BM x BN x BKT, NT threads = (NT/128) x 2 waves.
+// Block tile BM x BN x BKT, 256 threads = 2 x 2 waves.
 // VEC: operands are K-contiguous with ld, base and K bounds multiples of 8 (16-byte loads).
-template <int BM, int BN, bool AK, bool BK_, bool SPLIT, bool HAS_S, bool VEC, class Epi, int BKT = 32, int NT = 256,
-          bool DB = false, int PAD = 8>
+template <int BM, int BN, bool AK, bool BK_, bool SPLIT, bool HAS_S, bool VEC, class Epi, int BKT = 32>
 __device__ __forceinline__ void gemm_bf16_tile(const GemmDims& d, const Opnd<unsigned short>& A,
                                                const Opnd<unsigned short>& B, const float* __restrict__ s,
                                                long s_bs, const Epi& epi, int tm, int tn, int b, int ks) {
@@ -359,20 +358,15 @@ __device__ __forceinline__ void gemm_bf16_tile(const GemmDims& d, const Opnd<uns
   // padded rows are conflict-free as well.
   constexpr int BK = BKT;
   static_assert(BK == 32 || ((BK == 64 || BK == 128) && VEC), "BK 64 / 128 need vector loads");
-  static_assert(PAD % 8 == 0, "LDS rows must stay 16-byte aligned");
-  constexpr int PK = BK + PAD;  // padded LDS row (bf16 elements)
-  static_assert(NT == 256 || NT == 512, "256 or 512 threads");
-  constexpr int WM = BM / (NT / 128), WN = BN / 2;
+  constexpr int PK = BK + 8;  // padded LDS row (bf16 elements)
+  constexpr int NT = 256;
+  constexpr int WM = BM / 2, WN = BN / 2;
   constexpr int TM = WM / 16, TN = WN / 16;
   constexpr int NS = SPLIT ? 2 : 1;
   constexpr int LA = BM * BK / NT;
   constexpr int LB = BN * BK / NT;
-  // DB: two LDS stages; the next panel is stored into the idle stage after the MFMAs of the
-  // current one, so a K step needs one barrier instead of two
-  constexpr int NB = DB ? 2 : 1;
-  __shared__ __attribute__((aligned(16))) unsigned short As_[NB][NS][BM * PK];
-  __shared__ __attribute__((aligned(16))) unsigned short Bs_[NB][NS][BN * PK];
-  int stage = 0;
+  __shared__ __attribute__((aligned(16))) unsigned short As_[NS][BM * PK];
+  __shared__ __attribute__((aligned(16))) unsigned short Bs_[NS][BN * PK];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -447,13 +441,13 @@ __device__ __forceinline__ void gemm_bf16_tile(const GemmDims& d, const Opnd<uns
       for (int i = 0; i < VA; ++i) {
         int vid = tid + i * NT;
         int mm = vid / (BK / 8), kq = 8 * (vid % (BK / 8));
-        *reinterpret_cast<us8v*>(&As_[stage][q][mm * PK + kq]) = va[q][i];
+        *reinterpret_cast<us8v*>(&As_[q][mm * PK + kq]) = va[q][i];
       }
 #pragma unroll
       for (int i = 0; i < VB; ++i) {
         int vid = tid + i * NT;
         int nn = vid / (BK / 8), kq = 8 * (vid % (BK / 8));
-        *reinterpret_cast<us8v*>(&Bs_[stage][q][nn * PK + kq]) = vb[q][i];
+        *reinterpret_cast<us8v*>(&Bs_[q][nn * PK + kq]) = vb[q][i];
       }
     }
   };
@@ -505,32 +499,32 @@ __device__ __forceinline__ void gemm_bf16_tile(const GemmDims& d, const Opnd<uns
         int idx = tid + i * NT;
         int mm, kk;
         if (AK) { mm = idx / BK; kk = idx % BK; } else { mm = idx % BM; kk = idx / BM; }
-        As_[stage][q][mm * PK + kk] = ra[q][i];
+        As_[q][mm * PK + kk] = ra[q][i];
       }
 #pragma unroll
       for (int i = 0; i < LB; ++i) {
         int idx = tid + i * NT;
         int nn, kk;
         if (BK_) { nn = idx / BK; kk = idx % BK; } else { nn = idx % BN; kk = idx / BN; }
-        Bs_[stage][q][nn * PK + kk] = rb[q][i];
+        Bs_[q][nn * PK + kk] = rb[q][i];
       }
     }
   };
 
-  auto compute = [&](int st_) {
+  auto compute = [&]() {
 #pragma unroll
     for (int kk = 0; kk < BK / 32; ++kk) {
       const int kq = kk * 32 + 8 * (lane >> 4);
       bf8v ah[TM], bh[TN], al[TM], bl[TN];
 #pragma unroll
       for (int i = 0; i < TM; ++i) {
-        ah[i] = *reinterpret_cast<const bf8v*>(&As_[st_][0][(wm0 + i * 16 + (lane & 15)) * PK + kq]);
-        if (SPLIT) al[i] = *reinterpret_cast<const bf8v*>(&As_[st_][NS - 1][(wm0 + i * 16 + (lane & 15)) * PK + kq]);
+        ah[i] = *reinterpret_cast<const bf8v*>(&As_[0][(wm0 + i * 16 + (lane & 15)) * PK + kq]);
+        if (SPLIT) al[i] = *reinterpret_cast<const bf8v*>(&As_[NS - 1][(wm0 + i * 16 + (lane & 15)) * PK + kq]);
       }
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
-        bh[j] = *reinterpret_cast<const bf8v*>(&Bs_[st_][0][(wn0 + j * 16 + (lane & 15)) * PK + kq]);
-        if (SPLIT) bl[j] = *reinterpret_cast<const bf8v*>(&Bs_[st_][NS - 1][(wn0 + j * 16 + (lane & 15)) * PK + kq]);
+        bh[j] = *reinterpret_cast<const bf8v*>(&Bs_[0][(wn0 + j * 16 + (lane & 15)) * PK + kq]);
+        if (SPLIT) bl[j] = *reinterpret_cast<const bf8v*>(&Bs_[NS - 1][(wn0 + j * 16 + (lane & 15)) * PK + kq]);
       }
 #pragma unroll
       for (int i = 0; i < TM; ++i)
@@ -546,31 +540,13 @@ __device__ __forceinline__ void gemm_bf16_tile(const GemmDims& d, const Opnd<uns
   };
 
   if (kbeg < kend) {
-    if constexpr (DB) {
-      // stage s holds panel k0 while the registers carry panel k0 + BK; every wave has left
-      // stage s ^ 1 (the barrier closing the previous step) before it is overwritten
-      load(kbeg);
+    load(kbeg);
+    for (int k0 = kbeg; k0 < kend; k0 += BK) {
+      __syncthreads();
       store();
       __syncthreads();
-      for (int k0 = kbeg; k0 < kend; k0 += BK) {
-        const bool more = k0 + BK < kend;
-        if (more) load(k0 + BK);
-        compute(stage);
-        if (more) {
-          stage ^= 1;
-          store();
-        }
-        __syncthreads();
-      }
-    } else {
-      load(kbeg);
-      for (int k0 = kbeg; k0 < kend; k0 += BK) {
-        __syncthreads();
-        store();
-        __syncthreads();
-        if (k0 + BK < kend) load(k0 + BK);
-        compute(0);
-      }
+      if (k0 + BK < kend) load(k0 + BK);
+      compute();
     }
   }
   epilogue_store<TM, TN, 4>(
@@ -579,14 +555,12 @@ __device__ __forceinline__ void gemm_bf16_tile(const GemmDims& d, const Opnd<uns
   __syncthreads();  // LDS is reused by the next tile of a persistent caller
 }
 
-template <int BM, int BN, bool AK, bool BK_, bool SPLIT, bool HAS_S, bool VEC, class Epi, int BKT = 32, int NT = 256,
-          bool DB = false, int MINW = 1, int PAD = 8>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(MINW))) void gemm_bf16_kernel(
-    GemmDims d, Opnd<unsigned short> A, Opnd<unsigned short> B, const float* __restrict__ s, long s_bs, Epi epi) {
+template <int BM, int BN, bool AK, bool BK_, bool SPLIT, bool VEC, class Epi, int BKT = 32, int MINW = 1>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MINW))) void gemm_bf16_kernel(
+    GemmDims d, Opnd<unsigned short> A, Opnd<unsigned short> B, Epi epi) {
   int tm, tn;
   tile_of_block(d, tm, tn);
-  gemm_bf16_tile<BM, BN, AK, BK_, SPLIT, HAS_S, VEC, Epi, BKT, NT, DB, PAD>(d, A, B, s, s_bs, epi, tm, tn, blockIdx.z,
-                                                                       blockIdx.y);
+  gemm_bf16_tile<BM, BN, AK, BK_, SPLIT, false, VEC, Epi, BKT>(d, A, B, nullptr, 0, epi, tm, tn, blockIdx.z, blockIdx.y);
 }
 
 // ------------------------------------------------------------------ host launch helpers
@@ -628,25 +602,18 @@ inline hipError_t launch_gemm_f64(hipStream_t st, const GemmDims& d, Opnd<double
   return hipGetLastError();
 }
 
-// K-step of the vector-load path; d.kchunk must be a multiple of it (make_dims with this bk).
-inline bool bf16_vec(const Opnd<unsigned short>& A, const Opnd<unsigned short>& B, int K, long s_bs) {
-  return vec_ok(A, K, 8) && vec_ok(B, K, 8) && (s_bs % 8 == 0);
+inline bool bf16_vec(const Opnd<unsigned short>& A, const Opnd<unsigned short>& B, int K) {
+  return vec_ok(A, K, 8) && vec_ok(B, K, 8);
 }
 
-// 128 x 128 block tile, 256 threads, one LDS stage, K step BKT for both forms, compiled for at
-// least MINW waves per SIMD (registers capped accordingly).
-template <int MINW, int BKT, bool AK, bool BK_, class Epi, int PAD = 8>
+// 128 x 128 block tile of plain BF16, K step BKT, compiled for at least MINW waves per SIMD (registers
+// capped accordingly).
+template <int MINW, int BKT, bool AK, bool BK_, class Epi>
 inline hipError_t launch_gemm_bf16_occ(hipStream_t st, const GemmDims& d, Opnd<unsigned short> A,
-                                       Opnd<unsigned short> B, const float* s, long s_bs, bool split, Epi epi) {
+                                       Opnd<unsigned short> B, Epi epi) {
   static_assert(AK && BK_, "K-contiguous operands only");
   dim3 grid(gemm_tiles(d), d.ksplit, d.batch);
-  if (split) {
-    if (s) hipLaunchKernelGGL((gemm_bf16_kernel<128, 128, AK, BK_, true, true, true, Epi, BKT, 256, false, MINW, PAD>), grid, dim3(256), 0, st, d, A, B, s, s_bs, epi);
-    else hipLaunchKernelGGL((gemm_bf16_kernel<128, 128, AK, BK_, true, false, true, Epi, BKT, 256, false, MINW, PAD>), grid, dim3(256), 0, st, d, A, B, s, s_bs, epi);
-  } else {
-    if (s) hipLaunchKernelGGL((gemm_bf16_kernel<128, 128, AK, BK_, false, true, true, Epi, BKT, 256, false, MINW, PAD>), grid, dim3(256), 0, st, d, A, B, s, s_bs, epi);
-    else hipLaunchKernelGGL((gemm_bf16_kernel<128, 128, AK, BK_, false, false, true, Epi, BKT, 256, false, MINW, PAD>), grid, dim3(256), 0, st, d, A, B, s, s_bs, epi);
-  }
+  hipLaunchKernelGGL((gemm_bf16_kernel<128, 128, AK, BK_, false, true, Epi, BKT, MINW>), grid, dim3(256), 0, st, d, A, B, epi);
   return hipGetLastError();
 }
 
@@ -655,31 +622,25 @@ inline hipError_t launch_gemm_bf16_occ(hipStream_t st, const GemmDims& d, Opnd<u
 inline int bf16_wide_kstep(bool split) { return split ? 64 : 128; }
 
 template <int BM, int BN, bool AK, bool BK_, class Epi>
-inline hipError_t launch_gemm_bf16(hipStream_t st, const GemmDims& d, Opnd<unsigned short> A,
-                                   Opnd<unsigned short> B, const float* s, long s_bs, bool split,
-                                   Epi epi, bool wide = false) {
+inline hipError_t launch_gemm_bf16(hipStream_t st, const GemmDims& d, Opnd<unsigned short> A, Opnd<unsigned short> B,
+                                   bool split, Epi epi, bool wide = false) {
   dim3 grid(gemm_tiles(d), d.ksplit, d.batch);
-  const bool vec = AK && BK_ && bf16_vec(A, B, d.K, s_bs);
+  const bool vec = AK && BK_ && bf16_vec(A, B, d.K);
+#define XG_BF16_LAUNCH(SP, VV, BKT) \
+  hipLaunchKernelGGL((gemm_bf16_kernel<BM, BN, AK, BK_, SP, VV, Epi, BKT>), grid, dim3(256), 0, st, d, A, B, epi)
   if constexpr (AK && BK_) {
     if (vec && wide) {
-      if (split) {
-        if (s) hipLaunchKernelGGL((gemm_bf16_kernel<BM, BN, AK, BK_, true, true, true, Epi, 64>), grid, dim3(256), 0, st, d, A, B, s, s_bs, epi);
-        else hipLaunchKernelGGL((gemm_bf16_kernel<BM, BN, AK, BK_, true, false, true, Epi, 64>), grid, dim3(256), 0, st, d, A, B, s, s_bs, epi);
-      } else {
-        if (s) hipLaunchKernelGGL((gemm_bf16_kernel<BM, BN, AK, BK_, false, true, true, Epi, 128>), grid, dim3(256), 0, st, d, A, B, s, s_bs, epi);
-        else hipLaunchKernelGGL((gemm_bf16_kernel<BM, BN, AK, BK_, false, false, true, Epi, 128>), grid, dim3(256), 0, st, d, A, B, s, s_bs, epi);
-      }
+      if (split) XG_BF16_LAUNCH(true, true, 64);
+      else XG_BF16_LAUNCH(false, true, 128);
       return hipGetLastError();
     }
   }
-#define XG_BF16_LAUNCH(SP, HS, VV) \
-  hipLaunchKernelGGL((gemm_bf16_kernel<BM, BN, AK, BK_, SP, HS, VV, Epi>), grid, dim3(256), 0, st, d, A, B, s, s_bs, epi)
   if (vec) {
-    if (split) { if (s) XG_BF16_LAUNCH(true, true, true); else XG_BF16_LAUNCH(true, false, true); }
-    else { if (s) XG_BF16_LAUNCH(false, true, true); else XG_BF16_LAUNCH(false, false, true); }
+    if (split) XG_BF16_LAUNCH(true, true, 32);
+    else XG_BF16_LAUNCH(false, true, 32);
   } else {
-    if (split) { if (s) XG_BF16_LAUNCH(true, true, false); else XG_BF16_LAUNCH(true, false, false); }
-    else { if (s) XG_BF16_LAUNCH(false, true, false); else XG_BF16_LAUNCH(false, false, false); }
+    if (split) XG_BF16_LAUNCH(true, false, 32);
+    else XG_BF16_LAUNCH(false, false, 32);
   }
 #undef XG_BF16_LAUNCH
   return hipGetLastError();

@@ -93,12 +93,6 @@ __global__ __launch_bounds__(256) void colnorm_partial_kernel(const double* __re
   if (threadIdx.x == 0) part[(long)blockIdx.y * nb + blockIdx.x] = red[0];
 }
 
-// lane `from`'s value, in every lane
-__device__ __forceinline__ double lane_value(double x, int from) {
-  const unsigned long u = lane_value((long)__double_as_longlong(x), from);
-  return __longlong_as_double((long long)u);
-}
-
 __device__ __forceinline__ double wave_sum(double s) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);

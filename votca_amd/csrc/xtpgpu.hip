@@ -194,8 +194,8 @@ inline int tile_group(const GemmDims& d) {
 
 // Super-block size of the lower-triangle tile order (0 = row by row, the default): G x G tiles
 // keep G row and G column panels in flight per XCD instead of one row panel and every column
-// panel. XTPGPU_LOWER_GROUP=G selects it; on the eps builds it measured level with row by row
-// (FP64 51.6 / 51.4, BF16x3 210.8 / 212.1 TFLOP/s at P = 2000).
+// panel. XTPGPU_LOWER_GROUP=G selects it for the BF16 eps builds on 128 x 128 tiles, where it measured level
+// with row by row.
 inline int lower_tile_group(const GemmDims& d) {
   const char* e = std::getenv("XTPGPU_LOWER_GROUP");
   if (e) return std::max(0, std::atoi(e));
@@ -204,39 +204,36 @@ inline int lower_tile_group(const GemmDims& d) {
 }
 
 template <bool AK, bool BK_, class Epi>
-void gemm64(hipStream_t st, int M, int N, int K, int batch, int ksplit, Opnd<double> A, Opnd<double> B,
-            bool lower, Epi epi) {
+void gemm64(hipStream_t st, int M, int N, int K, int batch, int ksplit, Opnd<double> A, Opnd<double> B, Epi epi) {
   if (M <= 0 || N <= 0 || batch <= 0) return;
   K = std::max(K, 0);
   const long big_tiles = (long)((M + 127) / 128) * ((N + 127) / 128) * batch * std::max(ksplit, 1);
   if constexpr (AK && BK_) {
     // K-contiguous, 16-byte aligned operands: direct-to-LDS kernels. Up to 64 columns the tile is as
     // wide as N; beyond, 128 x 64 tiles while they give half the chip's 512 resident workgroups one
-    // each, 64 x 64 tiles below that and for a lower triangle.
-    if (f64_lds_ok(A, B, K, nullptr, 0)) {
+    // each, 64 x 64 tiles below that.
+    if (f64_lds_ok(A, B, K)) {
       const long big = (long)((M + 127) / 128) * ((N + 63) / 64) * batch * std::max(ksplit, 1);
-      if (!lower && N <= 64) {
+      if (N <= 64) {
         XG_HIP(launch_f64_narrow(st, M, N, K, batch, ksplit, A, B, epi));
-      } else if (!lower && M > 64 && big >= 256) {
+      } else if (M > 64 && big >= 256) {
         GemmDims d = make_dims<128, 64>(M, N, K, batch, ksplit, 16, false);
         d.group = tile_group(d);
         XG_HIP(launch_f64_big(st, d, A, B, epi));
       } else {
-        GemmDims d = make_dims<64, 64>(M, N, K, batch, ksplit, 16, lower);
-        if (lower) d.group = lower_tile_group(d);
-        XG_HIP(launch_f64_mid(st, d, A, B, epi));
+        XG_HIP(launch_f64_mid(st, make_dims<64, 64>(M, N, K, batch, ksplit, 16, false), A, B, epi));
       }
       return;
     }
   }
   // 128x128 tiles halve the operand traffic per FLOP; used when the grid still fills the chip
   if (ksplit <= 1 && M >= 256 && N >= 256 && big_tiles >= 512) {
-    GemmDims d = make_dims<128, 128>(M, N, K, batch, ksplit, 16, lower);
-    d.group = lower ? lower_tile_group(d) : tile_group(d);
+    GemmDims d = make_dims<128, 128>(M, N, K, batch, ksplit, 16, false);
+    d.group = tile_group(d);
     XG_HIP((launch_gemm_f64<128, 128, AK, BK_>(st, d, A, B, epi)));
     return;
   }
-  GemmDims d = make_dims<64, 64>(M, N, K, batch, ksplit, 16, lower);
+  GemmDims d = make_dims<64, 64>(M, N, K, batch, ksplit, 16, false);
   XG_HIP((launch_gemm_f64<64, 64, AK, BK_>(st, d, A, B, epi)));
 }
 
@@ -295,20 +292,20 @@ void gemm16(hipStream_t st, int M, int N, int K, int batch, int ksplit, Opnd<uns
         }
       }
     }
-    if (choice >= 1 && bf16_vec(A, B, K, 0)) {
+    if (choice >= 1 && bf16_vec(A, B, K)) {
       GemmDims d = make_dims<128, 128>(M, N, std::max(K, 0), batch, ksplit, 64, lower);
       d.group = lower ? lower_tile_group(d) : tile_group(d);
       // plain BF16: registers capped for three waves per SIMD (148 VGPRs, 37 KB LDS: three workgroups
       // per CU) -- latency hiding by occupancy; split: two workgroups per CU
       if (split)
-        XG_HIP((launch_gemm_bf16<128, 128, AK, BK_>(st, d, A, B, nullptr, 0, split, epi, true)));
+        XG_HIP((launch_gemm_bf16<128, 128, AK, BK_>(st, d, A, B, split, epi, true)));
       else
-        XG_HIP((launch_gemm_bf16_occ<3, 64, AK, BK_>(st, d, A, B, nullptr, 0, split, epi)));
+        XG_HIP((launch_gemm_bf16_occ<3, 64, AK, BK_>(st, d, A, B, epi)));
       return;
     }
   }
   GemmDims d = make_dims<128, 128>(M, N, std::max(K, 0), batch, ksplit, 32, lower);
-  XG_HIP((launch_gemm_bf16<128, 128, AK, BK_>(st, d, A, B, nullptr, 0, split, epi)));
+  XG_HIP((launch_gemm_bf16<128, 128, AK, BK_>(st, d, A, B, split, epi)));
 }
 
 // Number of K splits so that tiles*splits gives about four workgroups per CU, with K chunks
@@ -715,7 +712,7 @@ extern "C" int xtpgpu_mmn_multiply_right(xtpgpu_mmn mmn, const double* A, int64_
     for (long n0 = 0; n0 < MN; n0 += (1L << 30)) {
       int nn = (int)std::min<long>(MN - n0, 1L << 30);
       gemm64<true, false>(ctx->stream, (int)P, nn, (int)P, 1, 1, Opnd<double>{dA.as<double>(), nullptr, lda, 0},
-                          Opnd<double>{mmn->d() + n0, nullptr, MN, 0}, false,
+                          Opnd<double>{mmn->d() + n0, nullptr, MN, 0},
                           EpiStore{out.as<double>() + n0, MN, 1, 0, 1.0, 0.0});
     }
     XG_HIP(hipStreamSynchronize(ctx->stream));
@@ -743,12 +740,12 @@ extern "C" int xtpgpu_mmn_fill_ao2mo(xtpgpu_mmn mmn, const double* ao3c, int64_t
     const double* Cn = dC.as<double>() + (long)mmn->nmin * ldc;
     // A(m, mu) = Cm[mu + m*ldc] (K-contiguous); B(mu, nu) = T[Q][mu + nu*nb] (K-contiguous)
     gemm64<true, true>(ctx->stream, (int)mt, (int)nb, (int)nb, (int)P, 1, Opnd<double>{Cm, nullptr, ldc, 0},
-                       Opnd<double>{dT.as<double>(), nullptr, nb, nb * nb}, false,
+                       Opnd<double>{dT.as<double>(), nullptr, nb, nb * nb},
                        EpiStore{dH.as<double>(), nb, 1, mt * nb, 1.0, 0.0});
     // step 2: M[Q][m][n] = sum_nu H[Q](m, nu) Cn(nu, n)  ->  data[Q*mt*nt + m*nt + n]
     gemm64<true, true>(ctx->stream, (int)mt, (int)nt, (int)nb, (int)P, 1,
                        Opnd<double>{dH.as<double>(), nullptr, nb, mt * nb}, Opnd<double>{Cn, nullptr, ldc, 0},
-                       false, EpiStore{mmn->d(), nt, 1, mt * nt, 1.0, 0.0});
+                       EpiStore{mmn->d(), nt, 1, mt * nt, 1.0, 0.0});
     XG_HIP(hipStreamSynchronize(ctx->stream));
     mmn->version++;
   });
@@ -1047,7 +1044,7 @@ void rpa_epsilon_impl(xtpgpu_ctx ctx, xtpgpu_mmn mmn, const double* energies, in
       const Opnd<unsigned short> Bo{Bh, Bl, Kp, (long)plane};
       const long tl = (P + 127) / 128;
       // the default kernels keep 2 (split) or 3 (plain) 128 x 128 workgroups per CU resident
-      const int ks = (P >= 256 && bf16_kernel_choice() >= 1 && bf16_vec(A, Bo, (int)Kp, 0))
+      const int ks = (P >= 256 && bf16_kernel_choice() >= 1 && bf16_vec(A, Bo, (int)Kp))
                          ? eps_ksplit(tl * (tl + 1) / 2 * nw_g, (split ? 2L : 3L) * cus, Kp, 64) : 1;
       // split form from P = 1536: 256 x 256 tiles (one workgroup per CU), K split to fill their rounds;
       // below, the 128 x 128 tiles fill the chip better (a loop of the 256 uneven segments' builds,
@@ -1069,9 +1066,9 @@ void rpa_epsilon_impl(xtpgpu_ctx ctx, xtpgpu_mmn mmn, const double* energies, in
         if (split && bf16_kernel_choice() == 2 && lds_ok(A, Bo, (int)Kp, true))
           XG_HIP((launch_bf16_ring<2, 4, 4, 2, 2>(st, d, A, Bo, true, ep)));
         else if (split)
-          XG_HIP((launch_gemm_bf16<128, 128, true, true>(st, d, A, Bo, nullptr, 0, true, ep, true)));
+          XG_HIP((launch_gemm_bf16<128, 128, true, true>(st, d, A, Bo, true, ep, true)));
         else
-          XG_HIP((launch_gemm_bf16_occ<3, 64, true, true>(st, d, A, Bo, nullptr, 0, false, ep)));
+          XG_HIP((launch_gemm_bf16_occ<3, 64, true, true>(st, d, A, Bo, ep)));
         eps_reduce_splits(st, pb.as<float>(), d.ksplit, nw_g, P, out_dev + w0 * P * P);
       } else {
         gemm16<true, true>(st, (int)P, (int)P, (int)Kp, (int)nw_g, 1, A, Bo, split, true, eg);
@@ -1366,11 +1363,11 @@ void bse_matmul_impl(xtpgpu_bseop op, int precision, const double* X, long ldx, 
     const double cqp = op->cqp;
     // out_kv(c1, v1) += cqp * sum_c' Hc(c', c1) X_kv(c', v1)   (batched over kv)
     gemm64<true, true>(st, (int)ct, (int)vt, (int)ct, (int)k, 1, Opnd<double>{op->hc.as<double>(), nullptr, ct, 0},
-                       Opnd<double>{Xp, nullptr, ctp, vt * ctp}, false,
+                       Opnd<double>{Xp, nullptr, ctp, vt * ctp},
                        EpiStore{Y, 1, ct, ldy, cqp, 1.0});
     // out_kv(c1, v1) -= cqp * sum_v' X_kv(c1, v') Hv(v', v1)
     gemm64<false, true>(st, (int)ct, (int)vt, (int)vt, (int)k, 1, Opnd<double>{Xp, nullptr, ctp, vt * ctp},
-                        Opnd<double>{op->hv.as<double>(), nullptr, vt, 0}, false,
+                        Opnd<double>{op->hv.as<double>(), nullptr, vt, 0},
                         EpiStore{Y, 1, ct, ldy, -cqp, 1.0});
   }
 
@@ -1398,13 +1395,13 @@ void bse_matmul_impl(xtpgpu_bseop op, int precision, const double* X, long ldx, 
   auto stage2_fp64 = [&](Opnd<double> A, Opnd<double> B, long np, double alpha) {
     const long K2 = np * vtp;
     const int ks = splits64(f64_narrow_tiles(ct, vt) * k, K2, (size_t)ct * vt * k);
-    if (ks > 1 && f64_lds_ok(A, B, (int)K2, nullptr, 0)) {
+    if (ks > 1 && f64_lds_ok(A, B, (int)K2)) {
       double* pt = static_cast<double*>(part_p);
       const GemmDims dd = make_dims<128, 16>((int)ct, (int)vt, (int)K2, (int)k, ks, 16, false);
       XG_HIP(launch_f64_narrow(st, (int)ct, (int)vt, (int)K2, (int)k, ks, A, B, EpiPartial{pt, (int)ct, (int)vt, (int)k}));
       add_partials(st, pt, dd.ksplit, ct * vt, k, Y, ldy, alpha);
     } else {
-      gemm64<true, true>(st, (int)ct, (int)vt, (int)K2, (int)k, 1, A, B, false,
+      gemm64<true, true>(st, (int)ct, (int)vt, (int)K2, (int)k, 1, A, B,
                          EpiStore{Y, 1, ct, ldy, alpha, 1.0});
     }
   };
@@ -1420,8 +1417,8 @@ void bse_matmul_impl(xtpgpu_bseop op, int precision, const double* X, long ldx, 
     if (fits && vt <= 128 && bf16_kernel_choice() == 2 && lds_ok(A, B, (int)K2, split) &&
         bf16_tall_pays((int)ct, (int)vt, (int)k, dd.ksplit, split)) {
       XG_HIP(launch_bf16_tall(st, (int)ct, (int)vt, (int)K2, (int)k, ks, bk, A, B, split, ep));
-    } else if (fits && ks > 1 && bf16_vec(A, B, (int)K2, 0)) {
-      XG_HIP((launch_gemm_bf16<128, 128, true, true>(st, dd, A, B, nullptr, 0, split, ep, true)));
+    } else if (fits && ks > 1 && bf16_vec(A, B, (int)K2)) {
+      XG_HIP((launch_gemm_bf16<128, 128, true, true>(st, dd, A, B, split, ep, true)));
     } else {
       gemm16<true, true>(st, (int)ct, (int)vt, (int)K2, (int)k, 1, A, B, split, false, EpiStore{Y, 1, ct, ldy, alpha, 1.0});
       return;
@@ -1463,7 +1460,7 @@ void bse_matmul_impl(xtpgpu_bseop op, int precision, const double* X, long ldx, 
         {
           ProfScope prof(pctx, "hd_stage1_fp64", f1, b1);
           gemm64<true, true>(st, (int)M1, (int)N1, (int)round8(ct), 1, 1, Opnd<double>{mcc, nullptr, ctp, 0},
-                             Opnd<double>{Xp, nullptr, ctp, 0}, false, e1);
+                             Opnd<double>{Xp, nullptr, ctp, 0}, e1);
         }
         ProfScope prof(pctx, "hd_stage2_fp64", f2, b2);
         stage2_fp64(Opnd<double>{S, nullptr, k * np * vtp, np * vtp},
@@ -1509,7 +1506,7 @@ void bse_matmul_impl(xtpgpu_bseop op, int precision, const double* X, long ldx, 
         e1.S64 = S;
         gemm64<true, true>(st, (int)M1, (int)N1, (int)round8(ct), 1, 1,
                            Opnd<double>{op->Mvc.as<double>() + p0 * Np, nullptr, ctp, 0},
-                           Opnd<double>{Xp, nullptr, ctp, 0}, false, e1);
+                           Opnd<double>{Xp, nullptr, ctp, 0}, e1);
         stage2_fp64(Opnd<double>{op->McvT.as<double>() + p0 * vtp, nullptr, P * vtp, 0},
                     Opnd<double>{S, nullptr, np * vtp, vt * np * vtp}, np, alpha);
       } else {
@@ -1537,17 +1534,17 @@ void bse_matmul_impl(xtpgpu_bseop op, int precision, const double* X, long ldx, 
     GemmDims dd = make_dims<64, 64>((int)P, (int)k, (int)Np, 1, ks, 16, false);
     double* part = static_cast<double*>(part_p);
     gemm64<true, true>(st, (int)P, (int)k, (int)Np, 1, ks, Opnd<double>{op->Mvc.as<double>(), nullptr, Np, 0},
-                       Opnd<double>{Xp, nullptr, Np, 0}, false, EpiPartial{part, (int)P, (int)k, 1});
+                       Opnd<double>{Xp, nullptr, Np, 0}, EpiPartial{part, (int)P, (int)k, 1});
     // W[kv][Pp] (pads stay zero)
     reduce_partials_wave(st, part, dd.ksplit, P * k, Wb, P, Pp);
     const Opnd<double> vt_op{op->MvcT.as<double>(), nullptr, Pp, 0}, w_op{Wb, nullptr, Pp, 0};
     const int ksb = splits64(f64_narrow_tiles(N, k), Pp, (size_t)N * k);
-    if (ksb > 1 && f64_lds_ok(vt_op, w_op, (int)Pp, nullptr, 0)) {
+    if (ksb > 1 && f64_lds_ok(vt_op, w_op, (int)Pp)) {
       const GemmDims db = make_dims<128, 16>((int)N, (int)k, (int)Pp, 1, ksb, 16, false);
       XG_HIP(launch_f64_narrow(st, (int)N, (int)k, (int)Pp, 1, ksb, vt_op, w_op, EpiPartial{part, (int)N, (int)k, 1}));
       add_partials(st, part, db.ksplit, N, k, Y, ldy, (double)op->cx);
     } else {
-      gemm64<true, true>(st, (int)N, (int)k, (int)Pp, 1, 1, vt_op, w_op, false,
+      gemm64<true, true>(st, (int)N, (int)k, (int)Pp, 1, 1, vt_op, w_op,
                          EpiStore{Y, 1, ldy, 0, (double)op->cx, 1.0});
     }
   }
@@ -1737,8 +1734,8 @@ extern "C" int xtpgpu_bse_create(xtpgpu_ctx ctx, xtpgpu_mmn mmn, const double* e
                "xtpgpu_bse_create: BSE window exceeds the Mmn tensor");
     op->vt = vt; op->ct = ct; op->N = vt * ct; op->P = mmn->aux;
     op->ctp = ct >= 64 ? (ct + 63) / 64 * 64 : round8(ct); op->vtp = round8(vt); op->Pp = round8(op->P);
-    const long P = op->P, N = op->N, nt = mmn->ntotal, ps = (long)mmn->pstride();
-    const long ctp = op->ctp, vtp = op->vtp, Pp = op->Pp, Np = vt * ctp;
+    const long P = op->P, nt = mmn->ntotal, ps = (long)mmn->pstride();
+    const long ctp = op->ctp, vtp = op->vtp;
     XG_HIP(hipSetDevice(ctx->device));
     hipStream_t st = ctx->stream;
     setup_hqp_eps(op.get(), Hqp, ldhqp, eps0inv);
@@ -1956,7 +1953,7 @@ extern "C" int xtpgpu_bse_create_streamed(xtpgpu_ctx ctx, xtpgpu_mmn_chunk_fn so
       // p * vtp + j) and W's column q read as row q (W = eps^-1(0) is symmetric)
       gemm64<false, true>(st, (int)vtp, (int)P, (int)P, (int)vt, 1,
                           Opnd<double>{braw.as<double>(), nullptr, vtp, P * vtp},
-                          Opnd<double>{wm.as<double>(), nullptr, P, 0}, false,
+                          Opnd<double>{wm.as<double>(), nullptr, P, 0},
                           EpiStore{Bvv, 1, vtp, P * vtp, 1.0, 0.0});
       XG_HIP(hipStreamSynchronize(st));
     }
