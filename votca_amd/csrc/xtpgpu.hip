@@ -211,11 +211,14 @@ void gemm64(hipStream_t st, int M, int N, int K, int batch, int ksplit, Opnd<dou
   if constexpr (AK && BK_) {
     // K-contiguous, 16-byte aligned operands: direct-to-LDS kernels. Up to 64 columns the tile is as
     // wide as N; beyond, 128 x 64 tiles while they give half the chip's 512 resident workgroups one
-    // each, 64 x 64 tiles below that, and also for 33 to 64 columns on fewer than 256 workgroups, where a tile's own
-    // products are what is waited for (full Hqp of 60 x 450: 56.8 us against 71.6 for one vector, 85.8 / 87.4 for 33).
+    // each, 64 x 64 tiles below that. On fewer than 256 workgroups a tile's own products are what is waited
+    // for, and 33 to 64 columns go in two of 32 (full Hqp of 60 x 450: 56.2 us against 71.4 for one vector, 85.5 / 88.3 for
+    // 33; exchange of 6 x 30 x 48, 33 vectors: 35.6 / 38.7; 64 x 64 tiles 56.0, 86.3 and 40.4).
     if (f64_lds_ok(A, B, K)) {
       const long big = (long)((M + 127) / 128) * ((N + 63) / 64) * batch * std::max(ksplit, 1);
-      if (N <= 32 || (N <= 64 && big >= 256)) {
+      if (N > 32 && N <= 64 && big < 256) {
+        XG_HIP(launch_f64_narrow_tn<2>(st, M, N, K, batch, ksplit, A, B, epi));
+      } else if (N <= 64) {
         XG_HIP(launch_f64_narrow(st, M, N, K, batch, ksplit, A, B, epi));
       } else if (M > 64 && big >= 256) {
         GemmDims d = make_dims<128, 64>(M, N, K, batch, ksplit, 16, false);
