@@ -1265,28 +1265,26 @@ void add_partials(hipStream_t st, const T* part, int nsp, long n, long batch, do
 
 // Padded copies of the k input vectors (FP64, and BF16 hi / lo when Xh / Xl are given) and the start
 // of the result: Y = cqp (H_c - H_v) X for a diagonal Hqp (hc given), else 0. One thread per padded
-// element, grid (k * vt or less, row length / 256). Y may be X with its leading dimension: a thread reads its element
-// first; null: left alone.
-__global__ __launch_bounds__(256) void prep_vectors_kernel(const double* X, long ldx, long cols, int vt, int ct, int ctp,
-                                                           double* Xp, unsigned short* __restrict__ Xh,
+// element, grid (k * vt, row length / 256): indices in 32 bits, a 64-bit division takes 1.5 us of the 30 that a small
+// product takes. Y may be X with its leading dimension: a thread reads its element first; null: left alone.
+__global__ __launch_bounds__(256) void prep_vectors_kernel(const double* X, long ldx, int vt, int ct, int ctp, double* Xp,
+                                                           unsigned short* __restrict__ Xh,
                                                            unsigned short* __restrict__ Xl, double* Y, long ldy,
                                                            const double* __restrict__ hc,
                                                            const double* __restrict__ hv, double cqp) {
   const int c = blockIdx.y * 256 + threadIdx.x;
   if (c >= ctp) return;
-  for (long col = blockIdx.x; col < cols; col += gridDim.x) {
-    const long kv = col / vt, v = col - kv * vt;
-    const double x = c < ct ? X[kv * ldx + v * ct + c] : 0.0;
-    const long i = col * ctp + c;
-    Xp[i] = x;
-    if (Xh) {
-      unsigned short h, l;
-      split_bf16(x, h, l);
-      Xh[i] = h;
-      if (Xl) Xl[i] = l;
-    }
-    if (Y && c < ct) Y[kv * ldy + v * ct + c] = hc ? cqp * (hc[c] - hv[v]) * x : 0.0;
+  const int col = blockIdx.x, kv = col / vt, v = col - kv * vt;
+  const double x = c < ct ? X[kv * ldx + (long)v * ct + c] : 0.0;
+  const long i = (long)col * ctp + c;
+  Xp[i] = x;
+  if (Xh) {
+    unsigned short h, l;
+    split_bf16(x, h, l);
+    Xh[i] = h;
+    if (Xl) Xl[i] = l;
   }
+  if (Y && c < ct) Y[kv * ldy + (long)v * ct + c] = hc ? cqp * (hc[c] - hv[v]) * x : 0.0;
 }
 
 // BSE_OPERATOR::matmul (bse_operator.cc:39-119) on device buffers. Scratch comes from the
@@ -1350,10 +1348,14 @@ void bse_matmul_impl(xtpgpu_bseop op, int precision, const double* X, long ldx, 
     const double cqp = op->cqp;
     // a result that lies over other vectors or elements than its own starts once all of X is copied
     const bool apart = X + (k - 1) * ldx + N <= Y || Y + (k - 1) * ldy + N <= X || (X == Y && (ldx == ldy || k == 1));
-    hipLaunchKernelGGL(prep_vectors_kernel,
-                       dim3((unsigned)std::min<long>(k * vt, 1 << 20), (unsigned)((ctp + 255) / 256)), dim3(256), 0, st, X,
-                       ldx, k * vt, (int)vt, (int)ct, (int)ctp, Xp, Xh, Xl, apart ? Y : nullptr, ldy, hc, hv, cqp);
-    XG_HIP(hipGetLastError());
+    const long most = std::max<long>(1, (1L << 23) / vt);  // vectors of one launch, below 2^32 threads
+    for (long k0 = 0; k0 < k; k0 += most) {
+      const long o = k0 * Np;
+      hipLaunchKernelGGL(prep_vectors_kernel, dim3((unsigned)(std::min(most, k - k0) * vt), (unsigned)((ctp + 255) / 256)),
+                         dim3(256), 0, st, X + k0 * ldx, ldx, (int)vt, (int)ct, (int)ctp, Xp + o, Xh ? Xh + o : nullptr,
+                         Xl ? Xl + o : nullptr, apart ? Y + k0 * ldy : nullptr, ldy, hc, hv, cqp);
+      XG_HIP(hipGetLastError());
+    }
     if (!apart)
       launch_map(st, (size_t)N * k, [=] __device__(size_t i) {
         const long kv = (long)(i / N), r = (long)(i % N), v = r / ct, c = r % ct;
