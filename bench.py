@@ -36,7 +36,7 @@ PEAK = {"fp64": 78.6e12, "bf16": 2.5e15, "hbm": 8.0e12}
 # from rocprofv3 --pmc FETCH_SIZE and --pmc WRITE_SIZE runs of
 # `bench.py --workload matvec --steps 1 [--mixed bf16] --copy-calibration`, each scaled by what the
 # same counter reads for the 1 GiB copy16_kernel in that run (FETCH_SIZE 0.5 GiB -> x2.0,
-# WRITE_SIZE 1.0 GiB -> x1.0); FETCH_SIZE 4.462e6 / 3.159e6 KiB, WRITE_SIZE 3.450e6 / 3.490e6 KiB
+# WRITE_SIZE 1.0 GiB -> x1.0); FETCH_SIZE 2.750e6 / 2.520e6 KiB, WRITE_SIZE 3.440e6 / 3.448e6 KiB
 # per dispatch. The P-chunk keeps the stage-1 intermediate under 3 GiB: 286 levels for the split
 # form (two output planes), 573 for plain BF16.
 HD_STAGE1_TRAFFIC = {"bf16x3": {"read": 2.750e6 * 2.0 * 1024, "write": 3.440e6 * 1.0 * 1024,

@@ -264,8 +264,10 @@ inline int bf16_kernel_choice() {
 //   12 vectors of  30, 210, 960                       268 /  212 /  244     114 /   86 /   95
 //    4 vectors of  30, 210, 960                       127 /   90 /   94      70 /   42 /   47
 // The register-staged ones remain for plain products of vectors of odd length, whose 2-byte stores the three
-// workgroups per CU of theirs hide better; for these the large tiles pay without padding only (14, 15
-// vectors of 97, 513, 996: 9 and 0 % of it, 1320 / 1311 and 1369 / 1501).
+// workgroups per CU of theirs hide better than the 128 x 128 tiles. Against the large tiles they are level with a
+// tenth of padding (large / staged, 14 vectors of 97, 513, 996: 1266 / 1274; 21 of 61, 430, 1000: 890-962 / 935) and 1-18 %
+// slower without (15 of 97: 1290 / 1420; 8, 12, 16 of 61: 363 / 410, 527 / 580, 720 / 737; 14 of 35, 400, 900: 335 / 370; 30 of
+// 91, 700, 800: 1422 / 1603; 17 of 45, 385, 1200: 573 / 669).
 inline bool bf16_big_tiles(long M, long N, long K, long batch_ks, int padding) {
   const long t2 = (M + 255) / 256 * ((N + 255) / 256), t1 = (M + 127) / 128 * ((N + 127) / 128);
   return t2 * batch_ks >= 256 && 4 * t2 * 100 <= t1 * (100 + padding) && K >= 384;
@@ -627,6 +629,7 @@ extern "C" int xtpgpu_mmn_create(xtpgpu_ctx ctx, int64_t mmin, int64_t mmax, int
     XG_HIP(hipSetDevice(ctx->device));
     auto t = std::make_unique<xtpgpu_mmn_s>();
     t->ctx = ctx;
+    t->device = ctx->device;
     t->mmin = mmin; t->mmax = mmax; t->nmin = nmin; t->nmax = nmax;
     t->mtotal = mmax - mmin + 1;
     t->ntotal = nmax - nmin + 1;
@@ -642,9 +645,8 @@ extern "C" int xtpgpu_mmn_create(xtpgpu_ctx ctx, int64_t mmin, int64_t mmax, int
 extern "C" int xtpgpu_mmn_destroy(xtpgpu_mmn mmn) {
   return guarded([&] {
     if (!mmn) return;
-    (void)hipSetDevice(mmn->ctx->device);
-    (void)hipStreamSynchronize(mmn->ctx->stream);
-    delete mmn;
+    (void)hipSetDevice(mmn->device);
+    delete mmn;  // the device is waited for as its buffer goes
   });
 }
 
@@ -1119,6 +1121,7 @@ extern "C" int xtpgpu_rpa_epsilon(xtpgpu_ctx ctx, xtpgpu_mmn mmn, const double* 
 // so that every GEMM reads both operands K-contiguous with 16-byte vectors.
 struct xtpgpu_bseop_s {
   xtpgpu_ctx ctx = nullptr;
+  int device = 0;  // the context's, which may end first
   int cqp = 0, cx = 0, cd = 0, cd2 = 0;
   long vt = 0, ct = 0, N = 0, P = 0;
   long ctp = 0, vtp = 0, Pp = 0;
@@ -1728,6 +1731,7 @@ extern "C" int xtpgpu_bse_create(xtpgpu_ctx ctx, xtpgpu_mmn mmn, const double* e
     XG_REQUIRE((cd == 0 && cd2 == 0) || eps0inv, XTPGPU_ERR_ARG, "xtpgpu_bse_create: eps0inv required for Hd/Hd2");
     auto op = std::make_unique<xtpgpu_bseop_s>();
     op->ctx = ctx;
+    op->device = ctx->device;
     op->cqp = cqp; op->cx = cx; op->cd = cd; op->cd2 = cd2;
     op->mask = (precision_mask | 1u) & ((1u << XTPGPU_FP64) | (1u << XTPGPU_BF16) | (1u << XTPGPU_BF16X3));
     // BSE_OPERATOR::configure (bse_operator.cc:28-37)
@@ -1814,6 +1818,7 @@ extern "C" int xtpgpu_bse_create_streamed(xtpgpu_ctx ctx, xtpgpu_mmn_chunk_fn so
     XG_REQUIRE(vmin >= rpamin && homo >= vmin && cmax > homo, XTPGPU_ERR_SHAPE, "xtpgpu_bse_create_streamed: empty BSE window");
     auto op = std::make_unique<xtpgpu_bseop_s>();
     op->ctx = ctx;
+    op->device = ctx->device;
     op->cqp = cqp; op->cx = cx; op->cd = cd; op->cd2 = cd2;
     op->mask = (precision_mask | 1u) & ((1u << XTPGPU_FP64) | (1u << XTPGPU_BF16) | (1u << XTPGPU_BF16X3));
     const long vt = homo - vmin + 1, ct = cmax - homo;
@@ -2032,9 +2037,8 @@ extern "C" int xtpgpu_bse_memory(xtpgpu_bseop op, int64_t* bytes) {
 extern "C" int xtpgpu_bse_destroy(xtpgpu_bseop op) {
   return guarded([&] {
     if (!op) return;
-    (void)hipSetDevice(op->ctx->device);
-    (void)hipStreamSynchronize(op->ctx->stream);
-    delete op;
+    (void)hipSetDevice(op->device);
+    delete op;  // the device is waited for as its buffers go
   });
 }
 

@@ -38,8 +38,9 @@ struct Error : public std::runtime_error {
   } while (0)
 
 // Large blocks (kMinBlock and more) that DevBufs of one device have given up, at most kBound bytes of them,
-// the oldest freed first. Mapping and clearing device memory costs 0.3-10 ms per GiB and giving it back
-// about as much, which is most of an operator's set-up (2.1 GB at 40 x 280 x 1280: 4.5 ms with, 2.0 without). A
+// the oldest freed first. Mapping and clearing device memory costs 0.2-10 ms per GiB, the more the process has
+// mapped, and giving it back about as much: an operator's set-up of 2.1 GB (40 x 280 x 1280) takes 2.06 ms where it
+// finds blocks that another of its size left, 2.4 where it does not, and 50 in a process with much memory mapped. A
 // block enters once the device is idle, as hipFree would have waited, so whichever thread or stream
 // takes it finds nothing still using it. drain() returns them: when a context lets go of its scratch or
 // ends, and before an allocation of this library is refused (reclaim_current).
@@ -363,6 +364,7 @@ struct ProfScope {
 
 struct xtpgpu_mmn_s {
   xtpgpu_ctx ctx = nullptr;
+  int device = 0;  // the context's, which may end first (an interpreter's exit finalises objects in any order)
   int64_t mmin = 0, mmax = 0, nmin = 0, nmax = 0, mtotal = 0, ntotal = 0, aux = 0;
   // Device layout, aux-major: element (m, n, P) at data[P*mtotal*ntotal + m*ntotal + n].
   xg::DevBuf data;
