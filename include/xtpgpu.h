@@ -52,6 +52,7 @@ int xtpgpu_device_count(int* count);
 /* One context per (device, stream); replaces OpenMP_CUDA::SetNoGPUs / GPU_data
  * (xtp/src/libxtp/openmp_cuda.cc:28-71). flags must be 0. */
 int xtpgpu_ctx_create(int device, unsigned flags, xtpgpu_ctx* out);
+/* Handles made with the context may be destroyed after it, but not used. */
 int xtpgpu_ctx_destroy(xtpgpu_ctx ctx);
 int xtpgpu_ctx_synchronize(xtpgpu_ctx ctx);
 /* Free the context's grow-only scratch, kept between calls: the eps builds' scaled transition
