@@ -279,24 +279,35 @@ inline hipError_t launch_bf16_ring(hipStream_t st, const GemmDims& d, Opnd<unsig
   return hipGetLastError();
 }
 
-// Second-stage products for which launch_bf16_tall's tiles are the faster: where its 256-row tiles give three
-// quarters of the 256 CUs a workgroup, and else where 128 x 128 tiles would not, or with few plain columns. Narrow
-// / register-staged 128 x 128 tiles, us (4 K splits): (80 columns, 300 rows, 700 x 80 long, 4 vectors: 48
-// workgroups of the latter) split 238 / 407, plain 102 / 183; (100, 900, 500, 4 vectors: 128) 420 / 529,
-// 202 / 240; (97, 513, 996, 14: 280) 2157 / 1577, 720 / 668; (97, 360, 996, 16: 192) split 1669 / 1086; (61,
-// 430, 1000, 12: 192) 541 / 512, 227 / 261; (33, 189, 485, 26: 208) 207 / 190, 45 / 69.
-inline bool bf16_tall_pays(int M, int N, int batch, int ksplit, bool split) {
-  if ((long)((M + 255) / 256) * batch * ksplit >= 192) return true;
-  return (long)((M + 127) / 128) * batch * ksplit < 192 || (N <= 64 && !split);
+// Tiles of a second-stage product: M rows per batch entry, N <= 128 columns, a long K in ksplit chunks.
+enum class Bf16Second { kStaged, kRows256, kRows32 };
+
+// The form that gives the CU with the most workgroups the least to do. `c` workgroups of a form on one of the 256 CUs
+// take, per K, c times the weight below: 32-row tiles (2 to 5 of them run at a time) by their width, 256-row tiles (one at a
+// time), register-staged 128 x 128 tiles two at a time, or one for somewhat more than half of that (the plain
+// one of up to 64 columns for somewhat more). Weights: ns per 10^4 k of the split form, of which the plain
+// one takes 0.40 to 0.45, from 110 products on all three forms; the choice is within 4 % of the fastest on 109 of them and
+// 8 % on all. One threshold on the workgroups had missed the rounds (staged / 256 / 32 rows, split, us): 303 rows, 102
+// columns, 45 vectors, K = 105040 in 3: 270 of the 256-row tiles, 2706 / 4706 / 4218; 640, 100, 30, 72800 in 3: 270, 1922 /
+// 2799 / 3599; 256, 100, 20, 104000 in 4: 640 of the 32-row ones, 940 / 1457 / 1443. Where it had been right: 300, 97,
+// 28, 93600 in 4: 1734 / 1377 / 1901; 210, 30, 15, 30720 in 4: 251 / 319 / 143.
+inline Bf16Second bf16_second_form(int M, int N, int batch, int ksplit, bool split) {
+  const long n = (long)batch * ksplit;
+  auto per_cu = [&](int rows) { return ((M + rows - 1) / rows * n + 255) / 256; };
+  const bool narrow = N <= 64;
+  const long c = per_cu(128);
+  const long staged = c / 2 * (narrow ? 520 : 720) + c % 2 * (!narrow ? 410 : split ? 310 : 340);
+  const long rows256 = per_cu(256) * (narrow ? 490 : 600);
+  const long rows32 = per_cu(32) * (N <= 32 ? 95 : narrow ? 108 : 187);
+  if (staged <= rows256 && staged <= rows32) return Bf16Second::kStaged;
+  return rows256 <= rows32 ? Bf16Second::kRows256 : Bf16Second::kRows32;
 }
 
-// Second-stage products (M rows per batch entry, N <= 128 columns, long K in d.ksplit chunks):
-// 256-row tiles where they give three quarters of the 256 CUs a workgroup, else 32-row tiles. bk: what
-// K chunks are multiples of (64 / 128, as for the 128 x 128 tiles).
+// The 256-row or 32-row tiles. bk: what K chunks are multiples of (64 / 128, as for the 128 x 128 tiles).
 template <class Epi>
-inline hipError_t launch_bf16_tall(hipStream_t st, int M, int N, int K, int batch, int ksplit, int bk,
+inline hipError_t launch_bf16_tall(hipStream_t st, Bf16Second form, int M, int N, int K, int batch, int ksplit, int bk,
                                    Opnd<unsigned short> A, Opnd<unsigned short> B, bool split, Epi epi) {
-  if ((long)((M + 255) / 256) * batch * ksplit >= 192) {
+  if (form == Bf16Second::kRows256) {
     const int tn = (N + 15) / 16;
 #define XG_TALL(TN) \
   return launch_bf16_ring<2, TN, 8, 1, 3>(st, make_dims<256, 16 * TN>(M, N, K, batch, ksplit, bk, false), A, B, split, epi)
