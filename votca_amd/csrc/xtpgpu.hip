@@ -1203,12 +1203,24 @@ struct MatmulPlan {
 // workgroups cover the chip's 512 resident ones: as many as fit one round, at least 128 k each; from
 // a round on, up to four where they fill the last round. A second-stage product of one segment has
 // ct x vt outputs per vector over K = (P, v'): 30 tiles over K = 30720 at (30, 210, 960) with 15
-// vectors took 1606 us unsplit, 17 splits of it 120 us.
+// vectors took 1606 us unsplit, 17 splits of it 120 us. With 129 to 256 tiles two or three splits leave up to a third of
+// the places empty: more, of 1024 k or longer, where the busiest CU's workgroups (two at a time, one alone for 1.17 of half
+// of that: 240 tiles 8202 us unsplit, 7045 in two) take a tenth less: 180 tiles, K = 210840: 2 splits 27.5 ms, 4 21.2;
+// 140, 71808: 3 6.36, 7 5.28; 135, 105040: 3 8.10, 7 6.75. Not for less: 150, 61600: 3 4.47, 5 4.64.
 int f64_ksplit(long units, long K) {
   constexpr long kResident = 512;
   if (units <= 0) return 1;
-  if (units <= kResident / 2) return (int)std::max<long>(1, std::min<long>(kResident / units, K / 128));
-  return eps_ksplit(units, kResident, K, 16);
+  if (units > kResident / 2) return eps_ksplit(units, kResident, K, 16);
+  long best = std::max<long>(1, std::min<long>(kResident / units, K / 128));
+  if (units > kResident / 4) {
+    auto busiest = [&](long ks) {
+      const long c = (units * ks + kResident / 2 - 1) / (kResident / 2);
+      return (c / 2 * 2.0 + c % 2 * 1.17) / (double)ks;
+    };
+    for (long ks = best + 1; ks <= 8 && K / ks >= 1024; ++ks)
+      if (busiest(ks) < 0.9 * busiest(best)) best = ks;
+  }
+  return (int)best;
 }
 
 // Output tiles of the narrow FP64 kernel.
