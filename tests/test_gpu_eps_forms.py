@@ -68,3 +68,23 @@ def test_fp64_against_the_batch(o, v, P, nw, monkeypatch):
         d = np.sqrt(np.diagonal(ref[:, :, i]))
         assert (np.abs(got[:, :, i] - ref[:, :, i]) <= 2 * (o * v + 8) * 2.0**-53 * d[:, None] * d).all()
         assert np.array_equal(got[:, :, i], got[:, :, i].T)
+
+
+# flocks of 4, 3, 2 and 1 frequencies, and the sizes between which the tiles change: 64 x 64 up to 1216, 128 x 128 up to 1280
+# with three frequencies or more, then 64, 128 from 1345 on, all from 1536
+@pytest.mark.parametrize("P,nw", [(70, 3), (130, 9), (200, 6), (65, 11), (1216, 2), (1217, 3), (1280, 1), (1281, 4), (1344, 3),
+                                  (1345, 5), (1409, 9), (1472, 1), (1473, 2), (1473, 3)])
+def test_fp64_deal(P, nw):
+    o, v = 4, 9
+    rng = np.random.default_rng(P + nw)
+    M = rng.normal(scale=0.1, size=(o, o + v, P))
+    e = np.concatenate([np.sort(rng.uniform(-1, -0.3, o)), np.sort(rng.uniform(0.1, 2.0, v))])
+    w = np.linspace(0.0, 3.0, nw)
+    got = rpa_of(M, e, o).calculate_epsilon(px.EPS_IMAG, w)
+    A = M[:, o:, :].reshape(o * v, P)
+    D = (e[None, o:] - e[:o, None]).reshape(-1)
+    for i in range(nw):
+        ref = np.eye(P) + A.T @ ((4.0 * D / (D * D + w[i] * w[i]))[:, None] * A)
+        d = np.sqrt(np.diagonal(ref))
+        # sums of 36 products each way, of magnitudes |sum| <= sqrt(eps_ii eps_jj)
+        assert (np.abs(got[:, :, i] - ref) <= 2 * (o * v + 8) * 2.0**-53 * d[:, None] * d).all()

@@ -203,7 +203,6 @@ __global__ __launch_bounds__(64 * WR * WC) __attribute__((amdgpu_waves_per_eu(4)
     const long t1 = min(sh.steps, t0 + (end - pos));
     pos += t1 - t0;
     const int tile = (int)lane_value(u / sh.bgroups, 0), b = (int)(u - (long)tile * sh.bgroups) * sh.flock + member;
-    if (b >= d.batch) continue;
     int tm, tn;
     lower_tile(tile, tm, tn);
     tm = __builtin_amdgcn_readfirstlane(tm);
@@ -246,7 +245,7 @@ __global__ __launch_bounds__(256) void even_reduce_kernel(GemmDims d, EvenShare 
   const int member = blockIdx.y;
   const long g0 = sh.owner(u * sh.steps), g1 = sh.owner(u * sh.steps + sh.steps - 1);
   const int tile = (int)(u / sh.bgroups), b = (int)(u - (long)tile * sh.bgroups) * sh.flock + member;
-  if (g0 == g1 || b >= d.batch) return;
+  if (g0 == g1) return;
   int tm, tn;
   lower_tile(tile, tm, tn);
   for (int e = threadIdx.x; e < BM * BN; e += 256) {
@@ -295,10 +294,12 @@ inline hipError_t launch_f64_narrow_tn(hipStream_t st, int M, int N, int K, int 
 }
 
 // The even deal of `batch` weighted lower-triangle products (weights s + b s_bs) of order d.M over K:
-// 128 x 128 tiles (2 workgroups of 8 waves per CU) from an order of 1536, else 64 x 64 (4 of 4 waves),
-// whose edges waste less (12 frequencies: P = 2000 74.3 ms against 85.2 with 64 x 64; P = 937
-// 1.53 against 1.39 ms; P = 1300, 4 frequencies, 2.26 against 2.15 ms); at least 8 K steps a
-// workgroup, so a small matrix is not cut into more parts than it has work for.
+// 128 x 128 tiles (2 workgroups of 8 waves per CU), which do a given area in 0.87 of the time, or 64 x 64 (4 of 4 waves), whose
+// edges waste less: the larger ones unless they compute 1.13 times as much, from an order of 1536 (64 / 128, ms, K = 27000:
+// 1600, 12 frequencies 16.08 / 15.46) or of 1217 with three weight vectors or more (K = 27000: 1400, 11 and 12 frequencies 12.25 / 10.32
+// and 12.20 / 11.11; K = 24000: 1250, 1, 2 and 3 0.87 / 1.07, 1.57 / 1.62, 2.32 / 2.22; 1300, 12, at 1.14 times the area, 9.63 / 9.94);
+// below, their few units are cut into many parts (K = 20000: 1100, 4 and 12 1.77 / 1.78 and 5.10 / 4.97; 6293: 937, 12 1.39 / 1.53).
+// At least 8 K steps a workgroup, so a small matrix is not cut into more parts than it has work for.
 struct EvenPlan {
   int tile;
   EvenShare sh;
@@ -307,12 +308,16 @@ struct EvenPlan {
 };
 inline EvenPlan f64_even_plan(long P, long K, long batch, long cus) {
   EvenPlan p;
-  p.tile = P >= 1536 ? 128 : 64;
+  auto area = [&](long t) {
+    const long n = (P + t - 1) / t;
+    return n * (n + 1) / 2 * t * t;
+  };
+  p.tile = (P >= 1536 || (P > 1216 && batch >= 3)) && area(128) * 100 <= area(64) * 113 ? 128 : 64;
   const long tl = (P + p.tile - 1) / p.tile;
-  // the widest flock that leaves at most a tenth of its workgroups without a batch
-  for (p.sh.flock = 4; p.sh.flock > 1; p.sh.flock /= 2)
-    if ((batch + p.sh.flock - 1) / p.sh.flock * p.sh.flock * 9 <= batch * 10) break;
-  p.sh.bgroups = (int)((batch + p.sh.flock - 1) / p.sh.flock);
+  // the widest flock without idle members (P = 2000, K = 90000: 3 frequencies by 1 / 3 21.1 / 19.5 ms, 9 by 2 (one in ten
+  // idle) / 1 / 3 66.4 / 61.2 / 57.5, 11 by 4 / 1 76.8 / 74.0, 12 by 1 / 2 / 3 / 4 80.0 / 78.0 / 77.1 / 76.0)
+  for (p.sh.flock = 4; p.sh.flock > 1 && batch % p.sh.flock != 0;) --p.sh.flock;
+  p.sh.bgroups = (int)(batch / p.sh.flock);
   p.sh.units = tl * (tl + 1) / 2 * p.sh.bgroups;
   p.sh.steps = (K + 15) / 16;
   const long resident = (p.tile == 128 ? 2 : 4) * cus / p.sh.flock;
