@@ -263,11 +263,15 @@ inline int bf16_kernel_choice() {
 //   26 vectors of  34, 190, 485                       259 /  216 /  249      91 /   79 /   91
 //   12 vectors of  30, 210, 960                       268 /  212 /  244     114 /   86 /   95
 //    4 vectors of  30, 210, 960                       127 /   90 /   94      70 /   42 /   47
-// The register-staged ones remain for plain products of vectors of odd length, whose 2-byte stores the three
-// workgroups per CU of theirs hide better than the 128 x 128 tiles. Against the large tiles they are level with a
-// tenth of padding (large / staged, 14 vectors of 97, 513, 996: 1266 / 1274; 21 of 61, 430, 1000: 890-962 / 935) and 1-18 %
-// slower without (15 of 97: 1290 / 1420; 8, 12, 16 of 61: 363 / 410, 527 / 580, 720 / 737; 14 of 35, 400, 900: 335 / 370; 30 of
-// 91, 700, 800: 1422 / 1603; 17 of 45, 385, 1200: 573 / 669).
+// Plain products take the register-staged tiles, three workgroups per CU, where these hide the stores and the loads better:
+// where vectors of odd length are stored 2 bytes at a time, and, 128 x 128 ring / register-staged in geometric means over
+// 256 problems of 16-110 levels, 60-1200 virtual ones and 2-45 vectors, beyond K = 192 (0.92 below; 48 levels, 327 virtual,
+// 45 vectors: 1283 / 1144 us; 68, 267, 30: 962 / 854), save up to K = 256 where the product has at most 12288 tiles
+// (0.95; with more of them 1.04). Split operands: 0.85-0.97 throughout. The large tiles against them are slower
+// with padding up to K = 448 (1.01-1.04; 48, 400, 45: 1312 / 1254) and faster from there (0.96; 14 vectors of 97, 513, 996:
+// 1266 / 1274; odd: 21 of 61, 430, 1000: 890-962 / 935, so not there), and 1-18 % faster without (15 of 97: 1290 / 1420;
+// 8, 12, 16 of 61: 363 / 410, 527 / 580, 720 / 737; 14 of 35, 400, 900: 335 / 370; 30 of 91, 700, 800: 1422 / 1603; 17 of 45,
+// 385, 1200: 573 / 669).
 inline bool bf16_big_tiles(long M, long N, long K, long batch_ks, int padding) {
   const long t2 = (M + 255) / 256 * ((N + 255) / 256), t1 = (M + 127) / 128 * ((N + 127) / 128);
   return t2 * batch_ks >= 256 && 4 * t2 * 100 <= t1 * (100 + padding) && K >= 384;
@@ -282,7 +286,7 @@ void gemm16(hipStream_t st, int M, int N, int K, int batch, int ksplit, Opnd<uns
     if (choice == 2 && !lower && lds_ok(A, B, K, split)) {
       int padding = 10;
       if constexpr (epi_planes<Epi>::value)
-        if (!split && epi.width() == 1) padding = 2;
+        if (!split && (epi.width() == 1 || K < 448)) padding = 2;
       if (bf16_big_tiles(M, N, K / std::max(ksplit, 1), (long)batch * std::max(ksplit, 1), padding)) {
         GemmDims d = make_dims<256, 256>(M, N, std::max(K, 0), batch, ksplit, split ? 32 : 64, false);
         d.group = d.tiles_m >= 32 && d.tiles_n >= 4 ? 4 : 0;
@@ -290,8 +294,9 @@ void gemm16(hipStream_t st, int M, int N, int K, int batch, int ksplit, Opnd<uns
         return;
       }
       if constexpr (epi_planes<Epi>::value) {
-        if (split || epi.width() > 1) {
-          GemmDims d = make_dims<128, 128>(M, N, std::max(K, 0), batch, ksplit, 64, false);
+        GemmDims d = make_dims<128, 128>(M, N, std::max(K, 0), batch, ksplit, 64, false);
+        const bool few = (long)d.tiles_m * d.tiles_n * batch * std::max(ksplit, 1) <= 12288;
+        if (split || (epi.width() > 1 && (K <= 192 || (K <= 256 && few)))) {
           d.group = d.tiles_m >= 32 && d.tiles_n >= 2 ? 4 : 0;
           XG_HIP((launch_bf16_ring<2, 4, 4, 2, 2>(st, d, A, B, split, epi)));
           return;
