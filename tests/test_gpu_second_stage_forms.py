@@ -12,11 +12,7 @@ pytestmark = pytest.mark.gpu
 TOL = {"bf16": 2 * 4 * 2.0**-9, "bf16x3": 2 * 4 * 2.0**-17}
 
 
-@pytest.mark.parametrize("o,v,P", [(20, 260, 90), (32, 129, 70), (33, 128, 64), (64, 257, 66), (65, 256, 64), (102, 303, 41),
-                                   (128, 130, 33)])
-@pytest.mark.parametrize("k", [3, 16, 32, 43, 65])
-@pytest.mark.parametrize("c", [(0, 0, 1, 0), (0, 0, 0, 1)])
-def test_forms(o, v, P, k, c, monkeypatch):
+def check(o, v, P, k, c, monkeypatch):
     rng = np.random.default_rng(o * 1000 + v + P + k)
     n = o + v
     M = rng.normal(scale=0.05, size=(n, n, P))
@@ -33,3 +29,18 @@ def test_forms(o, v, P, k, c, monkeypatch):
         assert np.linalg.norm(got - ref) <= TOL[prec] * np.linalg.norm(ref)
         monkeypatch.setenv("XTPGPU_BF16_KERNEL", "staged64")
         assert np.array_equal(op.matmul(x, prec), got)
+
+
+@pytest.mark.parametrize("o,v,P", [(20, 260, 90), (32, 129, 70), (33, 128, 64), (64, 257, 66), (65, 256, 64), (102, 303, 41),
+                                   (128, 130, 33)])
+@pytest.mark.parametrize("k", [3, 16, 32, 43, 65])
+@pytest.mark.parametrize("c", [(0, 0, 1, 0), (0, 0, 0, 1)])
+def test_forms(o, v, P, k, c, monkeypatch):
+    check(o, v, P, k, c, monkeypatch)
+
+
+@pytest.mark.parametrize("o,v,P,k", [(77, 54, 110, 45), (77, 54, 110, 90), (66, 33, 130, 45), (128, 90, 70, 33), (128, 91, 70, 64),
+                                     (128, 94, 70, 45), (128, 211, 70, 32), (128, 213, 70, 33), (16, 7, 600, 64), (64, 65, 140, 90)])
+@pytest.mark.parametrize("c", [(0, 0, 1, 0), (0, 0, 0, 1)])
+def test_few_rows(o, v, P, k, c, monkeypatch):
+    check(o, v, P, k, c, monkeypatch)

@@ -286,19 +286,24 @@ enum class Bf16Second { kStaged, kRows256, kRows32 };
 // take, per K, c times the weight below: 32-row tiles (2 to 5 of them run at a time) by their width, 256-row tiles (one at a
 // time), register-staged 128 x 128 tiles two at a time, or one for somewhat more than half of that (the plain
 // one of up to 64 columns for somewhat more). Weights: ns per 10^4 k of the split form, of which the plain
-// one takes 0.40 to 0.45, from 110 products on all three forms; the choice is within 4 % of the fastest on 109 of them and
-// 8 % on all. One threshold on the workgroups had missed the rounds (staged / 256 / 32 rows, split, us): 303 rows, 102
-// columns, 45 vectors, K = 105040 in 3: 270 of the 256-row tiles, 2706 / 4706 / 4218; 640, 100, 30, 72800 in 3: 270, 1922 /
-// 2799 / 3599; 256, 100, 20, 104000 in 4: 640 of the 32-row ones, 940 / 1457 / 1443. Where it had been right: 300, 97,
-// 28, 93600 in 4: 1734 / 1377 / 1901; 210, 30, 15, 30720 in 4: 251 / 319 / 143.
+// one takes 0.40 to 0.45. Rows beyond the product load one and the same line, so products of few rows take less of a tile's
+// time: of two register-staged ones 0.65 up to 59 rows and all from 91 on, of a 256-row one 0.6 up to 94 and all from 212
+// on. Over 1390 products of 7-900 rows and 16-128 columns on all three forms the choice is within 5 % of the fastest on
+// 1345, 0.5 % off it on average, and more than 3 % behind the register-staged tiles on 27 (two thirds of their time on average).
+// One threshold on the workgroups had missed the rounds (staged / 256 / 32 rows, split, us): 303 rows, 102 columns, 45
+// vectors, K = 105040 in 3: 270 of the 256-row tiles, 2706 / 4706 / 4218; 640, 100, 30, 72800 in 3: 270, 1922 / 2799 / 3599; 256,
+// 100, 20, 104000 in 4: 640 of the 32-row ones, 940 / 1457 / 1443; full tiles' weights for all had missed the few rows: 54,
+// 77, 45, 45680 in 4: 344 / 314 / 421; 57, 114, 64, 90360 in 4: 782 / 662 / 901. Where both had been right: 300, 97, 28, 93600
+// in 4: 1734 / 1377 / 1901; 210, 30, 15, 30720 in 4: 251 / 319 / 143.
 inline Bf16Second bf16_second_form(int M, int N, int batch, int ksplit, bool split) {
   const long n = (long)batch * ksplit;
   auto per_cu = [&](int rows) { return ((M + rows - 1) / rows * n + 255) / 256; };
   const bool narrow = N <= 64;
   const long c = per_cu(128);
-  const long staged = c / 2 * (narrow ? 520 : 720) + c % 2 * (!narrow ? 410 : split ? 310 : 340);
-  const long rows256 = per_cu(256) * (narrow ? 490 : 600);
-  const long rows32 = per_cu(32) * (N <= 32 ? 95 : narrow ? 108 : 187);
+  const double pair = std::max(0.65, std::min(1.0, M / 91.0)) * (narrow ? 520 : 720);
+  const double staged = c / 2 * pair + c % 2 * (!narrow ? 410 : split ? 310 : 340);
+  const double rows256 = std::max(0.6, std::min(1.0, 0.28 + M / 294.0)) * per_cu(256) * (narrow ? 490 : 600);
+  const double rows32 = per_cu(32) * (N <= 32 ? 95 : narrow ? 108 : 187);
   if (staged <= rows256 && staged <= rows32) return Bf16Second::kStaged;
   return rows256 <= rows32 ? Bf16Second::kRows256 : Bf16Second::kRows32;
 }
