@@ -50,6 +50,12 @@ def test_split_bf16_tiles(o, v, P, nw, monkeypatch):
     assert np.array_equal(rpa.calculate_epsilon(px.EPS_IMAG, w, "bf16x3"), got)
 
 
+# 270 tiles in three K splits, to either side of 2.5 10^6 tiles x k: direct-to-LDS and register-staged tiles, the same bits
+@pytest.mark.parametrize("o,v", [(40, 228), (40, 234)])
+def test_split_bf16_long(o, v, monkeypatch):
+    test_split_bf16_tiles(o, v, 1100, 6, monkeypatch)
+
+
 # tiles shared by several workgroups, and workgroups that walk several tiles in pieces of K, at both tile sizes
 @pytest.mark.parametrize("o,v,P,nw", [(3, 40, 130, 1), (31, 203, 937, 3), (31, 203, 937, 12), (20, 210, 1600, 1),
                                       (30, 210, 1540, 8)])

@@ -1074,7 +1074,12 @@ void rpa_epsilon_impl(xtpgpu_ctx ctx, xtpgpu_mmn mmn, const double* energies, in
         DevBuf& pb = ctx->ws[2];
         pb.ensure((size_t)d.ksplit * nw_g * P * P * 4);
         const EpiPart32 ep{pb.as<float>(), P, P, nw_g};
-        if (split && bf16_kernel_choice() == 2 && lds_ok(A, Bo, (int)Kp, true))
+        // direct-to-LDS tiles for up to 2.5 10^6 tiles x k, where they hide the loads' latency the better; beyond, the chip
+        // streams the segments, which the register-staged ones do with fewer re-reads in flight (ring / staged, 357 builds of
+        // 257-1535 aux functions and 1-16 frequencies: 0.95 up to 2 10^6, 1.00 to 4, 1.06 to 20, 1.15 beyond; 1100 aux, K =
+        // 56295, 12 frequencies: 5699 / 4621 us; 1020, 1247, 12: 124 / 124)
+        if (split && bf16_kernel_choice() == 2 && lds_ok(A, Bo, (int)Kp, true) &&
+            (double)(tl * (tl + 1) / 2 * nw_g) * Kp <= 2.5e6)
           XG_HIP((launch_bf16_ring<2, 4, 4, 2, 2>(st, d, A, Bo, true, ep)));
         else if (split)
           XG_HIP((launch_gemm_bf16<128, 128, true, true>(st, d, A, Bo, true, ep, true)));
