@@ -40,7 +40,8 @@ def test_forms(o, v, P, k, c, monkeypatch):
 
 
 @pytest.mark.parametrize("o,v,P,k", [(77, 54, 110, 45), (77, 54, 110, 90), (66, 33, 130, 45), (128, 90, 70, 33), (128, 91, 70, 64),
-                                     (128, 94, 70, 45), (128, 211, 70, 32), (128, 213, 70, 33), (16, 7, 600, 64), (64, 65, 140, 90)])
+                                     (128, 94, 70, 45), (128, 211, 70, 32), (128, 213, 70, 33), (16, 7, 600, 64), (64, 65, 140, 90), (96, 130, 33, 70),
+                                     (97, 130, 33, 70)])
 @pytest.mark.parametrize("c", [(0, 0, 1, 0), (0, 0, 0, 1)])
 def test_few_rows(o, v, P, k, c, monkeypatch):
     check(o, v, P, k, c, monkeypatch)

@@ -287,23 +287,29 @@ enum class Bf16Second { kStaged, kRows256, kRows32 };
 // time), register-staged 128 x 128 tiles two at a time, or one for somewhat more than half of that (the plain
 // one of up to 64 columns for somewhat more). Weights: ns per 10^4 k of the split form, of which the plain
 // one takes 0.40 to 0.45. Rows beyond the product load one and the same line, so products of few rows take less of a tile's
-// time: of two register-staged ones 0.65 up to 59 rows and all from 91 on, of a 256-row one 0.6 up to 94 and all from 212
-// on. Over 1390 products of 7-900 rows and 16-128 columns on all three forms the choice is within 5 % of the fastest on
-// 1345, 0.5 % off it on average, and more than 3 % behind the register-staged tiles on 27 (two thirds of their time on average).
+// time: of two register-staged ones 0.65 up to 59 rows and all from 91 on; of a 256-row one 0.6 up to 94 and all from 212
+// on, with split operands of more than 64 columns 2.2 per row and column, from 300 to 600. `own_cols`: the columns' operand
+// is each batch entry's own and is read again by each tile of its rows; that, or few rows, costs the 32-row tiles of
+// split operands where several share a CU. Over 1390 products of 7-900 rows and 16-128 columns on all three forms the choice is
+// within 5 % of the fastest on 1353, 0.4 % off it on average, and more than 3 % behind the register-staged tiles on 16 (0.65
+// of their time on average); over 1258 with `own_cols` more than 3 % behind on 6 (0.56, both stages).
 // One threshold on the workgroups had missed the rounds (staged / 256 / 32 rows, split, us): 303 rows, 102 columns, 45
 // vectors, K = 105040 in 3: 270 of the 256-row tiles, 2706 / 4706 / 4218; 640, 100, 30, 72800 in 3: 270, 1922 / 2799 / 3599; 256,
 // 100, 20, 104000 in 4: 640 of the 32-row ones, 940 / 1457 / 1443; full tiles' weights for all had missed the few rows: 54,
-// 77, 45, 45680 in 4: 344 / 314 / 421; 57, 114, 64, 90360 in 4: 782 / 662 / 901. Where both had been right: 300, 97, 28, 93600
-// in 4: 1734 / 1377 / 1901; 210, 30, 15, 30720 in 4: 251 / 319 / 143.
-inline Bf16Second bf16_second_form(int M, int N, int batch, int ksplit, bool split) {
+// 77, 45, 45680 in 4: 344 / 314 / 421; 57, 114, 64, 90360 in 4: 782 / 662 / 901; 89, 124, 45, 117632 in 4: 1014 / 1298 / 1457;
+// own columns (both stages): 197, 112, 45, 128576: 5601 / 6914 / 6316. Where all had been right: 300, 97, 28, 93600 in 4: 1734 /
+// 1377 / 1901; 210, 30, 15, 30720 in 4: 251 / 319 / 143.
+inline Bf16Second bf16_second_form(int M, int N, int batch, int ksplit, bool split, bool own_cols) {
   const long n = (long)batch * ksplit;
   auto per_cu = [&](int rows) { return ((M + rows - 1) / rows * n + 255) / 256; };
   const bool narrow = N <= 64;
   const long c = per_cu(128);
   const double pair = std::max(0.65, std::min(1.0, M / 91.0)) * (narrow ? 520 : 720);
   const double staged = c / 2 * pair + c % 2 * (!narrow ? 410 : split ? 310 : 340);
-  const double rows256 = std::max(0.6, std::min(1.0, 0.28 + M / 294.0)) * per_cu(256) * (narrow ? 490 : 600);
-  const double rows32 = per_cu(32) * (N <= 32 ? 95 : narrow ? 108 : 187);
+  const double rows256 = per_cu(256) * (split && !narrow ? std::max(300.0, std::min(600.0, 2.2 * (std::min(M, 256) + N)))
+                                                         : std::max(0.6, std::min(1.0, 0.28 + M / 294.0)) * (narrow ? 490 : 600));
+  const bool reread = split && per_cu(32) > 1 && ((own_cols && N > 96) || M <= 100);
+  const double rows32 = per_cu(32) * (N <= 32 ? 95 : narrow ? 108 : reread ? 210 : 187);
   if (staged <= rows256 && staged <= rows32) return Bf16Second::kStaged;
   return rows256 <= rows32 ? Bf16Second::kRows256 : Bf16Second::kRows32;
 }

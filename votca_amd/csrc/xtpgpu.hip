@@ -1446,7 +1446,7 @@ void bse_matmul_impl(xtpgpu_bseop op, int precision, const double* X, long ldx, 
     const EpiPart32 ep{pt, ct, vt, k};
     const bool fits = (size_t)dd.ksplit * k * ct * vt * 4 <= part_bytes;
     const Bf16Second form = fits && vt <= 128 && bf16_kernel_choice() == 2 && lds_ok(A, B, (int)K2, split)
-                                ? bf16_second_form((int)ct, (int)vt, (int)k, dd.ksplit, split) : Bf16Second::kStaged;
+                                ? bf16_second_form((int)ct, (int)vt, (int)k, dd.ksplit, split, B.bs != 0) : Bf16Second::kStaged;
     if (form != Bf16Second::kStaged) {
       XG_HIP(launch_bf16_tall(st, form, (int)ct, (int)vt, (int)K2, (int)k, ks, bk, A, B, split, ep));
     } else if (fits && ks > 1 && bf16_vec(A, B, (int)K2)) {
