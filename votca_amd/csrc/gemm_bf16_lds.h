@@ -12,10 +12,10 @@
 //     of the Hd contraction at 128700 x 3000 x 900, split / plain: 2.64 / 0.98 ms with 128 x 128
 //     tiles, 2.00 / 0.83 here (347 / 840 TFLOP/s); eight waves of 128 x 64 2.11 / 0.85, of 64 x 128
 //     2.12 / 0.84, 256 x 128 tiles 2.42 / 1.01; the same without the stores 1.65 / 0.60.
-//   128 x 128, 8 waves of 32 x 64, 2 stages: products with fewer columns or a shorter K; two workgroups
-//     per CU, one's epilogue under the other's products (three stages leave room for one: 20-30% slower).
-//   256 rows x (16 TN) columns, 8 waves of 32 rows, 3 stages: second-stage products with enough of
-//     them (900 x 100 per vector, K = 29744, 30 vectors: 1193 -> 1054 us split, 440 -> 410 plain).
+//   128 x 128, 8 waves of 32 x 64, 2 stages: split products with fewer columns or a shorter K, plain ones with a
+//     short K; two workgroups per CU, one's epilogue under the other's products (three stages leave room for one: 20-30% slower).
+//   256 rows x (16 TN) columns, 8 waves of 32 rows, 3 stages: second-stage products that fill their
+//     rounds (900 x 100 per vector, K = 29744, 30 vectors: 1193 -> 1054 us split, 440 -> 410 plain).
 //   32 rows x (32, 64, 128) columns, 2 x 2 waves, 4 stages: the same with few outputs, where each
 //     workgroup walks a long K alone and the ring hides the latency (210 x 30 per vector,
 //     K = 30720 in 4 splits, 8 vectors: 197 -> 67 us split, 99 -> 35 plain).
